@@ -631,7 +631,8 @@ int w8a8_swiglu(void* stream, const void* gate, const void* up, size_t rows, uin
   const size_t a = out_align(dtype);
   if (!al(gate, a) || !al(up, a) || !al(act, a) || !al(maxima, 4)) return W8A8_EALIGN;
   if (!ready()) return W8A8_EINIT;
-  return hip_status(launch_swiglu((hipStream_t)stream, gate, up, rows, width, act, dtype, maxima));
+  return hip_status(launch_swiglu((hipStream_t)stream, gate, up, rows, width, act, dtype, maxima, nullptr,
+                                  nullptr));
 }
 
 // linear_swiglu, and with q_out the quantize_with_max of its act that the
@@ -677,9 +678,7 @@ static int run_swiglu(void* stream, const int8_t* q, const float* asc, size_t m,
   void* out[2] = {gate, up};
   s = w8a8_linear_grouped(stream, q, asc, m, k, 2, w, ws, nn, out, out_dtype);
   if (s != W8A8_OK) return s;
-  s = hip_status(launch_swiglu(st, gate, up, m, (uint32_t)n, act, out_dtype, maxima));
-  if (s != W8A8_OK || !q_out) return s;
-  return hip_status(launch_swiglu_quantize_rows(st, act, m, (uint32_t)n, out_dtype, maxima, q_out, scales_out));
+  return hip_status(launch_swiglu(st, gate, up, m, (uint32_t)n, act, out_dtype, maxima, q_out, scales_out));
 }
 
 int w8a8_linear_swiglu(void* stream, const int8_t* q, const float* asc, size_t m, uint32_t k,

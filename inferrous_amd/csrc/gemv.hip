@@ -967,7 +967,7 @@ __global__ __launch_bounds__((NS + kProdWaves) * kWave) void gemv_rowtail_split(
 
 // swiglu (src/kernels.rs:2172-2190): act = silu_mul(gate, up) elementwise
 // over rows x width (blockIdx.y = row); with maxima, each row's largest
-// |act| is published into maxima[row].
+// |act| is published into maxima[row].  Rows wider than swiglu_rows holds.
 __global__ __launch_bounds__(kGemvThreads) void swiglu_kernel(const void* gate, const void* up,
                                                                uint32_t width, void* act, int dtype,
                                                                uint32_t* maxima) {
@@ -981,6 +981,134 @@ __global__ __launch_bounds__(kGemvThreads) void swiglu_kernel(const void* gate, 
     bits = max(bits, abs_bits_no_nan(v));
   }
   if (maxima) publish_absmax_block(bits, maxima + r);
+}
+
+// VEC consecutive values of a BF16 or f32 array from element i (a 16-byte
+// access when VEC > 1: 8 BF16 or 4 f32 values).
+template <bool BF16, int VEC>
+__device__ __forceinline__ void load_vec(const void* p, size_t i, float (&v)[VEC]) {
+  if constexpr (VEC == 1) {
+    v[0] = load_val(p, i, BF16 ? W8A8_OUT_BF16 : W8A8_OUT_F32);
+  } else if constexpr (BF16) {
+    static_assert(VEC == 8, "16 bytes");
+    const v4i w = *reinterpret_cast<const v4i*>(reinterpret_cast<const uint16_t*>(p) + i);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      v[2 * e] = __uint_as_float((uint32_t)w[e] << 16);
+      v[2 * e + 1] = __uint_as_float((uint32_t)w[e] & 0xffff0000u);
+    }
+  } else {
+    static_assert(VEC == 4, "16 bytes");
+    const v4f w = *reinterpret_cast<const v4f*>(reinterpret_cast<const float*>(p) + i);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = w[e];
+  }
+}
+
+// The values are BF16 values already (bf16_rne), so the BF16 form is their
+// high halves.
+template <bool BF16, int VEC>
+__device__ __forceinline__ void store_vec(void* p, size_t i, const float (&v)[VEC]) {
+  if constexpr (VEC == 1) {
+    store_out(p, i, BF16 ? W8A8_OUT_BF16 : W8A8_OUT_F32, 0, v[0]);
+  } else if constexpr (BF16) {
+    v4i w;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      w[e] = (int)((__float_as_uint(v[2 * e]) >> 16) | (__float_as_uint(v[2 * e + 1]) & 0xffff0000u));
+    *reinterpret_cast<v4i*>(reinterpret_cast<uint16_t*>(p) + i) = w;
+  } else {
+    *reinterpret_cast<v4f*>(reinterpret_cast<float*>(p) + i) = v4f{v[0], v[1], v[2], v[3]};
+  }
+}
+
+// The SiLU product of one row per workgroup, its maximum, and (with q) its
+// codes: swiglu, the fold of the row's largest bits(|act|) into maxima[row],
+// and quantize_with_max with the folded maximum, in one pass over gate and
+// up.  Bound by HBM at many rows (gate and up in, act and the codes out) and
+// by one row's latency at few, so a row stays in registers between the two
+// halves: NV vectors of VEC values per thread, every load issued before the
+// first use (indices clamped to the row).  One atomicMax per row: swiglu_kernel
+// publishes from up to 64 workgroups per row, and on MI355X those atomics,
+// one after another at ~8 ns, were the whole kernel.  Per dispatch, rows of
+// 12,288, swiglu_kernel + the quantizing launch after it -> swiglu_rows with
+// q: 4,096 f32 rows 1,600 + 55 -> 118 us (5.5 TB/s of gate, up, act and
+// codes), 512 BF16 rows 246 + 11 -> 15.1, 129 f32 rows 77 + 5 -> 8.6, 32
+// BF16 rows 24.7 + 7.5 -> 7.1, 4 f32 rows 4.9 + 4.4 -> 6.1.  At 512 rows and
+// fewer the exp, the two divisions and the rounding (about 60 VALU
+// instructions a value) bound it, not the bytes.
+constexpr int kSwigluThreads = 512;
+constexpr uint32_t kSwigluRowMax = 16384;  // widest row held in registers
+
+template <bool BF16, int VEC, int NV>
+__global__ __launch_bounds__(kSwigluThreads) void swiglu_rows(const void* gate, const void* up, uint32_t width,
+                                                              void* act, uint32_t* maxima, int8_t* q,
+                                                              float* scales) {
+  constexpr int T = kSwigluThreads;
+  __shared__ uint32_t wmax[T / kWave];
+  const size_t r = blockIdx.x, base = r * (size_t)width;
+  const uint32_t t = threadIdx.x, nvec = width / VEC;
+  // only this workgroup folds into maxima[r] during the call
+  const uint32_t before = maxima[r];
+  float g[NV][VEC], v[NV][VEC];
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const size_t e = base + (size_t)min(t + i * T, nvec - 1) * VEC;
+    load_vec<BF16, VEC>(gate, e, g[i]);
+    load_vec<BF16, VEC>(up, e, v[i]);
+  }
+  uint32_t bits = 0;
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) v[i][e] = silu_mul(g[i][e], v[i][e]);
+    if (t + i * T < nvec) {  // not the clamped repeats: act may be gate's or up's own buffer
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) bits = max(bits, abs_bits_no_nan(v[i][e]));
+      store_vec<BF16, VEC>(act, base + (size_t)(t + i * T) * VEC, v[i]);
+    }
+  }
+  bits = wave_max_u32(bits);
+  if ((t & 63) == 0) wmax[t >> 6] = bits;
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < T / kWave; ++i) bits = max(bits, wmax[i]);
+  if (t == 0) atomicMax(maxima + r, bits);
+  if (!q) return;
+  const float s = __uint_as_float(max(before, bits)) / 127.0f;
+  const float rs = 1.0f / s;
+  if (t == 0) scales[r] = s;
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    int code[VEC];
+    quant_codes<VEC>(v[i], s, rs, code);
+    if (t + i * T >= nvec) continue;
+    int8_t* const o = q + base + (size_t)(t + i * T) * VEC;
+    if constexpr (VEC == 1) {
+      *o = (int8_t)code[0];
+    } else {
+#pragma unroll
+      for (int e = 0; e < VEC; e += 4)
+        reinterpret_cast<uint32_t*>(o)[e / 4] = (uint32_t)(uint8_t)code[e] | (uint32_t)(uint8_t)code[e + 1] << 8 |
+                                                (uint32_t)(uint8_t)code[e + 2] << 16 |
+                                                (uint32_t)(uint8_t)code[e + 3] << 24;
+    }
+  }
+}
+
+// swiglu without maxima: elementwise over the whole array, VEC values per
+// thread and step.
+template <bool BF16, int VEC>
+__global__ __launch_bounds__(kGemvThreads) void swiglu_flat(const void* gate, const void* up, size_t nvec,
+                                                            void* act) {
+  for (size_t j = (size_t)blockIdx.x * kGemvThreads + threadIdx.x; j < nvec; j += (size_t)gridDim.x * kGemvThreads) {
+    float g[VEC], v[VEC];
+    load_vec<BF16, VEC>(gate, j * VEC, g);
+    load_vec<BF16, VEC>(up, j * VEC, v);
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) v[e] = silu_mul(g[e], v[e]);
+    store_vec<BF16, VEC>(act, j * VEC, v);
+  }
 }
 
 // Standalone greedy selection over f32 values.  Each thread takes
@@ -1237,26 +1365,63 @@ hipError_t launch_gemv_rowtail(hipStream_t st, const RowtailArgs& d) {
   return bf16 ? launch_rowtail<EPI_PLAIN, true>(st, d) : launch_rowtail<EPI_PLAIN, false>(st, d);
 }
 
-hipError_t launch_swiglu_quantize_rows(hipStream_t st, const void* act, size_t rows, uint32_t width, int dtype,
-                                       const uint32_t* maxima, int8_t* q, float* scales) {
-  if (rows == 0 || width == 0) return hipSuccess;
-  if (rows > 0x7fffffffu) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(swiglu_row_tail<false>, dim3((unsigned)rows), dim3(kRowTailThreads), 0, st, act, width, dtype,
-                     const_cast<uint32_t*>(maxima), q, scales);
-  return hipGetLastError();
+template <bool BF16, int VEC>
+static void launch_swiglu_rows(hipStream_t st, const char* gate, const char* up, uint32_t rows, uint32_t width,
+                               char* act, uint32_t* maxima, int8_t* q, float* scales) {
+  const uint32_t nv = (width / VEC + kSwigluThreads - 1) / kSwigluThreads;  // vectors per thread
+  auto k = VEC == 8   ? (nv <= 1 ? swiglu_rows<BF16, VEC, 1> : nv <= 2 ? swiglu_rows<BF16, VEC, 2>
+                         : nv <= 3 ? swiglu_rows<BF16, VEC, 3> : swiglu_rows<BF16, VEC, 4>)
+           : VEC == 4 ? (nv <= 2 ? swiglu_rows<BF16, VEC, 2> : nv <= 4 ? swiglu_rows<BF16, VEC, 4>
+                         : nv <= 6 ? swiglu_rows<BF16, VEC, 6> : swiglu_rows<BF16, VEC, 8>)
+                      : (nv <= 8 ? swiglu_rows<BF16, VEC, 8> : nv <= 24 ? swiglu_rows<BF16, VEC, 24>
+                                                                        : swiglu_rows<BF16, VEC, 32>);
+  hipLaunchKernelGGL(k, dim3(rows), dim3(kSwigluThreads), 0, st, gate, up, width, act, maxima, q, scales);
 }
 
-hipError_t launch_swiglu(hipStream_t st, const void* gate, const void* up, size_t rows,
-                         uint32_t width, void* act, int dtype, uint32_t* maxima) {
+// swiglu over rows x width, the maxima fold (maxima optional) and the codes
+// (q with scales, optional, maxima required).  Without maxima one elementwise
+// pass; rows of up to kSwigluRowMax values (what a workgroup's registers
+// hold) by swiglu_rows, one workgroup per row; wider rows by swiglu_kernel's
+// many workgroups per row, then the row tail.
+hipError_t launch_swiglu(hipStream_t st, const void* gate, const void* up, size_t rows, uint32_t width, void* act,
+                         int dtype, uint32_t* maxima, int8_t* q, float* scales) {
   if (rows == 0 || width == 0) return hipSuccess;
+  const bool bf16 = dtype == W8A8_OUT_BF16;
+  const size_t esz = bf16 ? 2 : 4;
+  const uint32_t vec = bf16 ? 8 : 4;
+  const bool al = (((uintptr_t)gate | (uintptr_t)up | (uintptr_t)act) & 15) == 0 && ((uintptr_t)q & (vec - 1)) == 0;
+  if (!maxima) {
+    const size_t total = rows * (size_t)width;
+    const bool wide = al && total % vec == 0;
+    const size_t nvec = wide ? total / vec : total;
+    const uint32_t blocks = (uint32_t)std::min<size_t>((nvec + kGemvThreads - 1) / kGemvThreads, 1u << 20);
+    auto k = wide ? (bf16 ? swiglu_flat<true, 8> : swiglu_flat<false, 4>)
+                  : (bf16 ? swiglu_flat<true, 1> : swiglu_flat<false, 1>);
+    hipLaunchKernelGGL(k, dim3(blocks), dim3(kGemvThreads), 0, st, gate, up, nvec, act);
+    return hipGetLastError();
+  }
+  const bool held = width <= kSwigluRowMax, wide = al && width % vec == 0;
   const uint32_t bx = std::min<uint32_t>((width + kGemvThreads - 1) / kGemvThreads, 64u);
-  const size_t esz = dtype == W8A8_OUT_BF16 ? 2 : 4;
-  for (size_t r0 = 0; r0 < rows; r0 += 65535) {
-    const uint32_t ry = (uint32_t)std::min<size_t>(rows - r0, 65535);
-    const size_t off = r0 * width * esz;
-    hipLaunchKernelGGL(swiglu_kernel, dim3(bx, ry), dim3(kGemvThreads), 0, st,
-                       (const char*)gate + off, (const char*)up + off, width, (char*)act + off,
-                       dtype, maxima ? maxima + r0 : nullptr);
+  const size_t chunk = held ? size_t(1) << 22 : 65535;  // rows per launch (grid limits)
+  for (size_t r0 = 0; r0 < rows; r0 += chunk) {
+    const uint32_t nr = (uint32_t)std::min<size_t>(rows - r0, chunk);
+    const size_t off = r0 * width;
+    const char* const g = (const char*)gate + off * esz;
+    const char* const u = (const char*)up + off * esz;
+    char* const o = (char*)act + off * esz;
+    int8_t* const qr = q ? q + off : nullptr;
+    float* const sr = scales ? scales + r0 : nullptr;
+    if (held) {
+      if (wide && bf16) launch_swiglu_rows<true, 8>(st, g, u, nr, width, o, maxima + r0, qr, sr);
+      else if (wide) launch_swiglu_rows<false, 4>(st, g, u, nr, width, o, maxima + r0, qr, sr);
+      else if (bf16) launch_swiglu_rows<true, 1>(st, g, u, nr, width, o, maxima + r0, qr, sr);
+      else launch_swiglu_rows<false, 1>(st, g, u, nr, width, o, maxima + r0, qr, sr);
+    } else {
+      hipLaunchKernelGGL(swiglu_kernel, dim3(bx, nr), dim3(kGemvThreads), 0, st, g, u, width, o, dtype, maxima + r0);
+      if (q)
+        hipLaunchKernelGGL(swiglu_row_tail<false>, dim3(nr), dim3(kRowTailThreads), 0, st, o, width, dtype,
+                           maxima + r0, qr, sr);
+    }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }

@@ -169,11 +169,11 @@ hipError_t launch_gemv_timeline(hipStream_t st, const int8_t* q, const float* as
                                 uint64_t* stamps);
 hipError_t launch_gemv_argmax(hipStream_t st, GemvArgs& a);
 hipError_t launch_gemv_swiglu(hipStream_t st, const SwigluArgs& a);  // m == 1, k in {4096, 12288}
-hipError_t launch_swiglu(hipStream_t st, const void* gate, const void* up, size_t rows,
-                         uint32_t width, void* act, int dtype, uint32_t* maxima);
-// act rows quantized as quantize_with_max does with maxima (F32 or BF16 act)
-hipError_t launch_swiglu_quantize_rows(hipStream_t st, const void* act, size_t rows, uint32_t width, int dtype,
-                                       const uint32_t* maxima, int8_t* q, float* scales);
+// act = silu_mul(gate, up) over rows x width; with maxima each row's largest
+// |act| folded into it, and with q (and scales) act quantized as
+// quantize_with_max does with the folded maxima (F32 or BF16)
+hipError_t launch_swiglu(hipStream_t st, const void* gate, const void* up, size_t rows, uint32_t width, void* act,
+                         int dtype, uint32_t* maxima, int8_t* q, float* scales);
 hipError_t launch_select(hipStream_t st, const float* x, size_t n, uint64_t* keys, uint32_t* token);
 // u64 keys the fused selection of an n-row lm_head writes (an upper bound)
 size_t argmax_keys_bound(size_t n);

@@ -1,0 +1,94 @@
+"""The one-pass SwiGLU rows (swiglu_rows, gemv.hip) at the edges of its
+vectors, its register-held width and its alignment rule: act equal to the
+elementwise form bit for bit and within one BF16 ulp of the oracle, the
+maxima equal to the fold of what was written, and the codes equal to
+quantize_with_max of act with the folded maxima."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import oracle
+from inferrous_amd import CudaContext, DeviceBuffer, load
+from inferrous_amd._lib import OUT_BF16, OUT_F32, lib
+from test_gpu_swiglu import F32, FLOOR, act_close, bits, dev, fold_max
+
+pytestmark = pytest.mark.gpu
+
+INF, NAN = np.inf, np.nan
+
+
+@pytest.fixture(scope="module")
+def env():
+    ctx = CudaContext(0)
+    return load(ctx), ctx.new_stream()
+
+
+def values(buf, s):
+    a = buf.to_host_vec(s)
+    return a if a.dtype == F32 else (a.astype(np.uint32) << 16).view(F32)
+
+
+@pytest.mark.parametrize("width", [1, 7, 8, 2048, 2056, 4096, 4100, 8200, 12288, 16384, 16385, 16392])
+@pytest.mark.parametrize("dtype", [np.float32, np.uint16])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_rows_equal_the_elementwise_form(env, width, dtype, shift):
+    mod, s = env
+    rows = 5
+    rng = np.random.default_rng(width + shift)
+    g, u = (oracle.bf16_rne((rng.standard_normal(rows * width) * 3).astype(F32)) for _ in range(2))
+    g[:4], u[:4] = [NAN, INF, -INF, 0.0][:len(g[:4])], 1.0
+    u[-1] = INF
+    enc = (lambda a: a) if dtype == np.float32 else (lambda a: (bits(a) >> 16).astype(np.uint16))
+
+    def shifted(a):
+        """The array `shift` elements past a 16-byte boundary."""
+        whole = dev(s, np.concatenate([np.zeros(shift, dtype), a]))
+        return DeviceBuffer.view_of(whole, shift, len(a))
+
+    dg, du = shifted(enc(g)), shifted(enc(u))
+    flat, act = (shifted(np.zeros(rows * width, dtype)) for _ in range(2))
+    start = np.full(rows, FLOOR, np.uint32)
+    start[1] = bits(F32(1e30))[0]
+    mx = dev(s, start)
+    code = OUT_F32 if dtype == np.float32 else OUT_BF16
+    assert lib().w8a8_swiglu(s.handle, dg.ptr, du.ptr, rows, width, flat.ptr, None, code) == 0
+    assert lib().w8a8_swiglu(s.handle, dg.ptr, du.ptr, rows, width, act.ptr, mx.ptr, code) == 0
+    got, want = values(act, s).reshape(rows, width), values(flat, s).reshape(rows, width)
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+    fin = np.isfinite(got.ravel())
+    act_close(got.ravel()[fin], g[fin], u[fin])
+    maxima = mx.to_host_vec(s)
+    for r in range(rows):
+        assert int(maxima[r]) == max(int(start[r]), fold_max(got[r])), f"row {r}"
+    # in place: act over gate
+    assert lib().w8a8_swiglu(s.handle, dg.ptr, du.ptr, rows, width, dg.ptr, dev(s, start).ptr, code) == 0
+    assert np.array_equal(values(dg, s).view(np.uint32), got.ravel().view(np.uint32))
+
+
+@pytest.mark.parametrize("n", [7, 8, 2048, 4100, 16384, 16385])
+@pytest.mark.parametrize("dtype", [np.float32, np.uint16])
+@pytest.mark.parametrize("m", [6, 70])
+def test_row_codes(env, m, n, dtype):
+    """linear_swiglu_quantize at several rows: the codes and scales of act
+    under the folded maxima, one row's maximum set beforehand to a larger and
+    one to a smaller value than its own."""
+    mod, s = env
+    k = 32
+    rng = np.random.default_rng(m + n)
+    mats = [(dev(s, rng.integers(-127, 128, (n, k), dtype=np.int8)), dev(s, (rng.random(n) / 64).astype(F32)))
+            for _ in range(2)]
+    q, asc = dev(s, rng.integers(-127, 128, (m, k), dtype=np.int8)), dev(s, (rng.random(m) / 64).astype(F32))
+    g, u, act = (DeviceBuffer.zeroed(s, m * n, dtype) for _ in range(3))
+    start = np.full(m, FLOOR, np.uint32)
+    start[1] = bits(F32(1e6))[0]
+    mx = dev(s, start)
+    codes, sc = DeviceBuffer.zeroed(s, m * n, np.int8), DeviceBuffer.zeroed(s, m, F32)
+    mod.linear_swiglu_quantize(s, None, q, asc, k, *mats[0], g, *mats[1], u, act, mx, codes, sc)
+    a = values(act, s)
+    act_close(a, values(g, s), values(u, s))
+    want = [max(int(start[r]), fold_max(a.reshape(m, n)[r])) for r in range(m)]
+    assert mx.to_host_vec(s).tolist() == want
+    wq, ws = oracle.quantize_with_max(a, n, np.array(want, np.uint32))
+    assert np.array_equal(codes.to_host_vec(s), wq)
+    assert np.array_equal(bits(sc.to_host_vec(s)), bits(ws))
