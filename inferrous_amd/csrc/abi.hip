@@ -77,7 +77,8 @@ int check_linear(const int8_t* q, const float* asc, size_t m, const int8_t* w, c
 // MFMA routes at m = 2 (gemm_skinny at K not a multiple of 512, split-K) were
 // not measured to lead and keep the GEMV.  A split-K route needs the
 // caller's workspace; without it m = 3 and 4 keep the dot4 GEMV.  The grouped
-// projections keep one dot4 launch for every matrix up to m = 4 (kDot4MaxM).
+// projections take one GEMM launch from m = 2 where their route is gemm_narrow
+// or the 96-column tiles, and keep one dot4 launch up to m = 4 otherwise.
 constexpr size_t kDot4MaxM = 4;
 constexpr size_t kDot4AutoMaxM = 2;
 constexpr size_t kRowtailWidthAbi = 12288;  // the down projection's K (the MLP width)
@@ -598,24 +599,45 @@ int w8a8_linear_grouped(void* stream, const int8_t* q, const float* asc, size_t 
   if (m == 0) return W8A8_OK;
   if (!ready()) return W8A8_EINIT;
   hipStream_t st = (hipStream_t)stream;
+  // One GEMM launch over the matrices that have columns, where it has a route.
+  GemmGroup g{};
+  for (int i = 0; i < count; ++i) {
+    if (n[i] == 0) continue;
+    g.w[g.count] = w[i];
+    g.ws[g.count] = ws[i];
+    g.out[g.count] = out[i];
+    g.n[g.count++] = (uint32_t)n[i];
+  }
+  if (g.count == 0) return W8A8_OK;
+  const GemmRoute r = m > 1 ? gemm_group_route((uint32_t)m, k, g.n, g.count) : GemmRoute{};
+  const bool gemm = r.family != kRouteNone && (m > kDot4MaxM || r.family == kRouteNarrow || r.bn == 96);
+  if (gemm) {
+    GemmArgs a{};
+    a.q = q;
+    a.asc = asc;
+    a.m = (uint32_t)m;
+    a.k = k;
+    a.out_dtype = out_dtype;
+    return hip_status(launch_gemm_group(st, a, g));
+  }
   if (m <= kDot4MaxM) {
     GemvArgs a{};
     a.q = q;
     a.asc = asc;
     a.m = (uint32_t)m;
     a.k = k;
-    a.count = count;
-    for (int i = 0; i < count; ++i) {
-      a.w[i] = w[i];
-      a.ws[i] = ws[i];
-      a.n[i] = (uint32_t)n[i];
-      a.out[i] = out[i];
+    a.count = g.count;
+    for (int i = 0; i < g.count; ++i) {
+      a.w[i] = g.w[i];
+      a.ws[i] = g.ws[i];
+      a.n[i] = g.n[i];
+      a.out[i] = g.out[i];
     }
     a.out_dtype = out_dtype;
     return hip_status(launch_gemv(st, a));
   }
-  for (int i = 0; i < count; ++i) {
-    int s = run_linear(st, q, asc, m, w[i], ws[i], n[i], k, out[i], out_dtype, W8A8_PATH_MFMA,
+  for (int i = 0; i < g.count; ++i) {
+    int s = run_linear(st, q, asc, m, g.w[i], g.ws[i], g.n[i], k, g.out[i], out_dtype, W8A8_PATH_MFMA,
                        nullptr, nullptr);
     if (s != W8A8_OK) return s;
   }

@@ -265,6 +265,24 @@ __device__ __forceinline__ void wait_vmcnt() {
 enum { EP_I32 = 0, EP_F32 = 1, EP_BF16 = 2, EP_F32_RES = 3, EP_BF16_RES = 4, EP_SLAB = 5 };
 constexpr bool raw_i32(int ep) { return ep == EP_I32 || ep == EP_SLAB; }
 
+// Grouped launches (GROUP): the matrix that owns column tile t becomes the
+// launch's only one (a.w, a.ws, a.out, a.n), and the tile's index within it is
+// returned.  Every boundary and operand sits at a fixed kernel-argument
+// offset, so this is a batch of scalar loads, compares and selects.
+struct NoGroup {};
+template <bool GROUP>
+using GroupArg = std::conditional_t<GROUP, GemmGroup, NoGroup>;
+
+__device__ __forceinline__ uint32_t own_tile(GemmArgs&, const NoGroup&, uint32_t t) { return t; }
+__device__ __forceinline__ uint32_t own_tile(GemmArgs& a, const GemmGroup& g, uint32_t t) {
+  a.w = g.w[0], a.ws = g.ws[0], a.out = g.out[0], a.n = g.n[0];
+  uint32_t first = 0;
+#pragma unroll
+  for (int i = 1; i < kMaxGroup; ++i)
+    if (t >= g.tbegin[i]) a.w = g.w[i], a.ws = g.ws[i], a.out = g.out[i], a.n = g.n[i], first = g.tbegin[i];
+  return t - first;
+}
+
 // ---------------------------------------------------------------- narrow
 // Workgroup b owns output columns [16 b, 16 b + 16) and all M rows (MB
 // 16-row blocks).  Wave w sums ST = K / (128 S) of the 128-byte K chunks
@@ -289,8 +307,8 @@ constexpr bool raw_i32(int ep) { return ep == EP_I32 || ep == EP_SLAB; }
 // stage is waited for with vmcnt (every issued instruction has a live lane,
 // so the count is exact), and a slot is refilled only after the previous
 // stage's fragment reads have returned.
-template <int MB, int LAL, int S, int R>
-__global__ __launch_bounds__(64 * S) void gemm_narrow(GemmArgs a) {
+template <int MB, int LAL, int S, int R, bool GROUP = false>
+__global__ __launch_bounds__(64 * S) void gemm_narrow(GemmArgs a, GroupArg<GROUP> group) {
   constexpr int ROWS = 16 * (1 + MB);
   constexpr int STAGE = ROWS * 128;
   constexpr int L = 2 + LAL;  // DMA instructions per stage
@@ -302,7 +320,8 @@ __global__ __launch_bounds__(64 * S) void gemm_narrow(GemmArgs a) {
   __shared__ __attribute__((aligned(1024))) int8_t lds[S * RING];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const uint32_t n0 = blockIdx.x * 16, K = a.k, M = a.m, N = a.n;
+  const uint32_t n0 = own_tile(a, group, blockIdx.x) * 16;
+  const uint32_t K = a.k, M = a.m, N = a.n;
   const uint32_t ST = K / (128 * S);
   int8_t* const ring = lds + wave * RING;
 
@@ -480,9 +499,9 @@ __device__ __forceinline__ void store_blocks(const GemmArgs& a, const v16i (&acc
 // hit sixteen different 16-byte bank groups.  Sub-step i of a stage covers
 // k bytes [32i, 32i + 32): lane l (row / column l % 32, half h = l / 32)
 // reads chunk 2i + h -- the same lane -> k map for A and B.
-template <int BM, int BN, int WM, int WN, int SA, int SB, int EP, bool ROT = false>
+template <int BM, int BN, int WM, int WN, int SA, int SB, int EP, bool ROT = false, bool GROUP = false>
 __global__ __launch_bounds__(512) void gemm_dma(GemmArgs a, uint32_t tiles_m, uint32_t tiles_n,
-                                                uint32_t splits) {
+                                                uint32_t splits, GroupArg<GROUP> group) {
   constexpr int WAVES_N = BN / WN;
   static_assert((BM / WM) * (BN / WN) == 8, "eight waves per workgroup");
   static_assert(WM % 32 == 0 && WN % 32 == 0 && BM % 64 == 0 && BN % 64 == 0, "tile shape");
@@ -504,7 +523,7 @@ __global__ __launch_bounds__(512) void gemm_dma(GemmArgs a, uint32_t tiles_m, ui
   if (G % 8 == 0) Lt = (blockIdx.x % 8) * (G / 8) + blockIdx.x / 8;
   const uint32_t split = Lt / T;
   Lt %= T;
-  const uint32_t m0 = (Lt % tiles_m) * BM, n0 = (Lt / tiles_m) * BN;
+  const uint32_t m0 = (Lt % tiles_m) * BM, n0 = own_tile(a, group, Lt / tiles_m) * BN;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int wm0 = (wave / WAVES_N) * WM, wn0 = (wave % WAVES_N) * WN;
@@ -655,20 +674,20 @@ static hipError_t launch_dma(hipStream_t st, const GemmArgs& a) {
   const uint32_t tm = (a.m + BM - 1) / BM, tn = (a.n + BN - 1) / BN;
   const dim3 grid(tm * tn), block(512);
   if (a.out_dtype == W8A8_OUT_I32) {
-    hipLaunchKernelGGL((gemm_dma<BM, BN, WM, WN, SA, SB, EP_I32, kRotateK>), grid, block, 0, st, a, tm, tn, 1u);
+    hipLaunchKernelGGL((gemm_dma<BM, BN, WM, WN, SA, SB, EP_I32, kRotateK>), grid, block, 0, st, a, tm, tn, 1u, NoGroup{});
   } else if (a.residual) {
     if constexpr (kResidualTile<WM, WN>) {
       if (a.out_dtype == W8A8_OUT_F32)
-        hipLaunchKernelGGL((gemm_dma<BM, BN, WM, WN, SA, SB, EP_F32_RES, kRotateK>), grid, block, 0, st, a, tm, tn, 1u);
+        hipLaunchKernelGGL((gemm_dma<BM, BN, WM, WN, SA, SB, EP_F32_RES, kRotateK>), grid, block, 0, st, a, tm, tn, 1u, NoGroup{});
       else
-        hipLaunchKernelGGL((gemm_dma<BM, BN, WM, WN, SA, SB, EP_BF16_RES, kRotateK>), grid, block, 0, st, a, tm, tn, 1u);
+        hipLaunchKernelGGL((gemm_dma<BM, BN, WM, WN, SA, SB, EP_BF16_RES, kRotateK>), grid, block, 0, st, a, tm, tn, 1u, NoGroup{});
     } else {
       return hipErrorInvalidValue;
     }
   } else if (a.out_dtype == W8A8_OUT_F32) {
-    hipLaunchKernelGGL((gemm_dma<BM, BN, WM, WN, SA, SB, EP_F32, kRotateK>), grid, block, 0, st, a, tm, tn, 1u);
+    hipLaunchKernelGGL((gemm_dma<BM, BN, WM, WN, SA, SB, EP_F32, kRotateK>), grid, block, 0, st, a, tm, tn, 1u, NoGroup{});
   } else {
-    hipLaunchKernelGGL((gemm_dma<BM, BN, WM, WN, SA, SB, EP_BF16, kRotateK>), grid, block, 0, st, a, tm, tn, 1u);
+    hipLaunchKernelGGL((gemm_dma<BM, BN, WM, WN, SA, SB, EP_BF16, kRotateK>), grid, block, 0, st, a, tm, tn, 1u, NoGroup{});
   }
   return hipGetLastError();
 }
@@ -743,9 +762,9 @@ __device__ __forceinline__ void wait_vmcnt_dyn(int n) {
 // records the 100 MHz device clock at its start, once stage 0 has landed
 // (the prologue), after its last MFMA / DMA issue, and once its stores are
 // acknowledged, into stamps[4 g .. 4 g + 3] (g = workgroup * 8 + wave).
-template <int BN, int SA, int SB, int MA, int EP, bool ROT = false, bool TIMED = false>
+template <int BN, int SA, int SB, int MA, int EP, bool ROT = false, bool TIMED = false, bool GROUP = false>
 __global__ __launch_bounds__(512) void gemm_tall(GemmArgs a, uint32_t tiles_n, uint32_t splits,
-                                                 uint64_t* stamps) {
+                                                 uint64_t* stamps, GroupArg<GROUP> group) {
   uint64_t ts[4] = {0, 0, 0, 0};
   if constexpr (TIMED) ts[0] = __builtin_amdgcn_s_memrealtime();
   constexpr int FN = BN / 32;
@@ -765,7 +784,7 @@ __global__ __launch_bounds__(512) void gemm_tall(GemmArgs a, uint32_t tiles_n, u
   uint32_t Lt = blockIdx.x;
   if (G % 8 == 0) Lt = (blockIdx.x % 8) * (G / 8) + blockIdx.x / 8;
   const uint32_t split = Lt / tiles_n;
-  const uint32_t n0 = (Lt % tiles_n) * BN;
+  const uint32_t n0 = own_tile(a, group, Lt % tiles_n) * BN;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const uint32_t K = a.k, KT = K / 128 / splits;
@@ -1271,7 +1290,7 @@ static hipError_t launch_split(hipStream_t st, const GemmArgs& a, uint32_t split
   const uint32_t tm = (a.m + BM - 1) / BM, tn = (a.n + BN - 1) / BN;
   return launch_slabs(st, a, splits, false, [&](auto ep, const GemmArgs& p) {
     hipLaunchKernelGGL((gemm_dma<BM, BN, WM, WN, SA, SB, decltype(ep)::value, false>), dim3(tm * tn * splits),
-                       dim3(512), 0, st, p, tm, tn, splits);
+                       dim3(512), 0, st, p, tm, tn, splits, NoGroup{});
   });
 }
 
@@ -1282,18 +1301,18 @@ static hipError_t launch_tall(hipStream_t st, const GemmArgs& a, uint32_t splits
   if (splits > 1)
     return launch_slabs(st, a, splits, stream_slabs(a, splits), [&](auto ep, const GemmArgs& p) {
       hipLaunchKernelGGL((gemm_tall<BN, SA, SB, MA, decltype(ep)::value, false>), grid, block, 0, st, p, tn, splits,
-                         nullptr);
+                         nullptr, NoGroup{});
     });
   if (a.out_dtype == W8A8_OUT_I32)
-    hipLaunchKernelGGL((gemm_tall<BN, SA, SB, MA, EP_I32, kRotateK>), grid, block, 0, st, a, tn, 1u, nullptr);
+    hipLaunchKernelGGL((gemm_tall<BN, SA, SB, MA, EP_I32, kRotateK>), grid, block, 0, st, a, tn, 1u, nullptr, NoGroup{});
   else if (a.out_dtype == W8A8_OUT_F32 && a.residual)
-    hipLaunchKernelGGL((gemm_tall<BN, SA, SB, MA, EP_F32_RES, kRotateK>), grid, block, 0, st, a, tn, 1u, nullptr);
+    hipLaunchKernelGGL((gemm_tall<BN, SA, SB, MA, EP_F32_RES, kRotateK>), grid, block, 0, st, a, tn, 1u, nullptr, NoGroup{});
   else if (a.out_dtype == W8A8_OUT_F32)
-    hipLaunchKernelGGL((gemm_tall<BN, SA, SB, MA, EP_F32, kRotateK>), grid, block, 0, st, a, tn, 1u, nullptr);
+    hipLaunchKernelGGL((gemm_tall<BN, SA, SB, MA, EP_F32, kRotateK>), grid, block, 0, st, a, tn, 1u, nullptr, NoGroup{});
   else if (a.residual)
-    hipLaunchKernelGGL((gemm_tall<BN, SA, SB, MA, EP_BF16_RES, kRotateK>), grid, block, 0, st, a, tn, 1u, nullptr);
+    hipLaunchKernelGGL((gemm_tall<BN, SA, SB, MA, EP_BF16_RES, kRotateK>), grid, block, 0, st, a, tn, 1u, nullptr, NoGroup{});
   else
-    hipLaunchKernelGGL((gemm_tall<BN, SA, SB, MA, EP_BF16, kRotateK>), grid, block, 0, st, a, tn, 1u, nullptr);
+    hipLaunchKernelGGL((gemm_tall<BN, SA, SB, MA, EP_BF16, kRotateK>), grid, block, 0, st, a, tn, 1u, nullptr, NoGroup{});
   return hipGetLastError();
 }
 
@@ -1306,9 +1325,9 @@ static hipError_t launch_tall_timed(hipStream_t st, const GemmArgs& a, uint32_t 
   if (splits > 1)
     return launch_slabs(st, a, splits, stream_slabs(a, splits), [&](auto ep, const GemmArgs& p) {
       hipLaunchKernelGGL((gemm_tall<BN, SA, SB, MA, decltype(ep)::value, false, true>), grid, block, 0, st, p, tn,
-                         splits, stamps);
+                         splits, stamps, NoGroup{});
     });
-  hipLaunchKernelGGL((gemm_tall<BN, SA, SB, MA, EP_BF16, kRotateK, true>), grid, block, 0, st, a, tn, 1u, stamps);
+  hipLaunchKernelGGL((gemm_tall<BN, SA, SB, MA, EP_BF16, kRotateK, true>), grid, block, 0, st, a, tn, 1u, stamps, NoGroup{});
   return hipGetLastError();
 }
 
@@ -1438,7 +1457,7 @@ hipError_t launch_gemm_timeline(hipStream_t st, const GemmArgs& a, uint64_t* sta
 
 template <int MB, int LAL, int S, int R>
 static hipError_t launch_narrow_as(hipStream_t st, const GemmArgs& a, uint32_t grid) {
-  hipLaunchKernelGGL((gemm_narrow<MB, LAL, S, R>), dim3(grid), dim3(64 * S), 0, st, a);
+  hipLaunchKernelGGL((gemm_narrow<MB, LAL, S, R>), dim3(grid), dim3(64 * S), 0, st, a, NoGroup{});
   return hipGetLastError();
 }
 
@@ -1499,6 +1518,121 @@ hipError_t launch_gemm(hipStream_t st, const GemmArgs& a) {
     }
   }
   return hipErrorInvalidValue;
+}
+
+// ---------------------------------------------------------------- grouped
+template <int MB, int LAL, int S, int R>
+static hipError_t launch_narrow_group(hipStream_t st, const GemmArgs& a, const GemmGroup& g, uint32_t grid) {
+  hipLaunchKernelGGL((gemm_narrow<MB, LAL, S, R, true>), dim3(grid), dim3(64 * S), 0, st, a, g);
+  return hipGetLastError();
+}
+
+template <int BN, int SA, int SB, int MA>
+static hipError_t launch_tall_group(hipStream_t st, const GemmArgs& a, const GemmGroup& g, uint32_t tn) {
+  auto k = a.out_dtype == W8A8_OUT_I32   ? gemm_tall<BN, SA, SB, MA, EP_I32, kRotateK, false, true>
+           : a.out_dtype == W8A8_OUT_F32 ? gemm_tall<BN, SA, SB, MA, EP_F32, kRotateK, false, true>
+                                         : gemm_tall<BN, SA, SB, MA, EP_BF16, kRotateK, false, true>;
+  hipLaunchKernelGGL(k, dim3(tn), dim3(512), 0, st, a, tn, 1u, nullptr, g);
+  return hipGetLastError();
+}
+
+template <int BM, int BN, int WM, int WN, int SA, int SB>
+static hipError_t launch_dma_group(hipStream_t st, const GemmArgs& a, const GemmGroup& g, uint32_t tn) {
+  const uint32_t tm = (a.m + BM - 1) / BM;
+  auto k = a.out_dtype == W8A8_OUT_I32   ? gemm_dma<BM, BN, WM, WN, SA, SB, EP_I32, kRotateK, true>
+           : a.out_dtype == W8A8_OUT_F32 ? gemm_dma<BM, BN, WM, WN, SA, SB, EP_F32, kRotateK, true>
+                                         : gemm_dma<BM, BN, WM, WN, SA, SB, EP_BF16, kRotateK, true>;
+  hipLaunchKernelGGL(k, dim3(tm * tn), dim3(512), 0, st, a, tm, tn, 1u, g);
+  return hipGetLastError();
+}
+
+// The grouped route: the single projection's plans on the siblings' columns
+// together, so a group fills the chip where its matrices alone would not, and
+// pays one launch.  Groups have no workspace, so narrow groups of 17 to 256
+// rows take 32-column one-M-tile workgroups where a single projection would
+// split K.  Measured on MI355X, one launch per matrix -> one launch, per
+// dispatch: gate and up (12288 x 4096 each) at M = 4 24.3 (dot4) -> 18.3 us, at
+// M = 32 2 x 23.1 -> 18.2, at M = 129 2 x 33 -> 30.1, at M = 512 2 x 33.0 ->
+// 58.2; q, k and v (4096 + 1024 + 1024) at M = 4 8.7 (dot4) -> 8.1, at M = 129
+// 14.2 + 2 x 14 -> 20.9, at M = 512 3 x 16.5 -> 24.6, at M = 4096 99 + 2 x 42
+// -> 149.  gate and up at M = 4096 (several rounds of tiles either way) are
+// level.
+GemmRoute gemm_group_route(uint32_t m, uint32_t k, const uint32_t* n, int count) {
+  GemmRoute r{};
+  r.splits = 1;
+  r.grid_y = 1;
+  r.block = 512;
+  if (k % 128 != 0) return r;
+  uint64_t total = 0;
+  for (int i = 0; i < count; ++i) total += n[i];
+  if (total > 0xffffffffu) return r;
+  auto tiles = [&](uint32_t bn) {
+    uint64_t t = 0;
+    for (int i = 0; i < count; ++i) t += (n[i] + bn - 1) / bn;
+    return t;
+  };
+  int S, R, MB, LAL;
+  if (narrow_plan(m, (uint32_t)total, k, S, R, MB, LAL)) {
+    r.family = kRouteNarrow;
+    r.mt = MB, r.s = S, r.u = LAL, r.sa = R;
+    r.bn = 16;
+    r.block = 64 * S;
+    r.grid_x = (uint32_t)tiles(16);
+    return r;
+  }
+  if (m <= 256) {
+    r.family = kRouteTall;
+    r.ma = m <= 64 ? 64 : m <= 160 ? 160 : 256;
+    r.bn = tiles(96) >= 224 ? 96 : 32;
+    if (r.bn == 96) r.sa = r.ma == 256 ? 2 : 4, r.sb = 4;
+    else r.sa = r.sb = r.ma == 64 ? 8 : r.ma == 160 ? 5 : 4;
+    r.grid_x = (uint32_t)tiles(r.bn);
+    return r;
+  }
+  r.family = kRouteDma;
+  const uint64_t m256 = (m + 255) / 256, m128 = (m + 127) / 128;
+  if (m256 * tiles(192) >= 240) r.bm = 256, r.bn = 192, r.wm = 64, r.wn = 96, r.sa = 2, r.sb = 3;
+  else if (m128 * tiles(192) >= 240) r.bm = 128, r.bn = 192, r.wm = 32, r.wn = 96, r.sa = 2, r.sb = 4;
+  else if (total >= 6144) r.bm = 128, r.bn = 128, r.wm = 32, r.wn = 64, r.sa = 4, r.sb = 4;
+  else r.bm = 128, r.bn = 64, r.wm = 32, r.wn = 32, r.sa = 4, r.sb = 4;
+  const uint64_t grid = (m + r.bm - 1) / r.bm * tiles(r.bn);
+  if (grid > 0x7fffffu) return GemmRoute{};
+  r.grid_x = (uint32_t)grid;
+  return r;
+}
+
+hipError_t launch_gemm_group(hipStream_t st, const GemmArgs& a, GemmGroup& g) {
+  const GemmRoute r = gemm_group_route(a.m, a.k, g.n, g.count);
+  if (r.family == kRouteNone) return hipErrorInvalidValue;
+  uint32_t tn = 0;
+  for (int i = 0; i <= kMaxGroup; ++i) {
+    g.tbegin[i] = tn;
+    if (i < g.count) tn += (g.n[i] + r.bn - 1) / r.bn;
+  }
+  if (r.family == kRouteNarrow) {
+    if (r.s == 4) {
+      switch (r.u) {
+        case 1: return launch_narrow_group<1, 1, 4, 4>(st, a, g, tn);
+        case 2: return launch_narrow_group<1, 2, 4, 4>(st, a, g, tn);
+        case 3: return launch_narrow_group<2, 3, 4, 4>(st, a, g, tn);
+        default: return launch_narrow_group<2, 4, 4, 4>(st, a, g, tn);
+      }
+    }
+    return r.u == 1 ? launch_narrow_group<1, 1, 8, 4>(st, a, g, tn) : launch_narrow_group<1, 2, 8, 4>(st, a, g, tn);
+  }
+  if (r.family == kRouteTall) {
+    if (r.bn == 96)
+      return r.ma == 64    ? launch_tall_group<96, 4, 4, 64>(st, a, g, tn)
+             : r.ma == 160 ? launch_tall_group<96, 4, 4, 160>(st, a, g, tn)
+                           : launch_tall_group<96, 2, 4, 256>(st, a, g, tn);
+    return r.ma == 64    ? launch_tall_group<32, 8, 8, 64>(st, a, g, tn)
+           : r.ma == 160 ? launch_tall_group<32, 5, 5, 160>(st, a, g, tn)
+                         : launch_tall_group<32, 4, 4, 256>(st, a, g, tn);
+  }
+  if (r.bm == 256) return launch_dma_group<256, 192, 64, 96, 2, 3>(st, a, g, tn);
+  if (r.bn == 192) return launch_dma_group<128, 192, 32, 96, 2, 4>(st, a, g, tn);
+  if (r.bn == 128) return launch_dma_group<128, 128, 32, 64, 4, 4>(st, a, g, tn);
+  return launch_dma_group<128, 64, 32, 32, 4, 4>(st, a, g, tn);
 }
 
 }  // namespace w8a8

@@ -67,6 +67,18 @@ struct GemmArgs {
   size_t partial_bytes;
 };
 
+// Sibling projections of the same activations (linear_pair / _triple, gate and
+// up) in one GEMM launch: matrix i owns column tiles tbegin[i] ..
+// tbegin[i + 1] - 1 of the grid (tbegin[i] is the total for i >= count).
+struct GemmGroup {
+  int count;
+  const int8_t* w[kMaxGroup];
+  const float* ws[kMaxGroup];
+  void* out[kMaxGroup];
+  uint32_t n[kMaxGroup];
+  uint32_t tbegin[kMaxGroup + 1];  // set by the launcher
+};
+
 // Bytes of split-K workspace launch_gemm would use for this shape (0: none).
 size_t gemm_workspace_bytes(uint32_t m, uint32_t n, uint32_t k);
 
@@ -179,6 +191,11 @@ hipError_t launch_select(hipStream_t st, const float* x, size_t n, uint64_t* key
 size_t argmax_keys_bound(size_t n);
 
 hipError_t launch_gemm(hipStream_t st, const GemmArgs& a);
+// The route of a grouped call (r.bn: columns per tile; kRouteNone where one
+// launch per matrix is the route), and the launch (a: q, asc, m, k,
+// out_dtype; g: the matrices, every n >= 1).
+GemmRoute gemm_group_route(uint32_t m, uint32_t k, const uint32_t* n, int count);
+hipError_t launch_gemm_group(hipStream_t st, const GemmArgs& a, GemmGroup& g);
 
 // One entry of a decode-sequence table (device memory, 64 bytes).
 struct SeqEntry {
