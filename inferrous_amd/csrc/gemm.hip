@@ -405,46 +405,79 @@ __global__ __launch_bounds__(64 * S) void gemm_narrow(GemmArgs a, GroupArg<GROUP
 // is loaded first, at clamped, always valid addresses, and every store comes
 // after the last use of a load: stores count in the same in-order counter
 // as loads, so a load issued after a store would wait for the store too.
-template <int EP, int FM, int FN>
-__device__ __forceinline__ void store_blocks(const GemmArgs& a, const v16i (&acc)[FM][FN], uint32_t row0,
-                                             uint32_t col0, int lane) {
+//
+// FULL: the whole grid of blocks lies inside the output, so nothing is clamped
+// or guarded.  Every address is then a wave-uniform corner (scalar registers)
+// plus one 32-bit lane offset, the same for all values: 4 (l / 32) rows and
+// l % 32 columns (the routes keep N below kMaxCols, so its bytes fit).
+constexpr uint32_t kMaxCols = 1u << 26;
+// Residuals of up to this many values per lane are loaded with the scales; a
+// larger wave tile's, which the registers beside its accumulators do not hold,
+// block by block, the next block's ahead of a block's stores.
+constexpr int kResidualHeld = 64;
+
+template <int EP, bool FULL, int FM, int FN>
+__device__ __forceinline__ void store_blocks_as(const GemmArgs& a, const v16i (&acc)[FM][FN], uint32_t row0,
+                                                uint32_t col0, int lane) {
   constexpr bool RES = EP == EP_F32_RES || EP == EP_BF16_RES;
-  uint32_t rows[FM][16];
+  constexpr bool F32 = EP == EP_F32 || EP == EP_F32_RES;
+  constexpr int ESZ = raw_i32(EP) || F32 ? 4 : 2;
+  const uint32_t half = (uint32_t)lane >> 5, cl = (uint32_t)lane & 31;
+  const uint32_t lane_off = 4 * half * a.n + cl;
+  auto corner_row = [&](int i, int v) -> uint32_t { return row0 + 32 * i + (v >> 2) * 8 + (v & 3); };
+  // byte address of value v of block (i, j) in an array of E-byte elements
+  auto at = [&](const void* p, int i, int v, int j, auto esz) {
+    constexpr uint32_t E = decltype(esz)::value;
+    return (char*)p + ((size_t)corner_row(i, v) * a.n + col0 + 32 * j) * E + (size_t)(lane_off * E);
+  };
+  using E4 = std::integral_constant<uint32_t, 4>;
+  using EO = std::integral_constant<uint32_t, ESZ>;
+  auto inside = [&](int i, int v, int j) {
+    return FULL || (corner_row(i, v) + 4 * half < a.m && col0 + 32 * j + cl < a.n);
+  };
+  if constexpr (raw_i32(EP)) {
 #pragma unroll
-  for (int i = 0; i < FM; ++i)
-#pragma unroll
-    for (int v = 0; v < 16; ++v) rows[i][v] = row0 + 32 * i + (v >> 2) * 8 + (lane >> 5) * 4 + (v & 3);
-  if (raw_i32(EP)) {
-#pragma unroll
-    for (int j = 0; j < FN; ++j) {
-      const uint32_t c = col0 + 32 * j + (lane & 31);
+    for (int j = 0; j < FN; ++j)
 #pragma unroll
       for (int i = 0; i < FM; ++i)
 #pragma unroll
         for (int v = 0; v < 16; ++v)
-          if (rows[i][v] < a.m && c < a.n) {
-            int32_t* o = reinterpret_cast<int32_t*>(a.out) + (size_t)rows[i][v] * a.n + c;
+          if (inside(i, v, j)) {
+            int32_t* const o = (int32_t*)at(a.out, i, v, j, EO{});
             if (EP == EP_SLAB) __builtin_nontemporal_store(acc[i][j][v], o);
             else *o = acc[i][j][v];
           }
-    }
     return;
   }
+  constexpr int NB = FM * FN;  // block b: row block b % FM, column block b / FM
+  constexpr bool HELD = NB * 16 <= kResidualHeld;
+  constexpr int SLOTS = HELD ? NB : 2;
   float asc[FM][16], wsc[FN];
-  float res[RES ? FM : 1][RES ? FN : 1][16];
+  float res[RES ? SLOTS : 1][16];
+  auto load_res = [&](int b) {
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      const int i = b % FM, j = b / FM;
+      res[b % SLOTS][v] =
+          FULL ? *(const float*)at(a.residual, i, v, j, E4{})
+               : a.residual[(size_t)min(corner_row(i, v) + 4 * half, a.m - 1) * a.n + min(col0 + 32 * j + cl, a.n - 1)];
+    }
+  };
 #pragma unroll
   for (int i = 0; i < FM; ++i)
 #pragma unroll
-    for (int v = 0; v < 16; ++v) asc[i][v] = a.asc[min(rows[i][v], a.m - 1)];
+    for (int v = 0; v < 16; ++v) {
+      const uint32_t r = corner_row(i, v) + 4 * half;
+      asc[i][v] = a.asc[FULL ? r : min(r, a.m - 1)];
+    }
 #pragma unroll
   for (int j = 0; j < FN; ++j) {
-    const uint32_t cc = min(col0 + 32 * j + (lane & 31), a.n - 1);
-    wsc[j] = a.ws[cc];
-    if (RES)
+    const uint32_t c = col0 + 32 * j + cl;
+    wsc[j] = a.ws[FULL ? c : min(c, a.n - 1)];
+  }
+  if constexpr (RES) {
 #pragma unroll
-      for (int i = 0; i < FM; ++i)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) res[i][j][v] = a.residual[(size_t)min(rows[i][v], a.m - 1) * a.n + cc];
+    for (int b = 0; b < (HELD ? NB : 1); ++b) load_res(b);
   }
   // one wait for every load above, taken unconditionally: a wait first met
   // inside a guarded store would be repeated in each guarded store after it
@@ -454,28 +487,37 @@ __device__ __forceinline__ void store_blocks(const GemmArgs& a, const v16i (&acc
   // with random operands: o at M = 512 16.8 against 17.2-17.4 us, qkv
   // 22.5-22.7 against 23.0-23.3, gate_up at M = 129 30.9 against 31.2-31.4.
 #pragma unroll
-  for (int j = 0; j < FN; ++j) {
-    const uint32_t c = col0 + 32 * j + (lane & 31);
+  for (int b = 0; b < NB; ++b) {
+    const int i = b % FM, j = b / FM;
+    if constexpr (RES && !HELD) {
+      __builtin_amdgcn_sched_barrier(0);
+      if (b + 1 < NB) load_res(b + 1);
+      __builtin_amdgcn_sched_barrier(0);
+    }
 #pragma unroll
-    for (int i = 0; i < FM; ++i)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const uint32_t r = rows[i][v];
-        const float val = dequant(acc[i][j][v], asc[i][v], wsc[j]);
-        if (r >= a.m || c >= a.n) continue;
-        const size_t o = (size_t)r * a.n + c;
-        if (EP == EP_F32 || EP == EP_F32_RES) {
-          if (a.out) __builtin_nontemporal_store(val, reinterpret_cast<float*>(a.out) + o);
-          if (RES) reinterpret_cast<float*>(a.combined)[o] = bf16_rne(res[RES ? i : 0][RES ? j : 0][v] + val);
-        } else {
-          if (a.out)
-            __builtin_nontemporal_store((uint16_t)(__float_as_uint(val) >> 16), reinterpret_cast<uint16_t*>(a.out) + o);
-          if (RES)
-            reinterpret_cast<uint16_t*>(a.combined)[o] =
-                (uint16_t)(__float_as_uint(bf16_rne(res[RES ? i : 0][RES ? j : 0][v] + val)) >> 16);
-        }
+    for (int v = 0; v < 16; ++v) {
+      const float val = dequant(acc[i][j][v], asc[i][v], wsc[j]);
+      const float cmb = RES ? bf16_rne(res[RES ? b % SLOTS : 0][v] + val) : 0.f;
+      if (!inside(i, v, j)) continue;
+      if constexpr (F32) {
+        if (a.out) __builtin_nontemporal_store(val, (float*)at(a.out, i, v, j, EO{}));
+        if (RES) *(float*)at(a.combined, i, v, j, EO{}) = cmb;
+      } else {
+        if (a.out)
+          __builtin_nontemporal_store((uint16_t)(__float_as_uint(val) >> 16), (uint16_t*)at(a.out, i, v, j, EO{}));
+        if (RES) *(uint16_t*)at(a.combined, i, v, j, EO{}) = (uint16_t)(__float_as_uint(cmb) >> 16);
       }
+    }
   }
+}
+
+template <int EP, int FM, int FN>
+__device__ __forceinline__ void store_blocks(const GemmArgs& a, const v16i (&acc)[FM][FN], uint32_t row0,
+                                             uint32_t col0, int lane) {
+  if (row0 + 32 * FM <= a.m && col0 + 32 * FN <= a.n)
+    store_blocks_as<EP, true, FM, FN>(a, acc, row0, col0, lane);
+  else
+    store_blocks_as<EP, false, FM, FN>(a, acc, row0, col0, lane);
 }
 
 // Prefill GEMM.  Workgroup = 8 waves (two per SIMD: while one wave waits on
@@ -499,7 +541,17 @@ __device__ __forceinline__ void store_blocks(const GemmArgs& a, const v16i (&acc
 // hit sixteen different 16-byte bank groups.  Sub-step i of a stage covers
 // k bytes [32i, 32i + 32): lane l (row / column l % 32, half h = l / 32)
 // reads chunk 2i + h -- the same lane -> k map for A and B.
-template <int BM, int BN, int WM, int WN, int SA, int SB, int EP, bool ROT = false, bool GROUP = false>
+// Tiles are numbered XCD-aware (each XCD a contiguous run) and, within that,
+// in strips of kStrip M tiles that walk all N tiles, so that the 32 tiles an
+// XCD runs at once are about 4 x 8: they share 4 activation and 8 weight
+// panels through its L2 while they advance through K together.  M fastest over
+// all M tiles instead, with each tile starting K at its own stage, fetched
+// most panels once per tile: 24576 x 4096 at M = 4096, f32, 256 x 192 tiles
+// 484 -> 443 us; strips of 4 / 8 / 16 on 256 x 256 tiles 387 / 397 / 430.
+constexpr uint32_t kStrip = 4;
+constexpr uint32_t kMaxK = 1u << 23;  // 256 rows of K bytes stay within a 32-bit offset
+
+template <int BM, int BN, int WM, int WN, int SA, int SB, int EP, bool GROUP = false>
 __global__ __launch_bounds__(512) void gemm_dma(GemmArgs a, uint32_t tiles_m, uint32_t tiles_n,
                                                 uint32_t splits, GroupArg<GROUP> group) {
   constexpr int WAVES_N = BN / WN;
@@ -523,7 +575,9 @@ __global__ __launch_bounds__(512) void gemm_dma(GemmArgs a, uint32_t tiles_m, ui
   if (G % 8 == 0) Lt = (blockIdx.x % 8) * (G / 8) + blockIdx.x / 8;
   const uint32_t split = Lt / T;
   Lt %= T;
-  const uint32_t m0 = (Lt % tiles_m) * BM, n0 = own_tile(a, group, Lt / tiles_m) * BN;
+  const uint32_t strip = kStrip * (T / tiles_m), s0 = Lt / strip * kStrip, in = Lt % strip;
+  const uint32_t sm = min(kStrip, tiles_m - s0);  // M tiles of this strip
+  const uint32_t m0 = (s0 + in % sm) * BM, n0 = own_tile(a, group, in / sm) * BN;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int wm0 = (wave / WAVES_N) * WM, wn0 = (wave % WAVES_N) * WN;
@@ -532,49 +586,34 @@ __global__ __launch_bounds__(512) void gemm_dma(GemmArgs a, uint32_t tiles_m, ui
   if (raw_i32(EP)) a.out = reinterpret_cast<int32_t*>(a.out) + (size_t)split * a.m * a.n;
 
   // Sources of this wave's DMA loads (8 rows each); rows past M / N re-read
-  // row 0 (their products only reach accumulator cells that are never
+  // the tile's first row (their products only reach accumulator cells that are never
   // stored).  Lane l fills LDS chunk l % 8 of row l / 8 with global chunk
   // (l % 8) ^ key(row).
-  const int8_t* srcA[LA];
-  const int8_t* srcB[LB];
+  // An address is the tile's first row (scalar registers) plus a 32-bit lane
+  // offset (the routes keep K at kMaxK and below).
+  const int8_t* const srcA = a.q + (size_t)m0 * K + kbase;
+  const int8_t* const srcB = a.w + (size_t)n0 * K + kbase;
+  uint32_t offA[LA], offB[LB];
 #pragma unroll
   for (int j = 0; j < LA; ++j) {
-    const int row = 8 * (wave * LA + j) + (lane >> 3);
-    const uint32_t g = m0 + row;
-    srcA[j] = a.q + (size_t)(g < a.m ? g : 0) * K + kbase + ((lane & 7) ^ ((row >> 1) & 7)) * 16;
+    const uint32_t row = 8 * (wave * LA + j) + (lane >> 3);
+    offA[j] = (m0 + row < a.m ? row : 0) * K + ((lane & 7) ^ ((row >> 1) & 7)) * 16;
   }
 #pragma unroll
   for (int j = 0; j < LB; ++j) {
-    const int row = 8 * (wave * LB + j) + (lane >> 3);
-    const uint32_t g = n0 + row;
-    srcB[j] = a.w + (size_t)(g < a.n ? g : 0) * K + kbase + ((lane & 7) ^ ((row >> 1) & 7)) * 16;
+    const uint32_t row = 8 * (wave * LB + j) + (lane >> 3);
+    offB[j] = (n0 + row < a.n ? row : 0) * K + ((lane & 7) ^ ((row >> 1) & 7)) * 16;
   }
-  // ROT: stage kt reads global K chunk (kt + rot) mod KT, rot = tile mod KT.
-  const uint32_t rot = ROT ? Lt % KT : 0;
-  auto kc = [&](uint32_t kt) -> size_t {
-    const uint32_t c = kt + rot;
-    return (size_t)(c >= KT ? c - KT : c) * 128;
-  };
   auto loadA = [&](uint32_t kt, int j) {
-    __builtin_amdgcn_global_load_lds((const void*)(srcA[j] + kc(kt)),
+    __builtin_amdgcn_global_load_lds((const void*)(srcA + (size_t)kt * 128 + offA[j]),
                                      W8A8_LDS_PTR(ldsA + (kt % SA) * ASL + (wave * LA + j) * 1024 + lane * 16),
                                      16, 0, 0);
   };
   auto loadB = [&](uint32_t kt, int j) {
-    __builtin_amdgcn_global_load_lds((const void*)(srcB[j] + kc(kt)),
+    __builtin_amdgcn_global_load_lds((const void*)(srcB + (size_t)kt * 128 + offB[j]),
                                      W8A8_LDS_PTR(ldsB + (kt % SB) * BSL + (wave * LB + j) * 1024 + lane * 16),
                                      16, 0, 0);
   };
-  // Batch(kt), A first.
-  auto batch = [&](uint32_t kt) {
-    if (kt + SA - 1 < KT)
-#pragma unroll
-      for (int j = 0; j < LA; ++j) loadA(kt + SA - 1, j);
-    if (kt + SB - 1 < KT)
-#pragma unroll
-      for (int j = 0; j < LB; ++j) loadB(kt + SB - 1, j);
-  };
-
   const int fr = lane & 31, fh = lane >> 5;
   int off[4];
 #pragma unroll
@@ -598,6 +637,25 @@ __global__ __launch_bounds__(512) void gemm_dma(GemmArgs a, uint32_t tiles_m, ui
 #pragma unroll
       for (int j = 0; j < FN; ++j) acc[f][j] = mfma32(af[f], bf[j], acc[f][j]);
   };
+  // The same MFMAs with the loads load(0) .. load(N - 1) issued evenly between
+  // them, and kept there: the wave's MFMAs do not queue behind a burst of DMA
+  // issues after the barrier.
+  auto mm_load = [&](const v4i (&af)[FM], const v4i (&bf)[FN], auto n, auto load) {
+    constexpr int N = decltype(n)::value, MF = FM * FN;
+#pragma unroll
+    for (int i = 0; i < MF; ++i) {
+      acc[i / FN][i % FN] = mfma32(af[i / FN], bf[i % FN], acc[i / FN][i % FN]);
+      const int lo = (i * N + MF - 1) / MF, hi = ((i + 1) * N + MF - 1) / MF;
+      if (lo == hi) continue;
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int j = 0; j < N; ++j)
+        if (j >= lo && j < hi) load(j);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  using LoadsA = std::integral_constant<int, LA>;
+  using LoadsB = std::integral_constant<int, LB>;
 
   // Prologue: stages 0 .. SB - 2 (A only up to SA - 2), stage by stage, A
   // before B; then wait for stage 0.
@@ -614,28 +672,38 @@ __global__ __launch_bounds__(512) void gemm_dma(GemmArgs a, uint32_t tiles_m, ui
   else wait_vmcnt<0>();
   __builtin_amdgcn_s_barrier();
   v4i a0[FM], b0[FN], a1[FM], b1[FN];
-  batch(0);
+  if (SA - 1 < KT)
+#pragma unroll
+    for (int j = 0; j < LA; ++j) loadA(SA - 1, j);
   rd(0, 0, a0, b0);
   // Fragments of the next sub-step are read while the current one's MFMAs
   // run.  The loop body has no branch between a read and its use, so the
-  // compiler's LDS waits keep the newest reads in flight.
-  for (uint32_t kt = 0; kt + 1 < KT; ++kt) {
+  // compiler's LDS waits keep the newest reads in flight.  Batch(kt) goes out
+  // among the MFMAs of two sub-steps: A(kt + SA - 1) with the last ones of
+  // stage kt - 1 (after the barrier that released its slot), B(kt + SB - 1)
+  // with the first ones of stage kt.
+  auto stage = [&](uint32_t kt, auto all) {
+    constexpr bool ALL = decltype(all)::value;  // every load of this stage exists
+    const bool more_b = ALL || kt + SB - 1 < KT, more_a = ALL || kt + SA < KT;
     rd(kt, 1, a1, b1);
-    mm(a0, b0);
+    mm_load(a0, b0, LoadsB{}, [&](int j) { if (more_b) loadB(kt + SB - 1, j); });
     rd(kt, 2, a0, b0);
     mm(a1, b1);
     rd(kt, 3, a1, b1);
     mm(a0, b0);
     // A(kt + 1), B(kt + 1) landed (every load counted here exists while batch
     // kt was complete)
-    if (kt + SB - 1 < KT) wait_vmcnt<(SB > SA ? LB : 0) + (SA - 2) * L>();
+    if (more_b) wait_vmcnt<(SB > SA ? LB : 0) + (SA - 2) * L>();
     else wait_vmcnt<0>();
     __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): this wave's reads of stage kt returned
     __builtin_amdgcn_s_barrier();         // all waves: stage kt + 1 landed, stage kt read
-    batch(kt + 1);                        // into the slots stage kt released
     rd(kt + 1, 0, a0, b0);
-    mm(a1, b1);
-  }
+    mm_load(a1, b1, LoadsA{}, [&](int j) { if (more_a) loadA(kt + SA, j); });
+  };
+  uint32_t kt = 0;
+  constexpr uint32_t AHEAD = SB > SA ? SB - 1 : SA;
+  for (; kt + AHEAD < KT; ++kt) stage(kt, std::true_type{});
+  for (; kt + 1 < KT; ++kt) stage(kt, std::false_type{});
   rd(KT - 1, 1, a1, b1);
   mm(a0, b0);
   rd(KT - 1, 2, a0, b0);
@@ -647,48 +715,15 @@ __global__ __launch_bounds__(512) void gemm_dma(GemmArgs a, uint32_t tiles_m, ui
   store_blocks<EP, FM, FN>(a, acc, m0 + wm0, n0 + wn0, lane);
 }
 
-// Unsplit launches rotate each workgroup's K order (stage kt reads K chunk
-// (kt + tile) mod KT; the i32 sums are exact in any order, so outputs are
-// bit-identical).  Otherwise every workgroup reads the same 128-byte column
-// of its 4 KiB weight rows at the same time.  Measured on MI355X (graphs of 16
-// distinct-weight launches): gate_up 24576 x 4096 at M = 64 22.2 against
-// 25.1 us, M = 100 33.8 against 35.2, M = 129 29.4-29.7 against 30.3-31.4,
-// M = 193 32.8 against 34.5-35.0, M = 300 51.7-53.3 against 54.2-54.8,
-// M = 512 54.6-56.1 against 56.0-58.8; qkv at M = 512 21.9-22.5 against
-// 22.3-22.7; o level.  In the 36-layer prefill graphs, where each gate_up
-// follows qkv and o, the M = 512 and M = 129 totals came out level (A/B on
-// one box) while the ragged gate_up at M = 16 went from 4.20 to 4.85 TB/s.
-// Split-K launches, whose slabs already start at different K offsets,
-// measured level or up to 1.3% slower rotated, and keep the order.
-constexpr bool kRotateK = true;
-
-// The residual epilogue holds a residual per accumulator; with a 64 x 96
-// wave tile that is 96 more registers than the kernel has, and it spills.
-// Such tiles take no residual (launch_gemm routes residual outputs to
-// 128-row tiles).
-template <int WM, int WN>
-constexpr bool kResidualTile = WM * WN <= 32 * 96;
-
 template <int BM, int BN, int WM, int WN, int SA, int SB>
 static hipError_t launch_dma(hipStream_t st, const GemmArgs& a) {
   const uint32_t tm = (a.m + BM - 1) / BM, tn = (a.n + BN - 1) / BN;
   const dim3 grid(tm * tn), block(512);
-  if (a.out_dtype == W8A8_OUT_I32) {
-    hipLaunchKernelGGL((gemm_dma<BM, BN, WM, WN, SA, SB, EP_I32, kRotateK>), grid, block, 0, st, a, tm, tn, 1u, NoGroup{});
-  } else if (a.residual) {
-    if constexpr (kResidualTile<WM, WN>) {
-      if (a.out_dtype == W8A8_OUT_F32)
-        hipLaunchKernelGGL((gemm_dma<BM, BN, WM, WN, SA, SB, EP_F32_RES, kRotateK>), grid, block, 0, st, a, tm, tn, 1u, NoGroup{});
-      else
-        hipLaunchKernelGGL((gemm_dma<BM, BN, WM, WN, SA, SB, EP_BF16_RES, kRotateK>), grid, block, 0, st, a, tm, tn, 1u, NoGroup{});
-    } else {
-      return hipErrorInvalidValue;
-    }
-  } else if (a.out_dtype == W8A8_OUT_F32) {
-    hipLaunchKernelGGL((gemm_dma<BM, BN, WM, WN, SA, SB, EP_F32, kRotateK>), grid, block, 0, st, a, tm, tn, 1u, NoGroup{});
-  } else {
-    hipLaunchKernelGGL((gemm_dma<BM, BN, WM, WN, SA, SB, EP_BF16, kRotateK>), grid, block, 0, st, a, tm, tn, 1u, NoGroup{});
-  }
+  auto k = a.out_dtype == W8A8_OUT_I32 ? gemm_dma<BM, BN, WM, WN, SA, SB, EP_I32>
+           : a.out_dtype == W8A8_OUT_F32
+               ? (a.residual ? gemm_dma<BM, BN, WM, WN, SA, SB, EP_F32_RES> : gemm_dma<BM, BN, WM, WN, SA, SB, EP_F32>)
+               : (a.residual ? gemm_dma<BM, BN, WM, WN, SA, SB, EP_BF16_RES> : gemm_dma<BM, BN, WM, WN, SA, SB, EP_BF16>);
+  hipLaunchKernelGGL(k, grid, block, 0, st, a, tm, tn, 1u, NoGroup{});
   return hipGetLastError();
 }
 
@@ -758,10 +793,20 @@ __device__ __forceinline__ void wait_vmcnt_dyn(int n) {
 // and counts its waits with its own na, nb.  During stage kt it issues
 // A(kt + SA - 1), then B(kt + SB - 1).
 // Split-K as in gemm_dma: workgroup (tile, split) writes i32 slab `split`.
+// ROT (unsplit launches): each workgroup starts K at its own stage (stage kt
+// reads K chunk (kt + tile) mod KT; the i32 sums are exact in any order), so
+// that the workgroups do not all read the same 128-byte column of their
+// weight rows at once.  Measured on MI355X (graphs of 16 distinct-weight
+// launches): gate_up 24576 x 4096 at M = 64 22.2 against 25.1 us, M = 129
+// 29.4-29.7 against 30.3-31.4, M = 193 32.8 against 34.5-35.0.  Split-K
+// launches, whose slabs already start at different K offsets, measured level
+// or up to 1.3% slower rotated, and keep the order.
 // TIMED (diagnostics only, w8a8_diag_gemm_timeline): every wave also
 // records the 100 MHz device clock at its start, once stage 0 has landed
 // (the prologue), after its last MFMA / DMA issue, and once its stores are
 // acknowledged, into stamps[4 g .. 4 g + 3] (g = workgroup * 8 + wave).
+constexpr bool kRotateK = true;
+
 template <int BN, int SA, int SB, int MA, int EP, bool ROT = false, bool TIMED = false, bool GROUP = false>
 __global__ __launch_bounds__(512) void gemm_tall(GemmArgs a, uint32_t tiles_n, uint32_t splits,
                                                  uint64_t* stamps, GroupArg<GROUP> group) {
@@ -1111,14 +1156,65 @@ __global__ __launch_bounds__(256) void splitk_epilogue8(GemmArgs a, const int32_
   }
 }
 
-// gemm_dma's split-K plan (128 x 128 tiles, two slabs): M > 256 at K >= 8192,
-// the down projection's few, long tiles (measured on MI355X at M = 300 and
-// 512).  gemm_tall's plan covers M <= 256.
+// gemm_dma's tiles, and the time one takes with every CU busy: fixed + stages
+// x 128-byte K stages (ns, fitted to the launches below).  A launch runs its
+// tiles in rounds of one per CU, so the route is the tile with the least
+// rounds x time: large tiles move the fewest operand bytes per product but
+// leave CUs idle in their last round, small ones the other way about.
+// Measured on MI355X with random operands, us per launch (256 x 256 / 256 x 192
+// / 256 x 128 / 128 x 192 / 128 x 128 / 128 x 64): 24576 x 4096 f32 at M = 4096
+// 393 / 417 / 439 / 488 / 537 / -; 6144 x 4096 BF16 at M = 4096 112 / 97.7 / 103 /
+// 113 / 126 / -, at M = 1024 - / - / 30.3 / 28.1 / 38.2 / 39.4, at M = 512 - / - /
+// - / 23.5 / 19.4 / 25.5; 4096 x 4096 f32 with the residual at M = 4096 87 / - /
+// 91 / 103 / 112 / -, at M = 1024 - / - / 36 / 29.1 / 26.9 / 29.8, at M = 512 - /
+// - / 33.7 / 25.7 / 21.0 / 16.7; 4096 x 12288 likewise at M = 4096 196 / - / 211 /
+// - / 257 / -, at M = 512 - / - / 84 / 72 / 58 / 44.7.
+struct DmaTile {
+  int bm, bn, wm, wn, sa, sb;
+  uint32_t fixed, stage;
+};
+static const DmaTile kDmaTiles[] = {
+    {256, 256, 64, 128, 2, 3, 11000, 1700}, {256, 192, 64, 96, 2, 3, 10000, 1270},
+    {256, 128, 64, 64, 2, 4, 7000, 940},    {128, 192, 32, 96, 2, 4, 5000, 740},
+    {128, 128, 32, 64, 4, 4, 3000, 590},    {128, 64, 32, 32, 4, 4, 2500, 440},
+    {64, 128, 32, 32, 4, 4, 2500, 440},
+};
+constexpr uint64_t kCus = 256;
+
+// The cheapest tile for m rows and k, tiles_n(bn) column tiles.
+template <typename TilesN>
+static const DmaTile& dma_tile(uint32_t m, uint32_t k, TilesN tiles_n) {
+  const DmaTile* best = nullptr;
+  uint64_t least = ~0ull;
+  for (const DmaTile& t : kDmaTiles) {
+    const uint64_t tiles = (uint64_t)((m + t.bm - 1) / t.bm) * tiles_n(t.bn);
+    const uint64_t c = (tiles + kCus - 1) / kCus * (t.fixed + (uint64_t)(k / 128) * t.stage);
+    if (c < least) least = c, best = &t;
+  }
+  return *best;
+}
+
+static void set_tile(GemmRoute& r, const DmaTile& t) {
+  r.bm = t.bm, r.bn = t.bn, r.wm = t.wm, r.wn = t.wn, r.sa = t.sa, r.sb = t.sb;
+}
+
+// Whether gemm_dma and gemm_tall take the shape: K in whole 128-byte stages, and
+// their 32-bit lane offsets (kMaxK, kMaxCols).
+static bool staged_shape(uint32_t n, uint32_t k) { return k % 128 == 0 && k <= kMaxK && n <= kMaxCols; }
+
+// gemm_dma's split-K plan (128 x 128 tiles, two slabs): M > 256 at K >= 8192
+// where those tiles, unsplit, would leave more than a third of the CUs idle
+// for a long K (4096 x 12288 at M = 512: 36 + 8 us for the slab epilogue
+// against 58 unsplit and 44.7 on 128 x 64 tiles).  With more tiles the
+// slabs cost more than the CUs they fill: at M = 4096 288 + 64 us against 196
+// on 256 x 256 tiles.  A single column of tiles (N <= 128) keeps the plan at any
+// M.  gemm_tall's plan covers M <= 256.
 static bool split_plan(uint32_t m, uint32_t n, uint32_t k, uint32_t& splits) {
-  if (m <= 256 || k < 8192 || k % 128 != 0 || n % 4 != 0) return false;
+  if (m <= 256 || k < 8192 || !staged_shape(n, k) || n % 4 != 0) return false;
   const uint32_t kt = k / 128;
   splits = 2;
-  return kt % splits == 0 && kt / splits >= 4;
+  const uint64_t tiles = (uint64_t)((m + 127) / 128) * ((n + 127) / 128);
+  return kt % splits == 0 && kt / splits >= 4 && (tiles * 3 <= kCus * 2 || n <= 128);
 }
 
 // gemm_narrow's plan: S = 4 waves below K = 8192 and 8 from there (each wave
@@ -1176,7 +1272,7 @@ static bool narrow_plan(uint32_t m, uint32_t n, uint32_t k, int& S, int& R, int&
 // Returns false when no plan applies (the gemm_dma or gemm_skinny routes
 // then run).  ma: the M tile (64, 160 or 256 rows).
 static bool tall_plan(uint32_t m, uint32_t n, uint32_t k, int& bn, uint32_t& splits, int& ma) {
-  if (m == 0 || m > 256 || k % 128 != 0) return false;
+  if (m == 0 || m > 256 || !staged_shape(n, k)) return false;
   ma = m <= 64 ? 64 : m <= 160 ? 160 : 256;
   const uint32_t kt = k / 128, t96 = (n + 95) / 96;
   if (t96 >= 224) {
@@ -1289,7 +1385,7 @@ template <int BM, int BN, int WM, int WN, int SA, int SB>
 static hipError_t launch_split(hipStream_t st, const GemmArgs& a, uint32_t splits) {
   const uint32_t tm = (a.m + BM - 1) / BM, tn = (a.n + BN - 1) / BN;
   return launch_slabs(st, a, splits, false, [&](auto ep, const GemmArgs& p) {
-    hipLaunchKernelGGL((gemm_dma<BM, BN, WM, WN, SA, SB, decltype(ep)::value, false>), dim3(tm * tn * splits),
+    hipLaunchKernelGGL((gemm_dma<BM, BN, WM, WN, SA, SB, decltype(ep)::value>), dim3(tm * tn * splits),
                        dim3(512), 0, st, p, tm, tn, splits, NoGroup{});
   });
 }
@@ -1357,7 +1453,7 @@ GemmRoute gemm_route(const GemmArgs& a) {
   // Otherwise, for small m: from m = 8 the 8-wave kernel with 64-row tiles
   // streams the weights faster when n gives at least 128 tiles; below that
   // the skinny kernel's split-K keeps more CUs busy.
-  const bool wide = a.m >= 8 && a.k % 128 == 0 && (a.n + 127) / 128 >= 128;
+  const bool wide = a.m >= 8 && staged_shape(a.n, a.k) && (a.n + 127) / 128 >= 128;
   {
     int tile, ma;
     uint32_t splits;
@@ -1404,26 +1500,17 @@ GemmRoute gemm_route(const GemmArgs& a) {
     r.block = 64 * r.s;
     return r;
   }
-  if (a.k % 128 == 0) {
+  if (staged_shape(a.n, a.k)) {
     r.family = kRouteDma;
     uint32_t splits;
     if (a.partials && split_plan(a.m, a.n, a.k, splits) &&
         a.partial_bytes >= (size_t)splits * a.m * a.n * sizeof(int32_t)) {
-      r.bm = 128, r.bn = 128, r.wm = 32, r.wn = 64, r.sa = 4, r.sb = 4;
+      set_tile(r, kDmaTiles[4]);
       r.splits = splits;
       r.epi_cols = wide_epilogue(a) ? 8 : 4;
     } else {
-      // Tile per problem, measured on MI355X at M = 129 / 512 on the Qwen3-8B
-      // projection shapes: the largest tile that still gives about one tile
-      // per CU, smaller tiles for narrow N.  Residual outputs skip the
-      // 256 x 192 tile (kResidualTile); t128 is then at least 480.
-      const uint64_t t256 = (uint64_t)((a.m + 255) / 256) * ((a.n + 191) / 192);
-      const uint64_t t128 = (uint64_t)((a.m + 127) / 128) * ((a.n + 191) / 192);
-      if (t256 >= 240 && !a.residual) r.bm = 256, r.bn = 192, r.wm = 64, r.wn = 96, r.sa = 2, r.sb = 3;
-      else if (t128 >= 240) r.bm = 128, r.bn = 192, r.wm = 32, r.wn = 96, r.sa = 2, r.sb = 4;
-      else if (a.n >= 6144 && a.m >= 256) r.bm = 128, r.bn = 128, r.wm = 32, r.wn = 64, r.sa = 4, r.sb = 4;
-      else if (a.m >= 128) r.bm = 128, r.bn = 64, r.wm = 32, r.wn = 32, r.sa = 4, r.sb = 4;
-      else r.bm = 64, r.bn = 128, r.wm = 32, r.wn = 32, r.sa = 4, r.sb = 4;
+      set_tile(r, a.m <= 64 ? kDmaTiles[6]
+                            : dma_tile(a.m, a.k, [&](uint32_t bn) { return (uint64_t)(a.n + bn - 1) / bn; }));
     }
     r.grid_x = (a.m + r.bm - 1) / r.bm * ((a.n + r.bn - 1) / r.bn) * r.splits;
     return r;
@@ -1506,7 +1593,9 @@ hipError_t launch_gemm(hipStream_t st, const GemmArgs& a) {
       return hipGetLastError();
     case kRouteDma:
       if (r.splits > 1) return launch_split<128, 128, 32, 64, 4, 4>(st, a, r.splits);
+      if (is(256, 256, 64, 128, 2, 3)) return launch_dma<256, 256, 64, 128, 2, 3>(st, a);
       if (is(256, 192, 64, 96, 2, 3)) return launch_dma<256, 192, 64, 96, 2, 3>(st, a);
+      if (is(256, 128, 64, 64, 2, 4)) return launch_dma<256, 128, 64, 64, 2, 4>(st, a);
       if (is(128, 192, 32, 96, 2, 4)) return launch_dma<128, 192, 32, 96, 2, 4>(st, a);
       if (is(128, 128, 32, 64, 4, 4)) return launch_dma<128, 128, 32, 64, 4, 4>(st, a);
       if (is(128, 64, 32, 32, 4, 4)) return launch_dma<128, 64, 32, 32, 4, 4>(st, a);
@@ -1539,9 +1628,9 @@ static hipError_t launch_tall_group(hipStream_t st, const GemmArgs& a, const Gem
 template <int BM, int BN, int WM, int WN, int SA, int SB>
 static hipError_t launch_dma_group(hipStream_t st, const GemmArgs& a, const GemmGroup& g, uint32_t tn) {
   const uint32_t tm = (a.m + BM - 1) / BM;
-  auto k = a.out_dtype == W8A8_OUT_I32   ? gemm_dma<BM, BN, WM, WN, SA, SB, EP_I32, kRotateK, true>
-           : a.out_dtype == W8A8_OUT_F32 ? gemm_dma<BM, BN, WM, WN, SA, SB, EP_F32, kRotateK, true>
-                                         : gemm_dma<BM, BN, WM, WN, SA, SB, EP_BF16, kRotateK, true>;
+  auto k = a.out_dtype == W8A8_OUT_I32   ? gemm_dma<BM, BN, WM, WN, SA, SB, EP_I32, true>
+           : a.out_dtype == W8A8_OUT_F32 ? gemm_dma<BM, BN, WM, WN, SA, SB, EP_F32, true>
+                                         : gemm_dma<BM, BN, WM, WN, SA, SB, EP_BF16, true>;
   hipLaunchKernelGGL(k, dim3(tm * tn), dim3(512), 0, st, a, tm, tn, 1u, g);
   return hipGetLastError();
 }
@@ -1562,10 +1651,9 @@ GemmRoute gemm_group_route(uint32_t m, uint32_t k, const uint32_t* n, int count)
   r.splits = 1;
   r.grid_y = 1;
   r.block = 512;
-  if (k % 128 != 0) return r;
   uint64_t total = 0;
   for (int i = 0; i < count; ++i) total += n[i];
-  if (total > 0xffffffffu) return r;
+  if (total > kMaxCols || !staged_shape((uint32_t)total, k)) return r;
   auto tiles = [&](uint32_t bn) {
     uint64_t t = 0;
     for (int i = 0; i < count; ++i) t += (n[i] + bn - 1) / bn;
@@ -1590,11 +1678,7 @@ GemmRoute gemm_group_route(uint32_t m, uint32_t k, const uint32_t* n, int count)
     return r;
   }
   r.family = kRouteDma;
-  const uint64_t m256 = (m + 255) / 256, m128 = (m + 127) / 128;
-  if (m256 * tiles(192) >= 240) r.bm = 256, r.bn = 192, r.wm = 64, r.wn = 96, r.sa = 2, r.sb = 3;
-  else if (m128 * tiles(192) >= 240) r.bm = 128, r.bn = 192, r.wm = 32, r.wn = 96, r.sa = 2, r.sb = 4;
-  else if (total >= 6144) r.bm = 128, r.bn = 128, r.wm = 32, r.wn = 64, r.sa = 4, r.sb = 4;
-  else r.bm = 128, r.bn = 64, r.wm = 32, r.wn = 32, r.sa = 4, r.sb = 4;
+  set_tile(r, dma_tile(m, k, tiles));
   const uint64_t grid = (m + r.bm - 1) / r.bm * tiles(r.bn);
   if (grid > 0x7fffffu) return GemmRoute{};
   r.grid_x = (uint32_t)grid;
@@ -1629,7 +1713,10 @@ hipError_t launch_gemm_group(hipStream_t st, const GemmArgs& a, GemmGroup& g) {
            : r.ma == 160 ? launch_tall_group<32, 5, 5, 160>(st, a, g, tn)
                          : launch_tall_group<32, 4, 4, 256>(st, a, g, tn);
   }
-  if (r.bm == 256) return launch_dma_group<256, 192, 64, 96, 2, 3>(st, a, g, tn);
+  if (r.bm == 256 && r.bn == 256) return launch_dma_group<256, 256, 64, 128, 2, 3>(st, a, g, tn);
+  if (r.bm == 256 && r.bn == 192) return launch_dma_group<256, 192, 64, 96, 2, 3>(st, a, g, tn);
+  if (r.bm == 256) return launch_dma_group<256, 128, 64, 64, 2, 4>(st, a, g, tn);
+  if (r.bm == 64) return launch_dma_group<64, 128, 32, 32, 4, 4>(st, a, g, tn);
   if (r.bn == 192) return launch_dma_group<128, 192, 32, 96, 2, 4>(st, a, g, tn);
   if (r.bn == 128) return launch_dma_group<128, 128, 32, 64, 4, 4>(st, a, g, tn);
   return launch_dma_group<128, 64, 32, 32, 4, 4>(st, a, g, tn);

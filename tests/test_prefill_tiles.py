@@ -1,0 +1,90 @@
+"""gemm_dma's tiles: the strip numbering and the bounds of the 32-bit lane
+offsets on the CPU, and every tile with whole, ragged and several strips of M
+tiles on the GPU, against the oracle."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import oracle
+from test_indexing import route, xcd_slot
+
+STRIP, MAX_K, MAX_COLS = 4, 1 << 23, 1 << 26  # kStrip, kMaxK, kMaxCols (gemm.hip)
+
+
+@pytest.mark.parametrize("tm", [1, 2, 3, 4, 5, 7, 8, 9, 16, 33])
+@pytest.mark.parametrize("tn", [1, 2, 16, 31])
+@pytest.mark.parametrize("splits", [1, 2])
+def test_strip_numbering_visits_every_tile_once(tm, tn, splits):
+    T = tm * tn
+    L = xcd_slot(np.arange(T * splits), T * splits)
+    split, t = L // T, L % T
+    strip = STRIP * tn
+    s0, inside = t // strip * STRIP, t % strip
+    sm = np.minimum(STRIP, tm - s0)
+    mt, nt = s0 + inside % sm, inside // sm
+    assert mt.max() < tm and nt.max() < tn
+    assert len({*zip(split.tolist(), mt.tolist(), nt.tolist())}) == T * splits
+
+
+def test_lane_offsets_fit_32_bits():
+    """The routes that hold a lane's offset in 32 bits stop where it would not
+    fit, and the others take over."""
+    assert 255 * MAX_K + 127 < 1 << 32               # a tile's last row and chunk, in bytes
+    assert (4 * MAX_COLS + 31) * 4 < 1 << 32         # four rows and 31 columns of f32
+    for m in (1, 16, 40, 64, 100, 300, 5000):
+        for n, k, staged in ((1000, MAX_K, True), (1000, MAX_K + 128, False), (MAX_COLS, 128, True),
+                             (MAX_COLS + 4, 128, False)):
+            if m * n >= 1 << 32:
+                continue
+            fam = route(m, n, k, path=2)["family"]
+            assert staged or fam in ((11, 15) if m <= 64 else (14,)), (m, n, k, fam)
+            if m > 256 and staged:
+                assert fam == 13, (m, n, k, fam)
+
+
+TILES = [((128, 64), 1025, 1003), ((128, 128), 2049, 1003), ((128, 192), 1281, 3003), ((256, 128), 1025, 5503),
+         ((256, 192), 1025, 7253), ((64, 128), 1281, 1503), ((256, 256), 2049, 6003)]
+
+
+@pytest.mark.parametrize("tile,m,n", TILES)
+def test_tile_routes(tile, m, n):
+    r = route(m, n, 1280)
+    assert r["family"] == 13 and (r["bm"], r["bn"]) == tile
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile,m,n", TILES)
+@pytest.mark.parametrize("k", [1280])
+def test_every_tile(tile, m, n, k):
+    """Odd M and N (guarded edges beside whole tiles), K = 10 stages, every
+    output form, guard values past the output untouched."""
+    from inferrous_amd import CudaContext, DeviceBuffer, load
+    ctx = CudaContext(0)
+    mod, s = load(ctx), ctx.new_stream()
+    print(f"tile {tile} m={m} n={n} k={k}", flush=True)
+    rng = np.random.default_rng(m + n)
+    q = rng.integers(-127, 128, (m, k), dtype=np.int8)
+    w = rng.integers(-127, 128, (n, k), dtype=np.int8)
+    asc, ws = (rng.random(m) / 64).astype(np.float32), (rng.random(n) / 64).astype(np.float32)
+    res = oracle.bf16_rne(rng.standard_normal(m * n).astype(np.float32))
+    acc, of, ob = oracle.linear(q, asc, w, ws, k, threads=8)
+    comb = oracle.residual(res, of)
+    dev = lambda a: DeviceBuffer.from_host(s, np.ascontiguousarray(a))  # noqa: E731
+    dq, da, dw, dws, dres = dev(q), dev(asc), dev(w), dev(ws), dev(res)
+    guard = 512
+    for dtype, residual in ((np.int32, False), (np.float32, False), (np.uint16, False), (np.float32, True),
+                            (np.uint16, True)):
+        bufs = [dev(np.full(m * n + guard, 7, dtype)) for _ in range(1 + residual)]
+        out, *cb = [DeviceBuffer.view_of(b, 0, m * n) for b in bufs]
+        if residual:
+            mod.linear_residual(s, None, dq, da, dw, dws, k, dres, out, cb[0])
+        else:
+            mod.linear_mfma(s, None, dq, da, dw, dws, k, out)
+        want = [{np.int32: acc, np.float32: of, np.uint16: ob}[dtype]]
+        if residual:
+            want.append(comb if dtype == np.float32 else (comb.view(np.uint32) >> 16).astype(np.uint16))
+        for b, v in zip(bufs, want):
+            got = b.to_host_vec(s)
+            assert np.array_equal(got[:m * n].view(np.uint8), v.reshape(-1).view(np.uint8)), (dtype, residual)
+            assert (got[m * n:] == 7).all(), (dtype, residual)
