@@ -65,7 +65,7 @@ int w8a8_diag_gemm_timeline(void *stream, const int8_t *q, const float *asc,
  * arithmetic over exactly the grid the library launches.  Nothing runs on a
  * device; no device is needed.
  *   [0] family: 0 none (m or n is 0), 1 gemv_m1_one, 2 gemv_m1, 3 gemv_mt,
- *       11 gemm_skinny, 12 gemm_tall, 13 gemm_dma, 14 gemm_tiled, 15 gemm_narrow
+ *       11 gemm_skinny, 12 gemm_tall, 13 gemm_dma, 14 gemm_dma with four waves, 15 gemm_narrow
  *   [1] grid x  [2] grid y  [3] threads per workgroup
  *   [4] BM  [5] BN  [6] WM  [7] WN  [8] SA (gemm_narrow: ring stages)  [9] SB
  *   [10] MA (gemm_tall's M tile)

@@ -538,6 +538,8 @@ size_t w8a8_linear_workspace_bytes_path(size_t m, size_t n, uint32_t k, int path
   if (path == W8A8_PATH_AUTO && m <= kDot4AutoMaxM && auto_path(m, n, k, 0) == W8A8_PATH_DOT4)
     return 0;  // AUTO runs the dot4 GEMV there
   if (path != W8A8_PATH_AUTO && path != W8A8_PATH_MFMA) return 0;
+  if (path == W8A8_PATH_AUTO && m <= kU32Max && n <= kU32Max && gemm_unsplit_leads((uint32_t)m, (uint32_t)n, k))
+    return 0;  // faster without
   return w8a8_linear_workspace_bytes(m, n, k);
 }
 

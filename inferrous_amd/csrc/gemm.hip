@@ -18,19 +18,18 @@
 //     16 x i32 result of lane l holds rows 8*(v/4)+4*(l/32)+v%4, column l%32.
 //
 // Kernels:
-//  * gemm_dma (k % 128 == 0 and M > 64, or 8 <= M <= 64 when n gives >= 128
-//    tiles of 128 columns, wherever gemm_tall's plan does not apply): the
-//    prefill GEMM, built on
-//    v_mfma_i32_32x32x32_i8 (on gfx950 the 16x16x64 int8 form issues at half
-//    its rate), eight waves per workgroup (two per SIMD, so one wave's LDS
-//    reads overlap the other's MFMAs).  Operands move global -> LDS with
+//  * gemm_dma: the prefill GEMM, and every shape above 16 rows that no plan
+//    below takes; built on v_mfma_i32_32x32x32_i8 (on gfx950 the 16x16x64 int8
+//    form issues at half its rate), eight waves per workgroup (two per SIMD,
+//    so one wave's LDS reads overlap the other's MFMAs; four on the 64 x 64
+//    tile and for k % 128 != 0).  Operands move global -> LDS with
 //    global_load_lds_dwordx4 (no VGPR staging) in 128-byte K stages (whole
 //    cache lines) through two rings, activations and weights, the weights
-//    requested further ahead; one barrier per stage; the 16-byte chunks of
-//    each LDS row are XOR-swizzled so fragment reads spread over the banks.
-//    Workgroups are numbered XCD-aware (below).  Tile shape per problem is
-//    chosen by the host from the tile count.  With a caller workspace, some
-//    shapes run split-K (i32 slabs + splitk_epilogue).
+//    requested further ahead, the requests spread between the MFMAs; one
+//    barrier per stage; the 16-byte chunks of each LDS row are XOR-swizzled so
+//    fragment reads spread over the banks.  Workgroups are numbered XCD-aware
+//    (below).  Tile shape per problem by measured cost.  With a caller
+//    workspace, some shapes run split-K (i32 slabs + splitk_epilogue).
 //  * gemm_tall (M <= 256, k % 128 == 0, where its plan applies; M tiles of
 //    64, 160 or 256 rows): one M tile holds every activation row, so each
 //    weight tile streams from HBM once; the waves hold 32 x 32 output blocks
@@ -46,18 +45,12 @@
 //    loop has no workgroup barrier and no split-K slabs leave the CU.  The S
 //    partial 16 x 16 tiles are summed through LDS (exact) and stored by the
 //    fused epilogue.
-//  * gemm_skinny (small M on narrow n, HBM-bound, 16x16x64 MFMA): one
-//    workgroup owns 16 weight rows; its S waves split K and stream their
-//    weight fragments straight from HBM into MFMA B operands (no LDS round
-//    trip), activation fragments come from L1/L2.  Partial i32 tiles are
-//    summed through LDS -- exact.
-//  * gemm_tiled (M > 64 with k % 128 != 0): BM x BN output tile, 4 waves,
-//    128-byte K stages double-buffered in LDS (row pitch 144 B: a 16-lane
-//    ds_read_b128 column touches every bank once), global loads of stage
-//    k+1 in flight while stage k feeds the MFMAs.  Workgroups are numbered
-//    so that the M tiles sharing one weight panel run on the same XCD
-//    (workgroup id mod 8 picks the XCD), so the panel is fetched into that
-//    XCD's L2 once.
+//  * gemm_skinny (M <= 16 where gemm_narrow and gemm_tall do not run: k not in
+//    their stages, or a split-K plan without a workspace; HBM-bound, 16x16x64
+//    MFMA): one workgroup owns 16 weight rows; its S waves split K and stream
+//    their weight fragments straight from HBM into MFMA B operands (no LDS
+//    round trip), activation fragments come from L1/L2.  Partial i32 tiles
+//    are summed through LDS -- exact.
 #include <algorithm>
 #include <type_traits>
 
@@ -141,103 +134,6 @@ __global__ __launch_bounds__(64 * S) void gemm_skinny(GemmArgs a) {
     const uint32_t c = n0 + (l & 15);
     if (r < a.m && c < a.n) epilogue_store(a, r, c, sum);
   }
-}
-
-// ---------------------------------------------------------------- tiled
-template <int BM, int BN, int WM, int WN>
-__global__ __launch_bounds__(256) void gemm_tiled(GemmArgs a, uint32_t tiles_m, uint32_t tiles_n) {
-  constexpr int BK = 128;
-  constexpr int PITCH = BK + 16;
-  constexpr int WAVES_N = BN / WN;
-  static_assert((BM / WM) * (BN / WN) == 4, "four waves per workgroup");
-  constexpr int FM = WM / 16, FN = WN / 16;
-  constexpr int ACH = BM * (BK / 16) / 256, BCH = BN * (BK / 16) / 256;
-  static_assert(ACH >= 1 && BCH >= 1, "tile too small for 256 loaders");
-  __shared__ __attribute__((aligned(16))) int8_t As[2][BM * PITCH];
-  __shared__ __attribute__((aligned(16))) int8_t Bs[2][BN * PITCH];
-
-  // XCD-aware numbering: workgroups id, id+8, id+16, ... share an XCD; give
-  // each XCD a contiguous run of (n tile, m tile) pairs, m fastest.
-  const uint32_t T = tiles_m * tiles_n;
-  uint32_t L = blockIdx.x;
-  if (T % 8 == 0) L = (blockIdx.x % 8) * (T / 8) + blockIdx.x / 8;
-  const uint32_t mt = L % tiles_m, nt = L / tiles_m;
-  const uint32_t m0 = mt * BM, n0 = nt * BN;
-
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm0 = (wave / WAVES_N) * WM, wn0 = (wave % WAVES_N) * WN;
-  const uint32_t K = a.k, M = a.m, N = a.n;
-  const uint32_t KT = (K + BK - 1) / BK;
-
-  v4i ra[ACH], rb[BCH];
-  auto gload = [&](uint32_t kt) {
-#pragma unroll
-    for (int i = 0; i < ACH; ++i) {
-      const int id = tid + i * 256, row = id >> 3, kc = id & 7;
-      const uint32_t gm = m0 + row, kk = kt * BK + kc * 16;
-      ra[i] = (gm < M && kk < K) ? load16(a.q + (size_t)gm * K + kk) : v4i{0, 0, 0, 0};
-    }
-#pragma unroll
-    for (int i = 0; i < BCH; ++i) {
-      const int id = tid + i * 256, row = id >> 3, kc = id & 7;
-      const uint32_t gn = n0 + row, kk = kt * BK + kc * 16;
-      rb[i] = (gn < N && kk < K) ? load16(a.w + (size_t)gn * K + kk) : v4i{0, 0, 0, 0};
-    }
-  };
-  auto sstore = [&](int buf) {
-#pragma unroll
-    for (int i = 0; i < ACH; ++i) {
-      const int id = tid + i * 256, row = id >> 3, kc = id & 7;
-      *reinterpret_cast<v4i*>(&As[buf][row * PITCH + kc * 16]) = ra[i];
-    }
-#pragma unroll
-    for (int i = 0; i < BCH; ++i) {
-      const int id = tid + i * 256, row = id >> 3, kc = id & 7;
-      *reinterpret_cast<v4i*>(&Bs[buf][row * PITCH + kc * 16]) = rb[i];
-    }
-  };
-
-  v4i acc[FM][FN];
-#pragma unroll
-  for (int i = 0; i < FM; ++i)
-#pragma unroll
-    for (int j = 0; j < FN; ++j) acc[i][j] = v4i{0, 0, 0, 0};
-
-  gload(0);
-  sstore(0);
-  __syncthreads();
-  const int frow = lane & 15, fk = (lane >> 4) * 16;
-  for (uint32_t kt = 0; kt < KT; ++kt) {
-    const int buf = kt & 1;
-    if (kt + 1 < KT) gload(kt + 1);
-#pragma unroll
-    for (int ks = 0; ks < BK / 64; ++ks) {
-      v4i af[FM], bfr[FN];
-#pragma unroll
-      for (int i = 0; i < FM; ++i)
-        af[i] = *reinterpret_cast<const v4i*>(&As[buf][(wm0 + i * 16 + frow) * PITCH + ks * 64 + fk]);
-#pragma unroll
-      for (int j = 0; j < FN; ++j)
-        bfr[j] = *reinterpret_cast<const v4i*>(&Bs[buf][(wn0 + j * 16 + frow) * PITCH + ks * 64 + fk]);
-#pragma unroll
-      for (int i = 0; i < FM; ++i)
-#pragma unroll
-        for (int j = 0; j < FN; ++j) acc[i][j] = mfma16(af[i], bfr[j], acc[i][j]);
-    }
-    if (kt + 1 < KT) sstore(buf ^ 1);
-    __syncthreads();
-  }
-
-#pragma unroll
-  for (int i = 0; i < FM; ++i)
-#pragma unroll
-    for (int j = 0; j < FN; ++j)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const uint32_t r = m0 + wm0 + i * 16 + 4 * (lane >> 4) + v;
-        const uint32_t c = n0 + wn0 + j * 16 + (lane & 15);
-        if (r < M && c < N) epilogue_store(a, r, c, acc[i][j][v]);
-      }
 }
 
 // ---------------------------------------------------------------- dma
@@ -409,21 +305,22 @@ __global__ __launch_bounds__(64 * S) void gemm_narrow(GemmArgs a, GroupArg<GROUP
 // FULL: the whole grid of blocks lies inside the output, so nothing is clamped
 // or guarded.  Every address is then a wave-uniform corner (scalar registers)
 // plus one 32-bit lane offset, the same for all values: 4 (l / 32) rows and
-// l % 32 columns (the routes keep N below kMaxCols, so its bytes fit).
+// l % 32 columns (Off: 32 bits where the route keeps N at kMaxCols and below,
+// so that its bytes fit).
 constexpr uint32_t kMaxCols = 1u << 26;
 // Residuals of up to this many values per lane are loaded with the scales; a
 // larger wave tile's, which the registers beside its accumulators do not hold,
 // block by block, the next block's ahead of a block's stores.
 constexpr int kResidualHeld = 64;
 
-template <int EP, bool FULL, int FM, int FN>
+template <int EP, bool FULL, class Off, int FM, int FN>
 __device__ __forceinline__ void store_blocks_as(const GemmArgs& a, const v16i (&acc)[FM][FN], uint32_t row0,
                                                 uint32_t col0, int lane) {
   constexpr bool RES = EP == EP_F32_RES || EP == EP_BF16_RES;
   constexpr bool F32 = EP == EP_F32 || EP == EP_F32_RES;
   constexpr int ESZ = raw_i32(EP) || F32 ? 4 : 2;
   const uint32_t half = (uint32_t)lane >> 5, cl = (uint32_t)lane & 31;
-  const uint32_t lane_off = 4 * half * a.n + cl;
+  const Off lane_off = (Off)(4 * half) * a.n + cl;
   auto corner_row = [&](int i, int v) -> uint32_t { return row0 + 32 * i + (v >> 2) * 8 + (v & 3); };
   // byte address of value v of block (i, j) in an array of E-byte elements
   auto at = [&](const void* p, int i, int v, int j, auto esz) {
@@ -511,13 +408,13 @@ __device__ __forceinline__ void store_blocks_as(const GemmArgs& a, const v16i (&
   }
 }
 
-template <int EP, int FM, int FN>
+template <int EP, class Off = uint32_t, int FM, int FN>
 __device__ __forceinline__ void store_blocks(const GemmArgs& a, const v16i (&acc)[FM][FN], uint32_t row0,
                                              uint32_t col0, int lane) {
-  if (row0 + 32 * FM <= a.m && col0 + 32 * FN <= a.n)
-    store_blocks_as<EP, true, FM, FN>(a, acc, row0, col0, lane);
+  if ((size_t)row0 + 32 * FM <= a.m && (size_t)col0 + 32 * FN <= a.n)
+    store_blocks_as<EP, true, Off, FM, FN>(a, acc, row0, col0, lane);
   else
-    store_blocks_as<EP, false, FM, FN>(a, acc, row0, col0, lane);
+    store_blocks_as<EP, false, Off, FM, FN>(a, acc, row0, col0, lane);
 }
 
 // Prefill GEMM.  Workgroup = 8 waves (two per SIMD: while one wave waits on
@@ -551,15 +448,25 @@ __device__ __forceinline__ void store_blocks(const GemmArgs& a, const v16i (&acc
 constexpr uint32_t kStrip = 4;
 constexpr uint32_t kMaxK = 1u << 23;  // 256 rows of K bytes stay within a 32-bit offset
 
-template <int BM, int BN, int WM, int WN, int SA, int SB, int EP, bool GROUP = false>
-__global__ __launch_bounds__(512) void gemm_dma(GemmArgs a, uint32_t tiles_m, uint32_t tiles_n,
-                                                uint32_t splits, GroupArg<GROUP> group) {
+// TAIL (K % 128 != 0, any N): the last stage is partial.  A lane whose 16-byte
+// chunk lies past K reads zeros for the activation row, and its weight row's
+// first chunk (any bytes: their products are zero), so nothing outside the
+// operands is read and the sums are exact.  These launches take four waves
+// per workgroup (NW), as does the 64 x 64 tile; two workgroups share a CU where the
+// rings take 80 KiB.
+__device__ const v4i kZeroChunk = {0, 0, 0, 0};
+
+constexpr int waves_per_simd(int nw, int lds_bytes) { return nw == 8 || lds_bytes <= 80 * 1024 ? 2 : 1; }
+
+template <int BM, int BN, int WM, int WN, int SA, int SB, int EP, bool GROUP = false, int NW = 8, bool TAIL = false>
+__global__ __launch_bounds__(64 * NW, (waves_per_simd(NW, (SA * BM + SB * BN) * 128))) void gemm_dma(
+    GemmArgs a, uint32_t tiles_m, uint32_t tiles_n, uint32_t splits, GroupArg<GROUP> group) {
   constexpr int WAVES_N = BN / WN;
-  static_assert((BM / WM) * (BN / WN) == 8, "eight waves per workgroup");
-  static_assert(WM % 32 == 0 && WN % 32 == 0 && BM % 64 == 0 && BN % 64 == 0, "tile shape");
+  static_assert((BM / WM) * (BN / WN) == NW, "one wave tile per wave");
+  static_assert(WM % 32 == 0 && WN % 32 == 0 && BM % (8 * NW) == 0 && BN % (8 * NW) == 0, "tile shape");
   static_assert(SA >= 2 && SB >= SA && SB >= 3 && SB <= 8, "ring depths");
   constexpr int FM = WM / 32, FN = WN / 32;
-  constexpr int LA = BM / 64, LB = BN / 64;  // DMA loads (8 rows x 128 B) per wave per stage
+  constexpr int LA = BM / 8 / NW, LB = BN / 8 / NW;  // DMA loads (8 rows x 128 B) per wave per stage
   constexpr int L = LA + LB;
   constexpr int ASL = BM * 128, BSL = BN * 128;
   static_assert(SA * ASL + SB * BSL <= 160 * 1024, "LDS");
@@ -581,7 +488,7 @@ __global__ __launch_bounds__(512) void gemm_dma(GemmArgs a, uint32_t tiles_m, ui
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int wm0 = (wave / WAVES_N) * WM, wn0 = (wave % WAVES_N) * WN;
-  const uint32_t K = a.k, KT = K / 128 / splits;
+  const uint32_t K = a.k, KT = TAIL ? K / 128 + 1 : K / 128 / splits;
   const size_t kbase = (size_t)split * KT * 128;
   if (raw_i32(EP)) a.out = reinterpret_cast<int32_t*>(a.out) + (size_t)split * a.m * a.n;
 
@@ -591,26 +498,39 @@ __global__ __launch_bounds__(512) void gemm_dma(GemmArgs a, uint32_t tiles_m, ui
   // (l % 8) ^ key(row).
   // An address is the tile's first row (scalar registers) plus a 32-bit lane
   // offset (the routes keep K at kMaxK and below).
+  using Off = std::conditional_t<TAIL, size_t, uint32_t>;
   const int8_t* const srcA = a.q + (size_t)m0 * K + kbase;
   const int8_t* const srcB = a.w + (size_t)n0 * K + kbase;
-  uint32_t offA[LA], offB[LB];
+  auto lds_row = [&](int g) { return (uint32_t)(8 * g + (lane >> 3)); };  // row group g of 8 rows
+  auto chunk = [&](int g) { return (uint32_t)((lane & 7) ^ ((lds_row(g) >> 1) & 7)) * 16; };
+  Off offA[LA], offB[LB];
 #pragma unroll
   for (int j = 0; j < LA; ++j) {
-    const uint32_t row = 8 * (wave * LA + j) + (lane >> 3);
-    offA[j] = (m0 + row < a.m ? row : 0) * K + ((lane & 7) ^ ((row >> 1) & 7)) * 16;
+    const uint32_t row = lds_row(wave * LA + j);
+    offA[j] = (Off)(m0 + row < a.m ? row : 0) * K + (TAIL ? 0 : chunk(wave * LA + j));
   }
 #pragma unroll
   for (int j = 0; j < LB; ++j) {
-    const uint32_t row = 8 * (wave * LB + j) + (lane >> 3);
-    offB[j] = (n0 + row < a.n ? row : 0) * K + ((lane & 7) ^ ((row >> 1) & 7)) * 16;
+    const uint32_t row = lds_row(wave * LB + j);
+    offB[j] = (Off)(n0 + row < a.n ? row : 0) * K + (TAIL ? 0 : chunk(wave * LB + j));
   }
   auto loadA = [&](uint32_t kt, int j) {
-    __builtin_amdgcn_global_load_lds((const void*)(srcA + (size_t)kt * 128 + offA[j]),
+    const int8_t* p = srcA + (size_t)kt * 128 + offA[j];
+    if constexpr (TAIL) {
+      const uint32_t kk = kt * 128 + chunk(wave * LA + j);
+      p = kk < K ? srcA + offA[j] + kk : reinterpret_cast<const int8_t*>(&kZeroChunk);
+    }
+    __builtin_amdgcn_global_load_lds((const void*)p,
                                      W8A8_LDS_PTR(ldsA + (kt % SA) * ASL + (wave * LA + j) * 1024 + lane * 16),
                                      16, 0, 0);
   };
   auto loadB = [&](uint32_t kt, int j) {
-    __builtin_amdgcn_global_load_lds((const void*)(srcB + (size_t)kt * 128 + offB[j]),
+    const int8_t* p = srcB + (size_t)kt * 128 + offB[j];
+    if constexpr (TAIL) {
+      const uint32_t kk = kt * 128 + chunk(wave * LB + j);
+      p = srcB + offB[j] + (kk < K ? kk : 0);
+    }
+    __builtin_amdgcn_global_load_lds((const void*)p,
                                      W8A8_LDS_PTR(ldsB + (kt % SB) * BSL + (wave * LB + j) * 1024 + lane * 16),
                                      16, 0, 0);
   };
@@ -712,18 +632,27 @@ __global__ __launch_bounds__(512) void gemm_dma(GemmArgs a, uint32_t tiles_m, ui
   mm(a0, b0);
   mm(a1, b1);
 
-  store_blocks<EP, FM, FN>(a, acc, m0 + wm0, n0 + wn0, lane);
+  store_blocks<EP, Off>(a, acc, m0 + wm0, n0 + wn0, lane);
 }
 
-template <int BM, int BN, int WM, int WN, int SA, int SB>
+// A 128 x 128 wave tile's accumulators leave no registers for residuals.
+template <int WM, int WN>
+constexpr bool kResidualTile = WM * WN < 128 * 128;
+
+template <int BM, int BN, int WM, int WN, int SA, int SB, int NW = 8, bool TAIL = false>
 static hipError_t launch_dma(hipStream_t st, const GemmArgs& a) {
   const uint32_t tm = (a.m + BM - 1) / BM, tn = (a.n + BN - 1) / BN;
-  const dim3 grid(tm * tn), block(512);
-  auto k = a.out_dtype == W8A8_OUT_I32 ? gemm_dma<BM, BN, WM, WN, SA, SB, EP_I32>
-           : a.out_dtype == W8A8_OUT_F32
-               ? (a.residual ? gemm_dma<BM, BN, WM, WN, SA, SB, EP_F32_RES> : gemm_dma<BM, BN, WM, WN, SA, SB, EP_F32>)
-               : (a.residual ? gemm_dma<BM, BN, WM, WN, SA, SB, EP_BF16_RES> : gemm_dma<BM, BN, WM, WN, SA, SB, EP_BF16>);
-  hipLaunchKernelGGL(k, grid, block, 0, st, a, tm, tn, 1u, NoGroup{});
+  auto k = a.out_dtype == W8A8_OUT_I32   ? gemm_dma<BM, BN, WM, WN, SA, SB, EP_I32, false, NW, TAIL>
+           : a.out_dtype == W8A8_OUT_F32 ? gemm_dma<BM, BN, WM, WN, SA, SB, EP_F32, false, NW, TAIL>
+                                         : gemm_dma<BM, BN, WM, WN, SA, SB, EP_BF16, false, NW, TAIL>;
+  if (a.residual) {
+    if constexpr (kResidualTile<WM, WN>)
+      k = a.out_dtype == W8A8_OUT_F32 ? gemm_dma<BM, BN, WM, WN, SA, SB, EP_F32_RES, false, NW, TAIL>
+                                      : gemm_dma<BM, BN, WM, WN, SA, SB, EP_BF16_RES, false, NW, TAIL>;
+    else
+      return hipErrorInvalidValue;
+  }
+  hipLaunchKernelGGL(k, dim3(tm * tn), dim3(64 * NW), 0, st, a, tm, tn, 1u, NoGroup{});
   return hipGetLastError();
 }
 
@@ -966,7 +895,7 @@ __global__ __launch_bounds__(512) void gemm_tall(GemmArgs a, uint32_t tiles_n, u
                [&](const Frag& f) { acc = mfma32(f.a, f.b, acc); });
       stamp_stream_end();
       const v16i blocks[1][1] = {{acc}};
-      store_blocks<EP, 1, 1>(a, blocks, 32 * mb, n0 + 32 * nbk, lane);
+      store_blocks<EP>(a, blocks, 32 * mb, n0 + 32 * nbk, lane);
     } else {
       move_only();
       stamp_stream_end();
@@ -991,7 +920,7 @@ __global__ __launch_bounds__(512) void gemm_tall(GemmArgs a, uint32_t tiles_n, u
                });
       stamp_stream_end();
       const v16i (&blocks)[1][FN] = *reinterpret_cast<const v16i(*)[1][FN]>(&acc);
-      store_blocks<EP, 1, FN>(a, blocks, 32 * wave, n0, lane);
+      store_blocks<EP>(a, blocks, 32 * wave, n0, lane);
     } else {
       move_only();
       stamp_stream_end();
@@ -1156,46 +1085,76 @@ __global__ __launch_bounds__(256) void splitk_epilogue8(GemmArgs a, const int32_
   }
 }
 
-// gemm_dma's tiles, and the time one takes with every CU busy: fixed + stages
-// x 128-byte K stages (ns, fitted to the launches below).  A launch runs its
-// tiles in rounds of one per CU, so the route is the tile with the least
-// rounds x time: large tiles move the fewest operand bytes per product but
-// leave CUs idle in their last round, small ones the other way about.
-// Measured on MI355X with random operands, us per launch (256 x 256 / 256 x 192
-// / 256 x 128 / 128 x 192 / 128 x 128 / 128 x 64): 24576 x 4096 f32 at M = 4096
-// 393 / 417 / 439 / 488 / 537 / -; 6144 x 4096 BF16 at M = 4096 112 / 97.7 / 103 /
-// 113 / 126 / -, at M = 1024 - / - / 30.3 / 28.1 / 38.2 / 39.4, at M = 512 - / - /
-// - / 23.5 / 19.4 / 25.5; 4096 x 4096 f32 with the residual at M = 4096 87 / - /
-// 91 / 103 / 112 / -, at M = 1024 - / - / 36 / 29.1 / 26.9 / 29.8, at M = 512 - /
-// - / 33.7 / 25.7 / 21.0 / 16.7; 4096 x 12288 likewise at M = 4096 196 / - / 211 /
-// - / 257 / -, at M = 512 - / - / 84 / 72 / 58 / 44.7.
+// gemm_dma's tiles and what one costs (ns, fitted to the launches below): fixed +
+// K stages x stage with one workgroup on every CU, x pair with two (the tiles
+// whose rings take 80 KiB).  A launch runs its tiles in rounds, so the route is
+// the tile with the least sum over its rounds: large tiles move the fewest
+// operand bytes per product but leave CUs idle in their last round, small
+// ones the other way about.  A round that leaves CUs idle runs up to a
+// quarter faster (L2 and power are shared).
+//
+// kDmaTiles, K % 128 == 0: eight waves, and four on 64 x 64.  Measured on MI355X with random operands, us per
+// launch (256 x 256 / 256 x 192 / 256 x 128 / 128 x 192 / 128 x 128 / 128 x 64):
+// 24576 x 4096 f32 at M = 4096 393 / 417 / 439 / 488 / 537 / -; 6144 x 4096 BF16
+// at M = 4096 112 / 97.7 / 103 / 113 / 126 / -, at M = 1024 - / - / 30.3 / 28.1 /
+// 38.2 / 39.4, at M = 512 - / - / - / 23.5 / 19.4 / 25.5; 4096 x 4096 f32 with the
+// residual at M = 4096 87 / - / 91 / 103 / 112 / -, at M = 1024 - / - / 36 / 29.1
+// / 26.9 / 29.8, at M = 512 - / - / 33.7 / 25.7 / 21.0 / 16.7; 4096 x 12288
+// likewise at M = 4096 196 / - / 211 / - / 257 / -, at M = 512 - / - / 84 / 72 / 58 /
+// 44.7.
+//
+// 6144 x 4096 f32 at M = 129: 64 x 128 12.5, 64 x 64 16.5 (gemm_tall's split K with
+// its slab epilogue 16.4); 4096 x 4096 with the residual at M = 129 64 x 64 11.5
+// (split 13.6), at M = 256 12.7 (17.2).  Four-wave tiles of 128 x 64 and 128 x 32
+// were within 1 us of those on these shapes, and slower where they mattered.
+//
+// kTailTiles, K % 128 != 0: four waves.  gemm_tiled, the register-staged kernel
+// these replaced -> the tile the route takes: 4096 x 8000 x 5008 316 -> 168, 2000
+// x 8000 x 5008 145 -> 89, 1024 x 4096 x 4112 52 -> 26, 512 x 6000 x 4112 52 -> 30,
+// 300 x 3000 x 2000 28 -> 9.2, 77 x 5003 x 2000 27.7 -> 8.7, and gemm_skinny: 64 x
+// 4096 x 4112 16.0 -> 11.9, 30 x 12000 x 4112 28.6 -> 15.8 (M x N x K).
 struct DmaTile {
   int bm, bn, wm, wn, sa, sb;
-  uint32_t fixed, stage;
+  uint32_t fixed, stage, pair;  // pair 0: one workgroup per CU
 };
 static const DmaTile kDmaTiles[] = {
-    {256, 256, 64, 128, 2, 3, 11000, 1700}, {256, 192, 64, 96, 2, 3, 10000, 1270},
-    {256, 128, 64, 64, 2, 4, 7000, 940},    {128, 192, 32, 96, 2, 4, 5000, 740},
-    {128, 128, 32, 64, 4, 4, 3000, 590},    {128, 64, 32, 32, 4, 4, 2500, 440},
-    {64, 128, 32, 32, 4, 4, 2500, 440},
+    {256, 256, 64, 128, 2, 3, 11000, 1700, 0}, {256, 192, 64, 96, 2, 3, 10000, 1270, 0},
+    {256, 128, 64, 64, 2, 4, 7000, 940, 0},    {128, 192, 32, 96, 2, 4, 5000, 740, 0},
+    {128, 128, 32, 64, 4, 4, 3000, 590, 0},    {128, 64, 32, 32, 4, 4, 2500, 440, 0},
+    {64, 128, 32, 32, 4, 4, 2500, 440, 0},     {64, 64, 32, 32, 4, 4, 3000, 280, 460},
+};
+static const DmaTile kTailTiles[] = {
+    {256, 256, 128, 128, 2, 3, 11000, 1830, 0}, {256, 128, 128, 64, 2, 4, 7000, 1100, 0},
+    {128, 128, 64, 64, 2, 3, 5000, 620, 1340},  {128, 64, 64, 32, 3, 4, 4000, 420, 890},
+    {64, 64, 32, 32, 4, 4, 3000, 280, 460},
 };
 constexpr uint64_t kCus = 256;
 
-// The cheapest tile for m rows and k, tiles_n(bn) column tiles.
-template <typename TilesN>
-static const DmaTile& dma_tile(uint32_t m, uint32_t k, TilesN tiles_n) {
+static uint64_t launch_ns(const DmaTile& t, uint64_t tiles, uint64_t stages) {
+  const uint64_t at_once = t.pair ? 2 * kCus : kCus, rest = tiles % at_once;
+  const uint64_t full = t.fixed + stages * (t.pair ? t.pair : t.stage);
+  const uint64_t last = rest > kCus ? full : rest ? t.fixed + stages * t.stage * (3 * kCus + rest) / (4 * kCus) : 0;
+  return tiles / at_once * full + last;
+}
+
+// The cheapest of the tiles for m rows and k, tiles_n(bn) column tiles.
+template <size_t N, typename TilesN>
+static const DmaTile& cheapest(const DmaTile (&tiles)[N], uint32_t m, uint32_t k, bool residual, TilesN tiles_n) {
   const DmaTile* best = nullptr;
   uint64_t least = ~0ull;
-  for (const DmaTile& t : kDmaTiles) {
-    const uint64_t tiles = (uint64_t)((m + t.bm - 1) / t.bm) * tiles_n(t.bn);
-    const uint64_t c = (tiles + kCus - 1) / kCus * (t.fixed + (uint64_t)(k / 128) * t.stage);
-    if (c < least) least = c, best = &t;
+  for (const DmaTile& t : tiles) {
+    if (residual && t.wm * t.wn >= 128 * 128) continue;  // !kResidualTile
+    const uint64_t c = launch_ns(t, ((uint64_t)m + t.bm - 1) / t.bm * tiles_n(t.bn), ((uint64_t)k + 127) / 128);
+    if (c < least) best = &t, least = c;
   }
   return *best;
 }
 
+// The route's tile, family and block: the four-wave tiles are kRouteTiled.
 static void set_tile(GemmRoute& r, const DmaTile& t) {
   r.bm = t.bm, r.bn = t.bn, r.wm = t.wm, r.wn = t.wn, r.sa = t.sa, r.sb = t.sb;
+  r.block = 64 * (t.bm / t.wm) * (t.bn / t.wn);
+  r.family = r.block == 256 ? kRouteTiled : kRouteDma;
 }
 
 // Whether gemm_dma and gemm_tall take the shape: K in whole 128-byte stages, and
@@ -1286,6 +1245,24 @@ static bool tall_plan(uint32_t m, uint32_t n, uint32_t k, int& bn, uint32_t& spl
   if (splits == 1) return false;
   bn = t96 * splits >= 224 ? 96 : 64;
   return true;
+}
+
+// Whether one unsplit launch (64 x 64 or 64 x 128 tiles, gemm_dma) runs a shape of
+// gemm_tall's split plan faster than the split GEMM and its slab epilogue: above
+// 64 rows, up to a K that grows with the slabs (M N values).  Measured on
+// MI355X with residual, split / unsplit us, 4096 columns at K = 2048 / 4096 /
+// 5120 / 6144 / 8192: M = 65 9.3 / 10.9 / 12.0 / 12.7 / 14.3 against 7.7 / 11.5 /
+// 13.8 / 15.8 / 20.2, M = 129 11.6 / 13.3 / 14.7 / 15.3 / 17.5 against 8.1 / 11.7 /
+// 14.3 / 16.1 / 20.4, M = 200 13.6 / 15.3 / 17.4 / 18.1 / 20.2 against 8.2 / 11.9 /
+// 14.6 / 16.4 / 20.8, M = 256 14.2 / 16.7 / 19.0 / 19.5 / 22.4 against 8.5 / 12.6 /
+// 16.3 / 17.5 / 22.2; 6144 columns, M = 100 12.3 / 14.2 / 16.5 / 16.7 / 19.0 against
+// 8.1 / 12.7 / 16.0 / 17.4 / 21.6; 8192 columns, M = 129 19.8 / 25.2 / 28.3 / 30.4 /
+// 35.2 against 9.9 / 16.2 / 20.6 / 22.2 / 26.7.
+bool gemm_unsplit_leads(uint32_t m, uint32_t n, uint32_t k) {
+  int bn, ma;
+  uint32_t splits;
+  if (m <= 64 || !tall_plan(m, n, k, bn, splits, ma) || splits == 1) return false;
+  return k <= std::min<uint64_t>(std::max<uint64_t>((uint64_t)m * n / 104, 3584), 8192);
 }
 
 size_t gemm_workspace_bytes(uint32_t m, uint32_t n, uint32_t k) {
@@ -1490,35 +1467,29 @@ GemmRoute gemm_route(const GemmArgs& a) {
       return r;
     }
   }
-  const uint32_t nb16 = (a.n + 15) / 16;
-  if (a.m <= 64 && !wide) {
+  if (a.m <= 16 && !wide) {
     r.family = kRouteSkinny;
-    r.mt = a.m <= 16 ? 1 : a.m <= 32 ? 2 : 4;
+    r.mt = 1;
     r.s = 4;
-    r.u = a.m <= 32 ? 4 : 2;
-    r.grid_x = nb16;
+    r.u = 4;
+    r.grid_x = (a.n + 15) / 16;
     r.block = 64 * r.s;
     return r;
   }
-  if (staged_shape(a.n, a.k)) {
-    r.family = kRouteDma;
-    uint32_t splits;
-    if (a.partials && split_plan(a.m, a.n, a.k, splits) &&
-        a.partial_bytes >= (size_t)splits * a.m * a.n * sizeof(int32_t)) {
-      set_tile(r, kDmaTiles[4]);
-      r.splits = splits;
-      r.epi_cols = wide_epilogue(a) ? 8 : 4;
-    } else {
-      set_tile(r, a.m <= 64 ? kDmaTiles[6]
-                            : dma_tile(a.m, a.k, [&](uint32_t bn) { return (uint64_t)(a.n + bn - 1) / bn; }));
-    }
-    r.grid_x = (a.m + r.bm - 1) / r.bm * ((a.n + r.bn - 1) / r.bn) * r.splits;
-    return r;
+  auto tiles_n = [&](uint32_t bn) { return ((uint64_t)a.n + bn - 1) / bn; };
+  const bool residual = a.residual != nullptr;
+  uint32_t splits;
+  if (!staged_shape(a.n, a.k)) {
+    set_tile(r, cheapest(kTailTiles, a.m, a.k, residual, tiles_n));
+  } else if (a.partials && split_plan(a.m, a.n, a.k, splits) &&
+             a.partial_bytes >= (size_t)splits * a.m * a.n * sizeof(int32_t)) {
+    set_tile(r, kDmaTiles[4]);
+    r.splits = splits;
+    r.epi_cols = wide_epilogue(a) ? 8 : 4;
+  } else {
+    set_tile(r, cheapest(kDmaTiles, a.m, a.k, residual, tiles_n));
   }
-  r.family = kRouteTiled;
-  r.bm = 128, r.bn = 128, r.wm = 64, r.wn = 64;
-  r.grid_x = (a.m + r.bm - 1) / r.bm * ((a.n + r.bn - 1) / r.bn);
-  r.block = 256;
+  r.grid_x = (a.m + r.bm - 1) / r.bm * ((a.n + r.bn - 1) / r.bn) * r.splits;
   return r;
 }
 
@@ -1568,6 +1539,14 @@ static hipError_t launch_narrow(hipStream_t st, const GemmArgs& a, const GemmRou
   return hipErrorInvalidValue;
 }
 
+static hipError_t launch_tail(hipStream_t st, const GemmArgs& a, const GemmRoute& r) {
+  if (r.bm == 256 && r.bn == 256) return launch_dma<256, 256, 128, 128, 2, 3, 4, true>(st, a);
+  if (r.bm == 256) return launch_dma<256, 128, 128, 64, 2, 4, 4, true>(st, a);
+  if (r.bm == 128 && r.bn == 128) return launch_dma<128, 128, 64, 64, 2, 3, 4, true>(st, a);
+  if (r.bm == 128) return launch_dma<128, 64, 64, 32, 3, 4, 4, true>(st, a);
+  return launch_dma<64, 64, 32, 32, 4, 4, 4, true>(st, a);
+}
+
 hipError_t launch_gemm(hipStream_t st, const GemmArgs& a) {
   const GemmRoute r = gemm_route(a);
   auto is = [&](int bm, int bn, int wm, int wn, int sa, int sb) {
@@ -1587,9 +1566,7 @@ hipError_t launch_gemm(hipStream_t st, const GemmArgs& a) {
     case kRouteNarrow:
       return launch_narrow(st, a, r);
     case kRouteSkinny:
-      if (r.mt == 1) hipLaunchKernelGGL((gemm_skinny<1, 4, 4>), dim3(r.grid_x, 1), dim3(r.block), 0, st, a);
-      else if (r.mt == 2) hipLaunchKernelGGL((gemm_skinny<2, 4, 4>), dim3(r.grid_x, 1), dim3(r.block), 0, st, a);
-      else hipLaunchKernelGGL((gemm_skinny<4, 4, 2>), dim3(r.grid_x, 1), dim3(r.block), 0, st, a);
+      hipLaunchKernelGGL((gemm_skinny<1, 4, 4>), dim3(r.grid_x, 1), dim3(r.block), 0, st, a);
       return hipGetLastError();
     case kRouteDma:
       if (r.splits > 1) return launch_split<128, 128, 32, 64, 4, 4>(st, a, r.splits);
@@ -1600,11 +1577,8 @@ hipError_t launch_gemm(hipStream_t st, const GemmArgs& a) {
       if (is(128, 128, 32, 64, 4, 4)) return launch_dma<128, 128, 32, 64, 4, 4>(st, a);
       if (is(128, 64, 32, 32, 4, 4)) return launch_dma<128, 64, 32, 32, 4, 4>(st, a);
       return launch_dma<64, 128, 32, 32, 4, 4>(st, a);
-    case kRouteTiled: {
-      const uint32_t tm = (a.m + 127) / 128, tn = (a.n + 127) / 128;
-      hipLaunchKernelGGL((gemm_tiled<128, 128, 64, 64>), dim3(tm * tn), dim3(256), 0, st, a, tm, tn);
-      return hipGetLastError();
-    }
+    case kRouteTiled:
+      return staged_shape(a.n, a.k) ? launch_dma<64, 64, 32, 32, 4, 4, 4>(st, a) : launch_tail(st, a, r);
   }
   return hipErrorInvalidValue;
 }
@@ -1625,13 +1599,13 @@ static hipError_t launch_tall_group(hipStream_t st, const GemmArgs& a, const Gem
   return hipGetLastError();
 }
 
-template <int BM, int BN, int WM, int WN, int SA, int SB>
+template <int BM, int BN, int WM, int WN, int SA, int SB, int NW = 8>
 static hipError_t launch_dma_group(hipStream_t st, const GemmArgs& a, const GemmGroup& g, uint32_t tn) {
   const uint32_t tm = (a.m + BM - 1) / BM;
-  auto k = a.out_dtype == W8A8_OUT_I32   ? gemm_dma<BM, BN, WM, WN, SA, SB, EP_I32, true>
-           : a.out_dtype == W8A8_OUT_F32 ? gemm_dma<BM, BN, WM, WN, SA, SB, EP_F32, true>
-                                         : gemm_dma<BM, BN, WM, WN, SA, SB, EP_BF16, true>;
-  hipLaunchKernelGGL(k, dim3(tm * tn), dim3(512), 0, st, a, tm, tn, 1u, g);
+  auto k = a.out_dtype == W8A8_OUT_I32   ? gemm_dma<BM, BN, WM, WN, SA, SB, EP_I32, true, NW>
+           : a.out_dtype == W8A8_OUT_F32 ? gemm_dma<BM, BN, WM, WN, SA, SB, EP_F32, true, NW>
+                                         : gemm_dma<BM, BN, WM, WN, SA, SB, EP_BF16, true, NW>;
+  hipLaunchKernelGGL(k, dim3(tm * tn), dim3(64 * NW), 0, st, a, tm, tn, 1u, g);
   return hipGetLastError();
 }
 
@@ -1668,17 +1642,15 @@ GemmRoute gemm_group_route(uint32_t m, uint32_t k, const uint32_t* n, int count)
     r.grid_x = (uint32_t)tiles(16);
     return r;
   }
-  if (m <= 256) {
+  if (m <= 256 && tiles(96) >= 224) {
     r.family = kRouteTall;
     r.ma = m <= 64 ? 64 : m <= 160 ? 160 : 256;
-    r.bn = tiles(96) >= 224 ? 96 : 32;
-    if (r.bn == 96) r.sa = r.ma == 256 ? 2 : 4, r.sb = 4;
-    else r.sa = r.sb = r.ma == 64 ? 8 : r.ma == 160 ? 5 : 4;
+    r.bn = 96;
+    r.sa = r.ma == 256 ? 2 : 4, r.sb = 4;
     r.grid_x = (uint32_t)tiles(r.bn);
     return r;
   }
-  r.family = kRouteDma;
-  set_tile(r, dma_tile(m, k, tiles));
+  set_tile(r, cheapest(kDmaTiles, m, k, false, tiles));
   const uint64_t grid = (m + r.bm - 1) / r.bm * tiles(r.bn);
   if (grid > 0x7fffffu) return GemmRoute{};
   r.grid_x = (uint32_t)grid;
@@ -1705,14 +1677,11 @@ hipError_t launch_gemm_group(hipStream_t st, const GemmArgs& a, GemmGroup& g) {
     return r.u == 1 ? launch_narrow_group<1, 1, 8, 4>(st, a, g, tn) : launch_narrow_group<1, 2, 8, 4>(st, a, g, tn);
   }
   if (r.family == kRouteTall) {
-    if (r.bn == 96)
-      return r.ma == 64    ? launch_tall_group<96, 4, 4, 64>(st, a, g, tn)
-             : r.ma == 160 ? launch_tall_group<96, 4, 4, 160>(st, a, g, tn)
-                           : launch_tall_group<96, 2, 4, 256>(st, a, g, tn);
-    return r.ma == 64    ? launch_tall_group<32, 8, 8, 64>(st, a, g, tn)
-           : r.ma == 160 ? launch_tall_group<32, 5, 5, 160>(st, a, g, tn)
-                         : launch_tall_group<32, 4, 4, 256>(st, a, g, tn);
+    return r.ma == 64    ? launch_tall_group<96, 4, 4, 64>(st, a, g, tn)
+           : r.ma == 160 ? launch_tall_group<96, 4, 4, 160>(st, a, g, tn)
+                         : launch_tall_group<96, 2, 4, 256>(st, a, g, tn);
   }
+  if (r.family == kRouteTiled) return launch_dma_group<64, 64, 32, 32, 4, 4, 4>(st, a, g, tn);
   if (r.bm == 256 && r.bn == 256) return launch_dma_group<256, 256, 64, 128, 2, 3>(st, a, g, tn);
   if (r.bm == 256 && r.bn == 192) return launch_dma_group<256, 192, 64, 96, 2, 3>(st, a, g, tn);
   if (r.bm == 256) return launch_dma_group<256, 128, 64, 64, 2, 4>(st, a, g, tn);

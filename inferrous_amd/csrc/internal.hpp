@@ -81,6 +81,8 @@ struct GemmGroup {
 
 // Bytes of split-K workspace launch_gemm would use for this shape (0: none).
 size_t gemm_workspace_bytes(uint32_t m, uint32_t n, uint32_t k);
+// The split plan exists, but one unsplit launch without it is faster.
+bool gemm_unsplit_leads(uint32_t m, uint32_t n, uint32_t k);
 
 // The launch a GEMM call makes, decided on the host: the kernel family, its
 // compile-time shape and its grid.  launch_gemm runs exactly this route; the
@@ -91,7 +93,7 @@ enum { kRouteNone = 0, kRouteGemvM1One = 1, kRouteGemvM1 = 2, kRouteGemvMt = 3, 
 struct GemmRoute {
   int family;                       // kRouteSkinny, kRouteTall, kRouteDma, kRouteTiled, kRouteNarrow
                                     // (kRouteNone: m or n is 0)
-  int bm, bn, wm, wn, sa, sb, ma;   // dma / tiled tile; tall: bn, sa, sb, ma; narrow: sa = ring stages
+  int bm, bn, wm, wn, sa, sb, ma;   // gemm_dma tile (dma: eight waves, tiled: four); tall: bn, sa, sb, ma; narrow: sa = ring stages
   int mt, s, u;                     // skinny: 16-row tiles, waves, unroll; narrow: 16-row tiles, waves,
                                     // live activation DMA loads per stage
   uint32_t splits;                  // split-K slabs (1: none)

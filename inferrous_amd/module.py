@@ -183,7 +183,9 @@ class LoadedModule:
 
     def _workspace_for(self, stream, m: int, n: int, k: int, path: int):
         need = lib().w8a8_linear_workspace_bytes_path(m, n, k, path)
-        if need and not is_capturing(stream):
+        if not need:
+            return None, 0   # none used, or faster without
+        if not is_capturing(stream):
             self.reserve_workspace(need, stream)
         # under capture a missing or small workspace selects the unsplit
         # kernels (identical results), so nothing is allocated

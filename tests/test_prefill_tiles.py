@@ -38,27 +38,30 @@ def test_lane_offsets_fit_32_bits():
             if m * n >= 1 << 32:
                 continue
             fam = route(m, n, k, path=2)["family"]
-            assert staged or fam in ((11, 15) if m <= 64 else (14,)), (m, n, k, fam)
-            if m > 256 and staged:
-                assert fam == 13, (m, n, k, fam)
+            # unstaged: 64-bit row pointers (gemm_skinny, gemm_narrow, the four-wave tiles with a K tail)
+            assert staged or fam in ((11, 15) if m <= 16 else (14,)), (m, n, k, fam)
 
 
-TILES = [((128, 64), 1025, 1003), ((128, 128), 2049, 1003), ((128, 192), 1281, 3003), ((256, 128), 1025, 5503),
-         ((256, 192), 1025, 7253), ((64, 128), 1281, 1503), ((256, 256), 2049, 6003)]
+# (tile, family, m, n, k): eight waves (13), four waves (14), K tails of 16 and
+# 112 bytes, K below one stage
+TILES = [((128, 64), 13, 2049, 515, 1280), ((128, 128), 13, 1025, 2003, 1280), ((128, 192), 13, 1300, 3003, 1280),
+         ((256, 128), 13, 1025, 6003, 1280), ((256, 192), 13, 1300, 6003, 1280), ((64, 128), 13, 129, 6003, 1280),
+         ((256, 256), 13, 2049, 6003, 1280), ((64, 64), 14, 150, 515, 1280), ((64, 64), 14, 17, 33, 16),
+         ((64, 64), 14, 77, 1003, 112), ((64, 64), 14, 257, 515, 1392), ((128, 64), 14, 1025, 2003, 16),
+         ((128, 128), 14, 1300, 3003, 144), ((256, 128), 14, 2049, 2003, 1296), ((256, 256), 14, 1300, 6003, 1296)]
 
 
-@pytest.mark.parametrize("tile,m,n", TILES)
-def test_tile_routes(tile, m, n):
-    r = route(m, n, 1280)
-    assert r["family"] == 13 and (r["bm"], r["bn"]) == tile
+@pytest.mark.parametrize("tile,family,m,n,k", TILES)
+def test_tile_routes(tile, family, m, n, k):
+    r = route(m, n, k)
+    assert (r["family"], r["bm"], r["bn"]) == (family, *tile)
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("tile,m,n", TILES)
-@pytest.mark.parametrize("k", [1280])
-def test_every_tile(tile, m, n, k):
-    """Odd M and N (guarded edges beside whole tiles), K = 10 stages, every
-    output form, guard values past the output untouched."""
+@pytest.mark.parametrize("tile,family,m,n,k", TILES)
+def test_every_tile(tile, family, m, n, k):
+    """Odd M and N (guarded edges beside whole tiles), every output form,
+    guard values past the output untouched."""
     from inferrous_amd import CudaContext, DeviceBuffer, load
     ctx = CudaContext(0)
     mod, s = load(ctx), ctx.new_stream()
