@@ -68,6 +68,35 @@ __device__ __forceinline__ void quant_codes(const float (&v)[N], float s, float 
   }
 }
 
+// Four codes of quantize (src/kernels.rs:441-449, round(RN(v / s)) for
+// s = RN(m / 127), m >= |v|) in one word, without a division per value.  With
+// r = RN(1 / s), two steps q += (v - q s) r make q = RN(v / s): the first brings
+// the product v r within an ulp of the quotient, and by Markstein's theorem (IBM
+// J. Res. Dev. 34(1), 1990) the second, whose remainder is exact, rounds it
+// correctly.  Adding 1.5 * 2^23 then rounds q, ties to even, to the integer that
+// is its low byte; |q| < 127.5, so the clamp has nothing to do.  An infinite s
+// gives NaN, whose low byte is 0, as the code is.  Not for NaN v (its payload
+// would be the code) nor s below 2^-90 (r, or the remainder, could leave the
+// normal range): codes4 takes the division for those.  8 instructions a
+// value with the packing, against 18 with the division.
+__device__ __forceinline__ float code_bits(float v, float s, float r) {
+  float q = v * r;
+  q = __builtin_fmaf(__builtin_fmaf(-q, s, v), r, q);
+  q = __builtin_fmaf(__builtin_fmaf(-q, s, v), r, q);
+  return q + 12582912.0f;
+}
+__device__ __forceinline__ uint32_t pack4_fast(float a, float b, float c, float d, float s, float r) {
+  const uint32_t q0 = __float_as_uint(code_bits(a, s, r)), q1 = __float_as_uint(code_bits(b, s, r));
+  const uint32_t q2 = __float_as_uint(code_bits(c, s, r)), q3 = __float_as_uint(code_bits(d, s, r));
+  const uint32_t lo = __builtin_amdgcn_perm(q1, q0, 0x0c0c0400u), hi = __builtin_amdgcn_perm(q3, q2, 0x04000c0cu);
+  return lo | hi;
+}
+constexpr float kFastScaleMin = 0x1p-90f;
+
+// |x|'s bits: ordered for all but NaN, whose patterns lie above kInfBits.
+constexpr uint32_t kInfBits = 0x7f800000u;
+__device__ __forceinline__ uint32_t abs_bits(float x) { return __float_as_uint(x) & 0x7fffffffu; }
+
 // |x| as ordered bits with NaN mapped to 0 (f32::max ignores NaN,
 // src/kernels.rs:133-139); non-negative floats order like unsigned ints.
 __device__ __forceinline__ uint32_t abs_bits_no_nan(float x) {
@@ -87,6 +116,28 @@ __device__ __forceinline__ uint32_t pack4(float a, float b, float c, float d, fl
   uint32_t q0 = (uint8_t)round_i8(a / s), q1 = (uint8_t)round_i8(b / s);
   uint32_t q2 = (uint8_t)round_i8(c / s), q3 = (uint8_t)round_i8(d / s);
   return q0 | (q1 << 8) | (q2 << 16) | (q3 << 24);
+}
+
+// The four codes by the fast form, or by division where `slow` (a NaN among the
+// thread's values, or a scale below kFastScaleMin).
+__device__ __forceinline__ uint32_t codes4(float a, float b, float c, float d, float s, float r, bool slow) {
+  return slow ? pack4(a, b, c, d, s) : pack4_fast(a, b, c, d, s, r);
+}
+
+// A thread's largest |v| with NaN ignored, at least `floor`: one maximum over the
+// raw bits, and the filtered one only where a NaN shows in it (*nan).
+template <int N>
+__device__ __forceinline__ uint32_t absmax_bits(const float (&v)[N], uint32_t floor, bool* nan) {
+  uint32_t m = floor;
+#pragma unroll
+  for (int i = 0; i < N; ++i) m = max(m, abs_bits(v[i]));
+  *nan = m > kInfBits;
+  if (*nan) {
+    m = floor;
+#pragma unroll
+    for (int i = 0; i < N; ++i) m = max(m, abs_bits_no_nan(v[i]));
+  }
+  return m;
 }
 
 // SiLU(g) * u in the reference's operation order (src/kernels.rs:681,

@@ -1033,10 +1033,10 @@ __device__ __forceinline__ void store_vec(void* p, size_t i, const float (&v)[VE
 // one after another at ~8 ns, were the whole kernel.  Per dispatch, rows of
 // 12,288, swiglu_kernel + the quantizing launch after it -> swiglu_rows with
 // q: 4,096 f32 rows 1,600 + 55 -> 118 us (5.5 TB/s of gate, up, act and
-// codes), 512 BF16 rows 246 + 11 -> 15.1, 129 f32 rows 77 + 5 -> 8.6, 32
-// BF16 rows 24.7 + 7.5 -> 7.1, 4 f32 rows 4.9 + 4.4 -> 6.1.  At 512 rows and
-// fewer the exp, the two divisions and the rounding (about 60 VALU
-// instructions a value) bound it, not the bytes.
+// codes), 512 BF16 rows 246 + 11 -> 13.3, 129 f32 rows 77 + 5 -> 7.3, 32 BF16
+// rows 24.7 + 7.5 -> 5.7, 4 f32 rows 4.9 + 4.4 -> 5.7 (15.1, 8.6, 7.1 and 6.1 with a
+// division per code).  At 512 rows and fewer the exp, the division and the
+// rounding (about 50 VALU instructions a value) bound it, not the bytes.
 constexpr int kSwigluThreads = 512;
 constexpr uint32_t kSwigluRowMax = 16384;  // widest row held in registers
 
@@ -1058,13 +1058,15 @@ __global__ __launch_bounds__(kSwigluThreads) void swiglu_rows(const void* gate, 
     load_vec<BF16, VEC>(up, e, v[i]);
   }
   uint32_t bits = 0;
+  bool nan = false;
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
 #pragma unroll
     for (int e = 0; e < VEC; ++e) v[i][e] = silu_mul(g[i][e], v[i][e]);
     if (t + i * T < nvec) {  // not the clamped repeats: act may be gate's or up's own buffer
-#pragma unroll
-      for (int e = 0; e < VEC; ++e) bits = max(bits, abs_bits_no_nan(v[i][e]));
+      bool here;
+      bits = max(bits, absmax_bits(v[i], 0u, &here));
+      nan |= here;
       store_vec<BF16, VEC>(act, base + (size_t)(t + i * T) * VEC, v[i]);
     }
   }
@@ -1077,21 +1079,18 @@ __global__ __launch_bounds__(kSwigluThreads) void swiglu_rows(const void* gate, 
   if (!q) return;
   const float s = __uint_as_float(max(before, bits)) / 127.0f;
   const float rs = 1.0f / s;
+  const bool slow = nan || s < kFastScaleMin;
   if (t == 0) scales[r] = s;
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
-    int code[VEC];
-    quant_codes<VEC>(v[i], s, rs, code);
     if (t + i * T >= nvec) continue;
     int8_t* const o = q + base + (size_t)(t + i * T) * VEC;
     if constexpr (VEC == 1) {
-      *o = (int8_t)code[0];
+      *o = slow ? round_i8(v[i][0] / s) : (int8_t)__float_as_uint(code_bits(v[i][0], s, rs));
     } else {
 #pragma unroll
       for (int e = 0; e < VEC; e += 4)
-        reinterpret_cast<uint32_t*>(o)[e / 4] = (uint32_t)(uint8_t)code[e] | (uint32_t)(uint8_t)code[e + 1] << 8 |
-                                                (uint32_t)(uint8_t)code[e + 2] << 16 |
-                                                (uint32_t)(uint8_t)code[e + 3] << 24;
+        reinterpret_cast<uint32_t*>(o)[e / 4] = codes4(v[i][e], v[i][e + 1], v[i][e + 2], v[i][e + 3], s, rs, slow);
     }
   }
 }
@@ -1369,12 +1368,22 @@ template <bool BF16, int VEC>
 static void launch_swiglu_rows(hipStream_t st, const char* gate, const char* up, uint32_t rows, uint32_t width,
                                char* act, uint32_t* maxima, int8_t* q, float* scales) {
   const uint32_t nv = (width / VEC + kSwigluThreads - 1) / kSwigluThreads;  // vectors per thread
-  auto k = VEC == 8   ? (nv <= 1 ? swiglu_rows<BF16, VEC, 1> : nv <= 2 ? swiglu_rows<BF16, VEC, 2>
-                         : nv <= 3 ? swiglu_rows<BF16, VEC, 3> : swiglu_rows<BF16, VEC, 4>)
-           : VEC == 4 ? (nv <= 2 ? swiglu_rows<BF16, VEC, 2> : nv <= 4 ? swiglu_rows<BF16, VEC, 4>
-                         : nv <= 6 ? swiglu_rows<BF16, VEC, 6> : swiglu_rows<BF16, VEC, 8>)
-                      : (nv <= 8 ? swiglu_rows<BF16, VEC, 8> : nv <= 24 ? swiglu_rows<BF16, VEC, 24>
-                                                                        : swiglu_rows<BF16, VEC, 32>);
+  auto k = [&] {
+    if constexpr (VEC == 8)
+      return nv <= 1   ? swiglu_rows<BF16, VEC, 1>
+             : nv <= 2 ? swiglu_rows<BF16, VEC, 2>
+             : nv <= 3 ? swiglu_rows<BF16, VEC, 3>
+                       : swiglu_rows<BF16, VEC, 4>;
+    else if constexpr (VEC == 4)
+      return nv <= 2   ? swiglu_rows<BF16, VEC, 2>
+             : nv <= 4 ? swiglu_rows<BF16, VEC, 4>
+             : nv <= 6 ? swiglu_rows<BF16, VEC, 6>
+                       : swiglu_rows<BF16, VEC, 8>;
+    else
+      return nv <= 8    ? swiglu_rows<BF16, VEC, 8>
+             : nv <= 24 ? swiglu_rows<BF16, VEC, 24>
+                        : swiglu_rows<BF16, VEC, 32>;
+  }();
   hipLaunchKernelGGL(k, dim3(rows), dim3(kSwigluThreads), 0, st, gate, up, width, act, maxima, q, scales);
 }
 
