@@ -1184,20 +1184,29 @@ static hipError_t launch_mt(hipStream_t st, GemvArgs& a, const uint32_t* nn, uin
   return hipGetLastError();
 }
 
+// Widest activation row that M = 1 waves hold in registers, in KiB; for the
+// fused selection's 16-wave workgroups, whose waves have half the registers.
+constexpr uint32_t kMaxKC = 16, kMaxKCArgmax = 12;
+
 // Row-group shape: measured on MI355X, waves that issue one short batch
 // (one or two 4 KiB rows) and exit stream HBM better than longer batches or
 // grid-stride sweeps; two rows per wave helps only the small matrices.  M = 1
-// at K = 4096 / 12288: gemv_m1_one (one matrix) or gemv_m1 (siblings, or the
-// fused selection, whose workgroups carry 16 waves: a quarter of the keys of
-// the plain GEMV's 4-wave workgroups).  Otherwise gemv_mt with 4-row groups.
+// at K a multiple of 1024 up to 16 KiB: gemv_m1_one (one matrix) or gemv_m1
+// (siblings, or the fused selection, whose workgroups carry 16 waves: a
+// quarter of the keys of the plain GEMV's 4-wave workgroups), with enough rows
+// per wave for 4 KiB.  Otherwise gemv_mt with 4-row groups.  gemv_mt -> these
+// at other K than 4096 and 12288, us per launch: 13824 x 5120 14.3 -> 11.5, 5120 x
+// 5120 8.2 -> 5.6, 4096 x 8192 8.2 -> 6.5, 8192 x 16384 22.9 -> 21.7, 20480 x 2048
+// 8.7 -> 7.6, 8192 x 3072 6.5 -> 5.3, 16384 x 1024 5.5 -> 4.4; 151,936-row selection at
+// K = 5120 117 -> 113, at 2048 and 8192 level.
 GemvRoute gemv_route(uint32_t m, uint32_t k, const uint32_t* n, int count, bool argmax) {
   GemvRoute r{};
   uint64_t total = 0;
   for (int i = 0; i < count; ++i) total += n[i];
   r.grid_y = 1;
-  if (m == 1 && (k == 4096 || k == 12288)) {
+  if (m == 1 && k % 1024 == 0 && k / 1024 <= (argmax ? kMaxKCArgmax : kMaxKC)) {
     r.family = argmax || count != 1 ? kRouteGemvM1 : kRouteGemvM1One;
-    r.rows = k == 4096 && total <= 8192 ? 2 : 1;
+    r.rows = k == 1024 ? 4 : k == 2048 || k == 3072 || (k == 4096 && total <= 8192) ? 2 : 1;
     r.kc = (int)(k / 1024);
     r.waves = argmax ? 16 : kGemvWaves;
   } else {
@@ -1219,9 +1228,27 @@ static hipError_t dispatch(hipStream_t st, GemvArgs& a, uint32_t* blocks) {
   const GemvRoute r = gemv_route(a.m, a.k, a.n, a.count, EPI == EPI_ARGMAX);
   uint32_t nn[kMaxGroup];
   for (int i = 0; i < a.count; ++i) nn[i] = a.n[i];
-  if (r.family != kRouteGemvMt) {
-    if (r.kc == 12) return launch_m1<1, 12, EPI>(st, a, nn, blocks);
-    return r.rows == 2 ? launch_m1<2, 4, EPI>(st, a, nn, blocks) : launch_m1<1, 4, EPI>(st, a, nn, blocks);
+  switch (r.family != kRouteGemvMt ? r.kc : 0) {
+    case 1: return launch_m1<4, 1, EPI>(st, a, nn, blocks);
+    case 2: return launch_m1<2, 2, EPI>(st, a, nn, blocks);
+    case 3: return launch_m1<2, 3, EPI>(st, a, nn, blocks);
+    case 4: return r.rows == 2 ? launch_m1<2, 4, EPI>(st, a, nn, blocks) : launch_m1<1, 4, EPI>(st, a, nn, blocks);
+    case 5: return launch_m1<1, 5, EPI>(st, a, nn, blocks);
+    case 6: return launch_m1<1, 6, EPI>(st, a, nn, blocks);
+    case 7: return launch_m1<1, 7, EPI>(st, a, nn, blocks);
+    case 8: return launch_m1<1, 8, EPI>(st, a, nn, blocks);
+    case 9: return launch_m1<1, 9, EPI>(st, a, nn, blocks);
+    case 10: return launch_m1<1, 10, EPI>(st, a, nn, blocks);
+    case 11: return launch_m1<1, 11, EPI>(st, a, nn, blocks);
+    case 12: return launch_m1<1, 12, EPI>(st, a, nn, blocks);
+    case 13: case 14: case 15: case 16:
+      if constexpr (EPI != EPI_ARGMAX) {
+        if (r.kc == 13) return launch_m1<1, 13, EPI>(st, a, nn, blocks);
+        if (r.kc == 14) return launch_m1<1, 14, EPI>(st, a, nn, blocks);
+        if (r.kc == 15) return launch_m1<1, 15, EPI>(st, a, nn, blocks);
+        return launch_m1<1, 16, EPI>(st, a, nn, blocks);
+      }
+      return hipErrorInvalidValue;
   }
   if (r.mt == 1) return launch_mt<1, 4, EPI>(st, a, nn, blocks);
   if (r.mt == 2) return launch_mt<2, 4, EPI>(st, a, nn, blocks);
