@@ -36,7 +36,7 @@
 //    one each (M <= 64) or 32-row slices of all BN columns, and those
 //    holding none only move data; activation rows past M are never loaded;
 //    split-K on narrow n.
-//  * gemm_narrow (M <= 16, or M <= 32 on n <= 4096 at k <= 4096, where the
+//  * gemm_narrow (M <= 16, or M <= 64 on n <= 4096 at k <= 4096, where the
 //    n / 96 tiles are fewer than 224 and k splits into S slices of 128-byte
 //    stages): one workgroup owns 16 weight rows; its S waves split K
 //    (contiguous slices at S = 4, interleaved 128-byte chunks at S = 8), and
@@ -180,8 +180,9 @@ __device__ __forceinline__ uint32_t own_tile(GemmArgs& a, const GemmGroup& g, ui
 }
 
 // ---------------------------------------------------------------- narrow
-// Workgroup b owns output columns [16 b, 16 b + 16) and all M rows (MB
-// 16-row blocks).  Wave w sums ST = K / (128 S) of the 128-byte K chunks
+// Workgroup b owns output columns [16 NB b, 16 NB (b + 1)) and all M rows (MB
+// 16-row blocks); NB is 1 but for groups whose 16-column tiles would take
+// the CUs one and a half times.  (Below for NB = 1.)  Wave w sums ST = K / (128 S) of the 128-byte K chunks
 // (the host guarantees K % (128 S) == 0): with S = 4 the contiguous slice
 // w ST .. w ST + ST - 1, stage s reading chunk w ST + s; with S = 8 the
 // waves interleave, stage s reading chunk ((s + b) mod ST) S + w, so that a
@@ -203,20 +204,20 @@ __device__ __forceinline__ uint32_t own_tile(GemmArgs& a, const GemmGroup& g, ui
 // stage is waited for with vmcnt (every issued instruction has a live lane,
 // so the count is exact), and a slot is refilled only after the previous
 // stage's fragment reads have returned.
-template <int MB, int LAL, int S, int R, bool GROUP = false>
+template <int MB, int LAL, int S, int R, bool GROUP = false, int NB = 1>
 __global__ __launch_bounds__(64 * S) void gemm_narrow(GemmArgs a, GroupArg<GROUP> group) {
-  constexpr int ROWS = 16 * (1 + MB);
+  constexpr int ROWS = 16 * (NB + MB);
   constexpr int STAGE = ROWS * 128;
-  constexpr int L = 2 + LAL;  // DMA instructions per stage
+  constexpr int L = 2 * NB + LAL;  // DMA instructions per stage
   constexpr int RING = R * STAGE;
   static_assert(MB >= 1 && LAL >= 1 && LAL <= 2 * MB, "live activation loads");
   static_assert(R >= 2 && (R - 1) * L < 64, "ring depth");
   static_assert(S * RING <= 160 * 1024, "LDS");
-  static_assert(S * MB * 4 * 64 * (int)sizeof(int) <= S * RING, "the reduction reuses the rings");
+  static_assert(S * MB * NB * 4 * 64 * (int)sizeof(int) <= S * RING, "the reduction reuses the rings");
   __shared__ __attribute__((aligned(1024))) int8_t lds[S * RING];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const uint32_t n0 = own_tile(a, group, blockIdx.x) * 16;
+  const uint32_t n0 = own_tile(a, group, blockIdx.x) * 16 * NB;
   const uint32_t K = a.k, M = a.m, N = a.n;
   const uint32_t ST = K / (128 * S);
   int8_t* const ring = lds + wave * RING;
@@ -227,12 +228,12 @@ __global__ __launch_bounds__(64 * S) void gemm_narrow(GemmArgs a, GroupArg<GROUP
   for (int j = 0; j < L; ++j) {
     const int row = 8 * j + (lane >> 3);
     const size_t chunk = (size_t)(((lane & 7) ^ (row & 7)) * 16);
-    if (row < 16) {
+    if (row < 16 * NB) {
       const uint32_t g = n0 + row;
       src[j] = a.w + (size_t)(g < N ? g : N - 1) * K + chunk;
       live[j] = true;
     } else {
-      const uint32_t g = (uint32_t)(row - 16);
+      const uint32_t g = (uint32_t)(row - 16 * NB);
       live[j] = g < M;
       src[j] = a.q + (size_t)(live[j] ? g : 0) * K + chunk;
     }
@@ -248,9 +249,11 @@ __global__ __launch_bounds__(64 * S) void gemm_narrow(GemmArgs a, GroupArg<GROUP
   };
 
   const int fr = lane & 15, fq = lane >> 4;
-  v4i acc[MB];
+  v4i acc[MB][NB];
 #pragma unroll
-  for (int t = 0; t < MB; ++t) acc[t] = v4i{0, 0, 0, 0};
+  for (int t = 0; t < MB; ++t)
+#pragma unroll
+    for (int u = 0; u < NB; ++u) acc[t][u] = v4i{0, 0, 0, 0};
 #pragma unroll
   for (int s = 0; s < R - 1; ++s)
     if ((uint32_t)s < ST) load(s);
@@ -266,12 +269,15 @@ __global__ __launch_bounds__(64 * S) void gemm_narrow(GemmArgs a, GroupArg<GROUP
 #pragma unroll
     for (int h = 0; h < 2; ++h) {  // the stage's two 64-byte k steps
       const int c = 4 * h + fq;
-      const v4i b = *(const v4i*)(base + fr * 128 + ((c ^ (fr & 7)) * 16));
+      v4i b[NB];
+#pragma unroll
+      for (int u = 0; u < NB; ++u) b[u] = *(const v4i*)(base + (16 * u + fr) * 128 + ((c ^ (fr & 7)) * 16));
 #pragma unroll
       for (int t = 0; t < MB; ++t) {
-        const int row = 16 + 16 * t + fr;
+        const int row = 16 * NB + 16 * t + fr;
         const v4i av = *(const v4i*)(base + row * 128 + ((c ^ (row & 7)) * 16));
-        acc[t] = mfma16(av, b, acc[t]);
+#pragma unroll
+        for (int u = 0; u < NB; ++u) acc[t][u] = mfma16(av, b[u], acc[t][u]);
       }
     }
   }
@@ -280,16 +286,19 @@ __global__ __launch_bounds__(64 * S) void gemm_narrow(GemmArgs a, GroupArg<GROUP
 #pragma unroll
   for (int t = 0; t < MB; ++t)
 #pragma unroll
-    for (int v = 0; v < 4; ++v) red[((wave * MB + t) * 4 + v) * 64 + lane] = acc[t][v];
+    for (int u = 0; u < NB; ++u)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) red[(((wave * MB + t) * NB + u) * 4 + v) * 64 + lane] = acc[t][u][v];
   __syncthreads();
-  // value v of lane l of block t: row 16 t + 4 (l / 16) + v, column n0 + l % 16
-  for (int i = threadIdx.x; i < MB * 4 * 64; i += 64 * S) {
-    const int l = i & 63, v = (i >> 6) & 3, t = i >> 8;
+  // value v of lane l of block (t, u): row 16 t + 4 (l / 16) + v, column
+  // n0 + 16 u + l % 16
+  for (int i = threadIdx.x; i < MB * NB * 4 * 64; i += 64 * S) {
+    const int l = i & 63, v = (i >> 6) & 3, u = (i >> 8) % NB, t = (i >> 8) / NB;
     int sum = 0;
 #pragma unroll
-    for (int w = 0; w < S; ++w) sum += red[((w * MB + t) * 4 + v) * 64 + l];
+    for (int w = 0; w < S; ++w) sum += red[w * (MB * NB * 256) + i];
     const uint32_t r = 16 * t + 4 * (l >> 4) + v;
-    const uint32_t c = n0 + (l & 15);
+    const uint32_t c = n0 + 16 * u + (l & 15);
     if (r < M && c < N) epilogue_store(a, r, c, sum);
   }
 }
@@ -1179,8 +1188,9 @@ static bool split_plan(uint32_t m, uint32_t n, uint32_t k, uint32_t& splits) {
 // gemm_narrow's plan: S = 4 waves below K = 8192 and 8 from there (each wave
 // keeps eight or more 128-byte stages), R-deep rings, MB 16-row blocks, LAL
 // = ceil(M / 8) activation DMA loads per stage.  It takes M <= 16 on the
-// narrow shapes, and M <= 32 where one workgroup per 16 columns fits the
-// CUs once at K <= 4096; the wide shapes (n / 96 >= 224 tiles) keep
+// narrow shapes, and M <= 64 where one workgroup per 16 columns fits the
+// CUs once at K <= 4096 (o at M = 48 / 64 6.6 / 7.6 us against gemm_tall split
+// K's 8.9 / 8.8); the wide shapes (n / 96 >= 224 tiles) keep
 // gemm_tall's unsplit 96-column tiles.  Measured on MI355X, graphs of 36
 // distinct-weight launches, random operands, against the routes it
 // replaced (gemm_tall split-K 4 with its slab epilogue launch, gemm_skinny),
@@ -1197,13 +1207,13 @@ static bool split_plan(uint32_t m, uint32_t n, uint32_t k, uint32_t& splits) {
 // measured level or slower.  These down figures are for contiguous K slices;
 // the interleaved order the kernel now takes at S = 8 runs 2-3% faster.
 static bool narrow_plan(uint32_t m, uint32_t n, uint32_t k, int& S, int& R, int& MB, int& LAL) {
-  if (m == 0 || m > 32 || (n + 95) / 96 >= 224) return false;
+  if (m == 0 || m > 64 || (n + 95) / 96 >= 224) return false;
   S = k >= 8192 ? 8 : 4;
   if (k % (128u * S) != 0) return false;
   if (m > 16 && !(k <= 4096 && (n + 15) / 16 <= 256)) return false;
-  MB = m <= 16 ? 1 : 2;  // two blocks only at S = 4 (K <= 4096)
+  MB = (int)((m + 15) / 16);  // more than one only at S = 4 (K <= 4096)
   LAL = (int)((m + 7) / 8);
-  R = 4;
+  R = MB <= 3 ? 4 : 3;  // LDS
   return true;
 }
 
@@ -1513,28 +1523,32 @@ hipError_t launch_gemm_timeline(hipStream_t st, const GemmArgs& a, uint64_t* sta
   return launch_tall_timed<64, 4, 4, 256>(st, a, r.splits, stamps);
 }
 
-template <int MB, int LAL, int S, int R>
-static hipError_t launch_narrow_as(hipStream_t st, const GemmArgs& a, uint32_t grid) {
-  hipLaunchKernelGGL((gemm_narrow<MB, LAL, S, R>), dim3(grid), dim3(64 * S), 0, st, a, NoGroup{});
+template <int MB, int LAL, int S, int R, int NB = 1, class G>
+static hipError_t launch_narrow_as(hipStream_t st, const GemmArgs& a, const G& g, uint32_t grid) {
+  constexpr bool GROUP = std::is_same_v<G, GemmGroup>;
+  hipLaunchKernelGGL((gemm_narrow<MB, LAL, S, R, GROUP, NB>), dim3(grid), dim3(64 * S), 0, st, a, g);
   return hipGetLastError();
 }
 
-// The instantiations narrow_plan can ask for: S = 4 with one or two 16-row
-// blocks, S = 8 (K >= 8192) with one; LAL = ceil(M / 8); R = 4.
-static hipError_t launch_narrow(hipStream_t st, const GemmArgs& a, const GemmRoute& r) {
-  const uint32_t g = r.grid_x;
+// The instantiations the plans can ask for: S = 4 with one to four 16-row
+// blocks, S = 8 (K >= 8192) with one; LAL = ceil(M / 8); NB = 2 from two blocks
+// on, for groups.
+template <int NB, class G>
+static hipError_t launch_narrow(hipStream_t st, const GemmArgs& a, const G& g, const GemmRoute& r) {
+  const uint32_t n = r.grid_x;
   if (r.s == 4) {
     switch (r.u) {
-      case 1: return launch_narrow_as<1, 1, 4, 4>(st, a, g);
-      case 2: return launch_narrow_as<1, 2, 4, 4>(st, a, g);
-      case 3: return launch_narrow_as<2, 3, 4, 4>(st, a, g);
-      case 4: return launch_narrow_as<2, 4, 4, 4>(st, a, g);
+      case 3: return launch_narrow_as<2, 3, 4, 4, NB>(st, a, g, n);
+      case 4: return launch_narrow_as<2, 4, 4, 4, NB>(st, a, g, n);
+      case 5: return launch_narrow_as<3, 5, 4, 4, NB>(st, a, g, n);
+      case 6: return launch_narrow_as<3, 6, 4, 4, NB>(st, a, g, n);
+      case 7: return launch_narrow_as<4, 7, 4, 3, NB>(st, a, g, n);
+      case 8: return launch_narrow_as<4, 8, 4, 3, NB>(st, a, g, n);
     }
-  } else if (r.s == 8) {
-    switch (r.u) {
-      case 1: return launch_narrow_as<1, 1, 8, 4>(st, a, g);
-      case 2: return launch_narrow_as<1, 2, 8, 4>(st, a, g);
-    }
+    if constexpr (NB == 1)
+      return r.u == 1 ? launch_narrow_as<1, 1, 4, 4>(st, a, g, n) : launch_narrow_as<1, 2, 4, 4>(st, a, g, n);
+  } else if constexpr (NB == 1) {
+    return r.u == 1 ? launch_narrow_as<1, 1, 8, 4>(st, a, g, n) : launch_narrow_as<1, 2, 8, 4>(st, a, g, n);
   }
   return hipErrorInvalidValue;
 }
@@ -1564,7 +1578,7 @@ hipError_t launch_gemm(hipStream_t st, const GemmArgs& a) {
         return r.splits > 1 ? launch_tall<96, 3, 3, 256>(st, a, r.splits) : launch_tall<96, 2, 4, 256>(st, a, r.splits);
       return launch_tall<64, 4, 4, 256>(st, a, r.splits);
     case kRouteNarrow:
-      return launch_narrow(st, a, r);
+      return launch_narrow<1>(st, a, NoGroup{}, r);
     case kRouteSkinny:
       hipLaunchKernelGGL((gemm_skinny<1, 4, 4>), dim3(r.grid_x, 1), dim3(r.block), 0, st, a);
       return hipGetLastError();
@@ -1584,12 +1598,6 @@ hipError_t launch_gemm(hipStream_t st, const GemmArgs& a) {
 }
 
 // ---------------------------------------------------------------- grouped
-template <int MB, int LAL, int S, int R>
-static hipError_t launch_narrow_group(hipStream_t st, const GemmArgs& a, const GemmGroup& g, uint32_t grid) {
-  hipLaunchKernelGGL((gemm_narrow<MB, LAL, S, R, true>), dim3(grid), dim3(64 * S), 0, st, a, g);
-  return hipGetLastError();
-}
-
 template <int BN, int SA, int SB, int MA>
 static hipError_t launch_tall_group(hipStream_t st, const GemmArgs& a, const GemmGroup& g, uint32_t tn) {
   auto k = a.out_dtype == W8A8_OUT_I32   ? gemm_tall<BN, SA, SB, MA, EP_I32, kRotateK, false, true>
@@ -1642,6 +1650,17 @@ GemmRoute gemm_group_route(uint32_t m, uint32_t k, const uint32_t* n, int count)
     r.grid_x = (uint32_t)tiles(16);
     return r;
   }
+  // Two 16-column blocks per workgroup where that fits the CUs once: 6144 x 4096
+  // at M = 24 / 32 / 48 / 64 7.9 / 8.1 / 9.6 / 10.5 us against 11.6 / 11.2 / 11.5 /
+  // 11.5 on 64 x 64 tiles.
+  if (m > 16 && m <= 64 && k <= 4096 && k % 512 == 0 && tiles(32) <= kCus) {
+    r.family = kRouteNarrow;
+    r.mt = (int)((m + 15) / 16), r.s = 4, r.u = (int)((m + 7) / 8), r.sa = m <= 48 ? 4 : 3;
+    r.bn = 32;
+    r.block = 256;
+    r.grid_x = (uint32_t)tiles(32);
+    return r;
+  }
   if (m <= 256 && tiles(96) >= 224) {
     r.family = kRouteTall;
     r.ma = m <= 64 ? 64 : m <= 160 ? 160 : 256;
@@ -1665,17 +1684,7 @@ hipError_t launch_gemm_group(hipStream_t st, const GemmArgs& a, GemmGroup& g) {
     g.tbegin[i] = tn;
     if (i < g.count) tn += (g.n[i] + r.bn - 1) / r.bn;
   }
-  if (r.family == kRouteNarrow) {
-    if (r.s == 4) {
-      switch (r.u) {
-        case 1: return launch_narrow_group<1, 1, 4, 4>(st, a, g, tn);
-        case 2: return launch_narrow_group<1, 2, 4, 4>(st, a, g, tn);
-        case 3: return launch_narrow_group<2, 3, 4, 4>(st, a, g, tn);
-        default: return launch_narrow_group<2, 4, 4, 4>(st, a, g, tn);
-      }
-    }
-    return r.u == 1 ? launch_narrow_group<1, 1, 8, 4>(st, a, g, tn) : launch_narrow_group<1, 2, 8, 4>(st, a, g, tn);
-  }
+  if (r.family == kRouteNarrow) return r.bn == 32 ? launch_narrow<2>(st, a, g, r) : launch_narrow<1>(st, a, g, r);
   if (r.family == kRouteTall) {
     return r.ma == 64    ? launch_tall_group<96, 4, 4, 64>(st, a, g, tn)
            : r.ma == 160 ? launch_tall_group<96, 4, 4, 160>(st, a, g, tn)

@@ -56,6 +56,14 @@ def test_rows_and_ragged_columns(env, m, k, ns):
     check(env, m, k, ns, np.uint16)
 
 
+@pytest.mark.parametrize("m", [17, 24, 25, 32, 33, 40, 41, 48, 49, 56, 57, 64])
+@pytest.mark.parametrize("k,ns", [(512, (4100, 33, 1, 7)), (4096, (4096, 1024, 1024))])
+def test_narrow_two_column_blocks(env, m, k, ns):
+    """gemm_narrow on 32 columns per workgroup (and, for the single
+    projections, on 16), every count of live activation loads."""
+    check(env, m, k, ns, np.uint16)
+
+
 @pytest.mark.parametrize("m", [3, 16, 40, 130, 250])
 @pytest.mark.parametrize("dtype", [np.float32, np.int32])
 def test_wide_group_one_m_tile(env, m, dtype):
