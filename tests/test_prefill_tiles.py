@@ -57,6 +57,26 @@ def test_tile_routes(tile, family, m, n, k):
     assert (r["family"], r["bm"], r["bn"]) == (family, *tile)
 
 
+@pytest.mark.parametrize("tile,family,m,n,k", [c for c in TILES if c[4] % 128])
+def test_tail_reads_stay_inside(tile, family, m, n, k):
+    """gemm_dma's DMA sources with a partial last stage (loadA, loadB): every
+    16-byte read of every tile lies inside its operand, each live row's chunks
+    below K are read once, and a chunk past K meets zeros."""
+    bm, bn = tile
+    stages = k // 128 + 1
+    for rows, b in ((m, bm), (n, bn)):
+        row, c = np.divmod(np.arange(b * 8), 8)
+        chunk = (c ^ ((row >> 1) & 7)) * 16
+        kk = np.arange(stages)[:, None] * 128 + chunk
+        for first in range(0, rows, b):
+            src = np.where(first + row < rows, row, 0)
+            live = kk < k
+            at = (first + src) * k + np.where(live, kk, 0)  # weights; activations past K read zeros instead
+            assert at.min() >= 0 and (at + 16).max() <= rows * k
+            for r in {0, min(b, rows - first) - 1}:
+                assert np.array_equal(np.sort(kk[:, row == r][live[:, row == r]]), np.arange(0, k, 16))
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("tile,family,m,n,k", TILES)
 def test_every_tile(tile, family, m, n, k):
