@@ -1079,7 +1079,7 @@ __global__ __launch_bounds__(kSwigluThreads) void swiglu_rows(const void* gate, 
   if (!q) return;
   const float s = __uint_as_float(max(before, bits)) / 127.0f;
   const float rs = 1.0f / s;
-  const bool slow = nan || s < kFastScaleMin;
+  const bool slow = nan || !(s >= kFastScaleMin);  // also a NaN maximum's scale: its payload would be the codes
   if (t == 0) scales[r] = s;
 #pragma unroll
   for (int i = 0; i < NV; ++i) {

@@ -92,3 +92,28 @@ def test_row_codes(env, m, n, dtype):
     wq, ws = oracle.quantize_with_max(a, n, np.array(want, np.uint32))
     assert np.array_equal(codes.to_host_vec(s), wq)
     assert np.array_equal(bits(sc.to_host_vec(s)), bits(ws))
+
+
+@pytest.mark.parametrize("n", [7, 2048])
+@pytest.mark.parametrize("dtype", [np.float32, np.uint16])
+def test_row_codes_under_a_nan_maximum(env, n, dtype):
+    """A maximum whose bits are a NaN (the caller's: no producer folds one)
+    gives a NaN scale and the codes 0, as quantize_with_max does, whatever
+    the payload."""
+    mod, s = env
+    m, k = 5, 32
+    rng = np.random.default_rng(n)
+    mats = [(dev(s, rng.integers(-127, 128, (n, k), dtype=np.int8)), dev(s, (rng.random(n) / 64).astype(F32)))
+            for _ in range(2)]
+    q, asc = dev(s, rng.integers(-127, 128, (m, k), dtype=np.int8)), dev(s, (rng.random(m) / 64).astype(F32))
+    g, u, act = (DeviceBuffer.zeroed(s, m * n, dtype) for _ in range(3))
+    start = np.array([0x7f800055, 0x7fc00001, 0xffffffff, 0x7fabcdef, FLOOR], np.uint32)
+    mx = dev(s, start)
+    codes, sc = dev(s, np.full(m * n, 9, np.int8)), DeviceBuffer.zeroed(s, m, F32)
+    mod.linear_swiglu_quantize(s, None, q, asc, k, *mats[0], g, *mats[1], u, act, mx, codes, sc)
+    a = values(act, s)
+    got, scales = codes.to_host_vec(s).reshape(m, n), sc.to_host_vec(s)
+    assert np.isnan(scales[:4]).all() and (got[:4] == 0).all()
+    assert mx.to_host_vec(s)[:4].tolist() == start[:4].tolist()
+    wq, _ = oracle.quantize_with_max(a[4 * n:], n, np.array([fold_max(a[4 * n:])], np.uint32))
+    assert np.array_equal(got[4], wq)
