@@ -1418,7 +1418,14 @@ static void launch_swiglu_rows(hipStream_t st, const char* gate, const char* up,
 // (q with scales, optional, maxima required).  Without maxima one elementwise
 // pass; rows of up to kSwigluRowMax values (what a workgroup's registers
 // hold) by swiglu_rows, one workgroup per row; wider rows by swiglu_kernel's
-// many workgroups per row, then the row tail.
+// many workgroups per row, then the row tail.  swiglu_rows writes a row's
+// codes while other rows' gate and up are still to be read, so codes or scales
+// that share memory with those (a caller may reuse either once act exists) are
+// written by the row tail too.
+static bool overlap(const void* a, size_t abytes, const void* b, size_t bbytes) {
+  return (uintptr_t)a < (uintptr_t)b + bbytes && (uintptr_t)b < (uintptr_t)a + abytes;
+}
+
 hipError_t launch_swiglu(hipStream_t st, const void* gate, const void* up, size_t rows, uint32_t width, void* act,
                          int dtype, uint32_t* maxima, int8_t* q, float* scales) {
   if (rows == 0 || width == 0) return hipSuccess;
@@ -1436,7 +1443,11 @@ hipError_t launch_swiglu(hipStream_t st, const void* gate, const void* up, size_
     hipLaunchKernelGGL(k, dim3(blocks), dim3(kGemvThreads), 0, st, gate, up, nvec, act);
     return hipGetLastError();
   }
+  const size_t values = rows * (size_t)width, in_bytes = values * esz;
+  const bool shared = overlap(q, values, gate, in_bytes) || overlap(q, values, up, in_bytes) ||
+                      overlap(scales, 4 * rows, gate, in_bytes) || overlap(scales, 4 * rows, up, in_bytes);
   const bool held = width <= kSwigluRowMax, wide = al && width % vec == 0;
+  const bool one_pass = held && q && !shared;
   const uint32_t bx = std::min<uint32_t>((width + kGemvThreads - 1) / kGemvThreads, 64u);
   const size_t chunk = held ? size_t(1) << 22 : 65535;  // rows per launch (grid limits)
   for (size_t r0 = 0; r0 < rows; r0 += chunk) {
@@ -1445,19 +1456,23 @@ hipError_t launch_swiglu(hipStream_t st, const void* gate, const void* up, size_
     const char* const g = (const char*)gate + off * esz;
     const char* const u = (const char*)up + off * esz;
     char* const o = (char*)act + off * esz;
-    int8_t* const qr = q ? q + off : nullptr;
-    float* const sr = scales ? scales + r0 : nullptr;
-    if (held) {
-      if (wide && bf16) launch_swiglu_rows<true, 8>(st, g, u, nr, width, o, maxima + r0, qr, sr);
-      else if (wide) launch_swiglu_rows<false, 4>(st, g, u, nr, width, o, maxima + r0, qr, sr);
-      else if (bf16) launch_swiglu_rows<true, 1>(st, g, u, nr, width, o, maxima + r0, qr, sr);
-      else launch_swiglu_rows<false, 1>(st, g, u, nr, width, o, maxima + r0, qr, sr);
-    } else {
+    int8_t* const qr = one_pass ? q + off : nullptr;
+    float* const sr = one_pass ? scales + r0 : nullptr;
+    if (!held)
       hipLaunchKernelGGL(swiglu_kernel, dim3(bx, nr), dim3(kGemvThreads), 0, st, g, u, width, o, dtype, maxima + r0);
-      if (q)
-        hipLaunchKernelGGL(swiglu_row_tail<false>, dim3(nr), dim3(kRowTailThreads), 0, st, o, width, dtype,
-                           maxima + r0, qr, sr);
-    }
+    else if (wide && bf16) launch_swiglu_rows<true, 8>(st, g, u, nr, width, o, maxima + r0, qr, sr);
+    else if (wide) launch_swiglu_rows<false, 4>(st, g, u, nr, width, o, maxima + r0, qr, sr);
+    else if (bf16) launch_swiglu_rows<true, 1>(st, g, u, nr, width, o, maxima + r0, qr, sr);
+    else launch_swiglu_rows<false, 1>(st, g, u, nr, width, o, maxima + r0, qr, sr);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  if (!q || one_pass) return hipSuccess;
+  constexpr size_t kTailRows = size_t(1) << 21;  // rows per launch (grid limits)
+  for (size_t r0 = 0; r0 < rows; r0 += kTailRows) {
+    const size_t off = r0 * width;
+    hipLaunchKernelGGL(swiglu_row_tail<false>, dim3((uint32_t)std::min(rows - r0, kTailRows)), dim3(kRowTailThreads), 0,
+                       st, (char*)act + off * esz, width, dtype, maxima + r0, q + off, scales + r0);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }

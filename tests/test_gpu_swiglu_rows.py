@@ -117,3 +117,36 @@ def test_row_codes_under_a_nan_maximum(env, n, dtype):
     assert mx.to_host_vec(s)[:4].tolist() == start[:4].tolist()
     wq, _ = oracle.quantize_with_max(a[4 * n:], n, np.array([fold_max(a[4 * n:])], np.uint32))
     assert np.array_equal(got[4], wq)
+
+
+@pytest.mark.parametrize("n", [8, 2048, 16400])
+@pytest.mark.parametrize("dtype", [np.float32, np.uint16])
+@pytest.mark.parametrize("reuse", ["gate", "up"])
+def test_codes_over_gate_or_up(env, n, dtype, reuse):
+    """The codes and scales may take the memory of gate or up, which nothing
+    reads once act exists (rows that other workgroups have not read yet
+    included)."""
+    mod, s = env
+    m, k = 70, 32
+    rng = np.random.default_rng(n)
+    mats = [(dev(s, rng.integers(-127, 128, (n, k), dtype=np.int8)), dev(s, (rng.random(n) / 64).astype(F32)))
+            for _ in range(2)]
+    q, asc = dev(s, rng.integers(-127, 128, (m, k), dtype=np.int8)), dev(s, (rng.random(m) / 64).astype(F32))
+    size = m * n * np.dtype(dtype).itemsize
+    whole = DeviceBuffer.zeroed(s, size + 4 * m, np.int8)
+    shared = DeviceBuffer.view_of(whole, 0, m * n, dtype)
+    other, act = (DeviceBuffer.zeroed(s, m * n, dtype) for _ in range(2))
+    g, u = (shared, other) if reuse == "gate" else (other, shared)
+    codes = DeviceBuffer.view_of(whole, size - m * n, m * n)  # the buffer's last bytes: the last rows' inputs
+    sc = DeviceBuffer.view_of(whole, 0, m, np.float32) if dtype == np.float32 else DeviceBuffer.zeroed(s, m, F32)
+    mx = dev(s, np.full(m, FLOOR, np.uint32))
+    mod.linear_swiglu_quantize(s, None, q, asc, k, *mats[0], g, *mats[1], u, act, mx, codes, sc)
+    a = values(act, s)
+    plain = [DeviceBuffer.zeroed(s, m * n, dtype) for _ in range(3)]
+    mod.linear_swiglu(s, None, q, asc, k, *mats[0], plain[0], *mats[1], plain[1], plain[2], None)
+    assert np.array_equal(a.view(np.uint32), values(plain[2], s).view(np.uint32))
+    want = [fold_max(row) for row in a.reshape(m, n)]
+    assert mx.to_host_vec(s).tolist() == want
+    wq, ws = oracle.quantize_with_max(a, n, np.array(want, np.uint32))
+    assert np.array_equal(codes.to_host_vec(s), wq)
+    assert np.array_equal(bits(sc.to_host_vec(s)), bits(ws))
