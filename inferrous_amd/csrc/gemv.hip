@@ -967,7 +967,8 @@ __global__ __launch_bounds__((NS + kProdWaves) * kWave) void gemv_rowtail_split(
 
 // swiglu (src/kernels.rs:2172-2190): act = silu_mul(gate, up) elementwise
 // over rows x width (blockIdx.y = row); with maxima, each row's largest
-// |act| is published into maxima[row].  Rows wider than swiglu_rows holds.
+// |act| is published into maxima[row].  Rows wider than swiglu_rows holds, and
+// few or narrow rows without codes.
 __global__ __launch_bounds__(kGemvThreads) void swiglu_kernel(const void* gate, const void* up,
                                                                uint32_t width, void* act, int dtype,
                                                                uint32_t* maxima) {
@@ -1418,7 +1419,14 @@ static void launch_swiglu_rows(hipStream_t st, const char* gate, const char* up,
 // (q with scales, optional, maxima required).  Without maxima one elementwise
 // pass; rows of up to kSwigluRowMax values (what a workgroup's registers
 // hold) by swiglu_rows, one workgroup per row; wider rows by swiglu_kernel's
-// many workgroups per row, then the row tail.  swiglu_rows writes a row's
+// many workgroups per row, then the row tail.  Without codes swiglu_kernel also
+// leads where its atomics are few (up to 4 rows, or 32 in all) or a row fills
+// no more than its own one or two workgroups; swiglu_kernel / swiglu_rows with
+// a maxima reset before each, us, f32: 1 x 12,288 4.1 / 6.0, 4 x 16,384 6.2 / 7.5,
+// 8 x 4096 4.9 / 4.3, 8 x 1024 4.0 / 4.2, 16 x 1024 4.2 / 4.2, 4,096 x 64 6.1 /
+// 16.4, 65,536 x 128 53 / 203, 65,536 x 512 128 / 213, 16,384 x 1000 95 / 62.
+// With codes its second launch costs more than that (linear_swiglu_quantize at
+// K = 32, 4,096 x 64 46 / 22, 65,536 x 64 303 / 230).  swiglu_rows writes a row's
 // codes while other rows' gate and up are still to be read, so codes or scales
 // that share memory with those (a caller may reuse either once act exists) are
 // written by the row tail too.
@@ -1446,9 +1454,10 @@ hipError_t launch_swiglu(hipStream_t st, const void* gate, const void* up, size_
   const size_t values = rows * (size_t)width, in_bytes = values * esz;
   const bool shared = overlap(q, values, gate, in_bytes) || overlap(q, values, up, in_bytes) ||
                       overlap(scales, 4 * rows, gate, in_bytes) || overlap(scales, 4 * rows, up, in_bytes);
-  const bool held = width <= kSwigluRowMax, wide = al && width % vec == 0;
-  const bool one_pass = held && q && !shared;
+  const bool wide = al && width % vec == 0, one_pass = width <= kSwigluRowMax && q && !shared;
   const uint32_t bx = std::min<uint32_t>((width + kGemvThreads - 1) / kGemvThreads, 64u);
+  const bool few = rows <= 4 || width <= 512 || rows * bx <= 32;  // atomics, above
+  const bool held = one_pass || (width <= kSwigluRowMax && !few);
   const size_t chunk = held ? size_t(1) << 22 : 65535;  // rows per launch (grid limits)
   for (size_t r0 = 0; r0 < rows; r0 += chunk) {
     const uint32_t nr = (uint32_t)std::min<size_t>(rows - r0, chunk);

@@ -150,3 +150,27 @@ def test_codes_over_gate_or_up(env, n, dtype, reuse):
     wq, ws = oracle.quantize_with_max(a, n, np.array(want, np.uint32))
     assert np.array_equal(codes.to_host_vec(s), wq)
     assert np.array_equal(bits(sc.to_host_vec(s)), bits(ws))
+
+
+@pytest.mark.parametrize("rows,width", [(1, 16384), (4, 12288), (5, 12288), (300, 512), (300, 513), (8, 1024),
+                                        (8, 1025), (32, 256), (70000, 3)])
+@pytest.mark.parametrize("dtype", [np.float32, np.uint16])
+def test_route_edges_without_codes(env, rows, width, dtype):
+    """Either side of the lines between swiglu_kernel and swiglu_rows (and
+    more rows than a grid's y extent): act and the folded maxima."""
+    mod, s = env
+    rng = np.random.default_rng(rows + width)
+    g, u = (oracle.bf16_rne((rng.standard_normal(rows * width) * 3).astype(F32)) for _ in range(2))
+    enc = (lambda a: a) if dtype == np.float32 else (lambda a: (bits(a) >> 16).astype(np.uint16))
+    dg, du = dev(s, enc(g)), dev(s, enc(u))
+    flat, act = (DeviceBuffer.zeroed(s, rows * width, dtype) for _ in range(2))
+    start = np.full(rows, FLOOR, np.uint32)
+    start[rows // 2] = bits(F32(1e30))[0]
+    mx = dev(s, start)
+    code = OUT_F32 if dtype == np.float32 else OUT_BF16
+    assert lib().w8a8_swiglu(s.handle, dg.ptr, du.ptr, rows, width, flat.ptr, None, code) == 0
+    assert lib().w8a8_swiglu(s.handle, dg.ptr, du.ptr, rows, width, act.ptr, mx.ptr, code) == 0
+    got = values(act, s).reshape(rows, width)
+    assert np.array_equal(got.view(np.uint32), values(flat, s).reshape(rows, width).view(np.uint32))
+    act_close(got.ravel(), g, u)
+    assert np.array_equal(mx.to_host_vec(s), np.maximum(start, (got.view(np.uint32) & 0x7fffffff).max(axis=1)))
