@@ -455,6 +455,19 @@ __device__ __forceinline__ void store_blocks(const GemmArgs& a, const v16i (&acc
 // most panels once per tile: 24576 x 4096 at M = 4096, f32, 256 x 192 tiles
 // 484 -> 443 us; strips of 4 / 8 / 16 on 256 x 256 tiles 387 / 397 / 430.
 constexpr uint32_t kStrip = 4;
+// Rotated K (unsplit, K % 128 == 0): stage kt of tile t reads K chunk (kt + t)
+// mod KT, so that the workgroups do not all read the same 128-byte column of
+// their rows at once; the i32 sums are exact in any order.  It pays in a
+// launch of one round whose M tiles are few, and with one column of tiles,
+// where every workgroup walks the same weights (K = 16384 puts all their rows
+// on one channel); with several strips it loses the panels that they share.
+// Distinct weights, BF16, in order -> rotated, us: 6144 x 4096 at M = 256 16.4
+// -> 16.1, M = 512 21.6 -> 21.1, 4096 x 4096 at M = 300 16.5 -> 15.9, M = 768
+// 21.3 -> 20.8, 64 x 16384 at M = 22,000 87 -> 69; not taken: 6144 x 4096 at M =
+// 2048 51.8 -> 56.8, 4096 x 4096 at M = 4096 66 -> 69, and on 64 x 64 tiles 4096 x
+// 4096 at M = 129 11.7 -> 11.8.
+constexpr uint32_t kRotateTiles = 256;  // one per CU
+constexpr uint32_t kRotateRows = 768;
 constexpr uint32_t kMaxK = 1u << 23;  // 256 rows of K bytes stay within a 32-bit offset
 
 // TAIL (K % 128 != 0, any N): the last stage is partial.  A lane whose 16-byte
@@ -500,6 +513,13 @@ __global__ __launch_bounds__(64 * NW, (waves_per_simd(NW, (SA * BM + SB * BN) * 
   const uint32_t K = a.k, KT = TAIL ? K / 128 + 1 : K / 128 / splits;
   const size_t kbase = (size_t)split * KT * 128;
   if (raw_i32(EP)) a.out = reinterpret_cast<int32_t*>(a.out) + (size_t)split * a.m * a.n;
+  const bool turned =
+      !TAIL && splits == 1 && T <= kRotateTiles && (tiles_n == 1 || (NW == 8 && a.m <= kRotateRows));
+  const uint32_t rot = turned ? Lt % KT : 0;
+  auto kc = [&](uint32_t kt) -> size_t {  // byte offset of stage kt
+    const uint32_t c = kt + rot;
+    return (size_t)(c >= KT ? c - KT : c) * 128;
+  };
 
   // Sources of this wave's DMA loads (8 rows each); rows past M / N re-read
   // the tile's first row (their products only reach accumulator cells that are never
@@ -524,7 +544,7 @@ __global__ __launch_bounds__(64 * NW, (waves_per_simd(NW, (SA * BM + SB * BN) * 
     offB[j] = (Off)(n0 + row < a.n ? row : 0) * K + (TAIL ? 0 : chunk(wave * LB + j));
   }
   auto loadA = [&](uint32_t kt, int j) {
-    const int8_t* p = srcA + (size_t)kt * 128 + offA[j];
+    const int8_t* p = srcA + kc(kt) + offA[j];
     if constexpr (TAIL) {
       const uint32_t kk = kt * 128 + chunk(wave * LA + j);
       p = kk < K ? srcA + offA[j] + kk : reinterpret_cast<const int8_t*>(&kZeroChunk);
@@ -534,7 +554,7 @@ __global__ __launch_bounds__(64 * NW, (waves_per_simd(NW, (SA * BM + SB * BN) * 
                                      16, 0, 0);
   };
   auto loadB = [&](uint32_t kt, int j) {
-    const int8_t* p = srcB + (size_t)kt * 128 + offB[j];
+    const int8_t* p = srcB + kc(kt) + offB[j];
     if constexpr (TAIL) {
       const uint32_t kk = kt * 128 + chunk(wave * LB + j);
       p = srcB + offB[j] + (kk < K ? kk : 0);

@@ -111,3 +111,24 @@ def test_every_tile(tile, family, m, n, k):
             got = b.to_host_vec(s)
             assert np.array_equal(got[:m * n].view(np.uint8), v.reshape(-1).view(np.uint8)), (dtype, residual)
             assert (got[m * n:] == 7).all(), (dtype, residual)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k", [(512, 6003, 128), (512, 6003, 1280), (768, 4003, 1280), (769, 4003, 1280),
+                                   (5000, 60, 1280), (22000, 60, 640), (33000, 61, 256), (300, 2003, 16384)])
+def test_rotated_k(m, n, k):
+    """Both sides of gemm_dma's rule for starting each tile at its own K stage
+    (one round of tiles at up to 768 rows, or one column of tiles): the sums."""
+    from inferrous_amd import CudaContext, DeviceBuffer, load
+    ctx = CudaContext(0)
+    mod, s = load(ctx), ctx.new_stream()
+    print(f"rotated m={m} n={n} k={k}", flush=True)
+    rng = np.random.default_rng(m + n)
+    q = rng.integers(-127, 128, (m, k), dtype=np.int8)
+    w = rng.integers(-127, 128, (n, k), dtype=np.int8)
+    asc, ws = np.ones(m, np.float32), np.ones(n, np.float32)
+    acc, _, _ = oracle.linear(q, asc, w, ws, k, threads=8)
+    dq, da, dw, dws = (DeviceBuffer.from_host(s, np.ascontiguousarray(a)) for a in (q, asc, w, ws))
+    out = DeviceBuffer.zeroed(s, m * n, np.int32)
+    mod.linear(s, None, dq, da, dw, dws, k, out)
+    assert np.array_equal(out.to_host_vec(s), acc.reshape(-1))
