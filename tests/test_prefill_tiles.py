@@ -57,6 +57,15 @@ def test_tile_routes(tile, family, m, n, k):
     assert (r["family"], r["bm"], r["bn"]) == (family, *tile)
 
 
+@pytest.mark.parametrize("m,n,k,tile", [(300, 4096, 4096, (128, 64)), (700, 2560, 8192, (128, 64)),
+                                        (400, 3584, 8192, (128, 64)), (129, 6144, 4096, (64, 128))])
+def test_measured_tile_choice(m, n, k, tile):
+    """Between the two tiles of 8192 outputs: the one that was faster with
+    distinct weights (128 x 64 but where it needs more tiles)."""
+    r = route(m, n, k)
+    assert (r["bm"], r["bn"]) == tile
+
+
 @pytest.mark.parametrize("tile,family,m,n,k", [c for c in TILES if c[4] % 128])
 def test_tail_reads_stay_inside(tile, family, m, n, k):
     """gemm_dma's DMA sources with a partial last stage (loadA, loadB): every
