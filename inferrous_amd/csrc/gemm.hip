@@ -1139,7 +1139,10 @@ __global__ __launch_bounds__(256) void splitk_epilogue8(GemmArgs a, const int32_
 // 64 x 128 costs more than 128 x 64 although it moves as much: with distinct
 // weights, BF16, 64 x 128 / 128 x 64, 4096 columns at M = 300, K = 4096 15.8 / 14.1
 // and K = 8192 28.2 / 24.8, 2560 x 8192 at M = 700 41.2 / 28.2, 3584 x 8192 at M =
-// 400 37.6 / 26.6.
+// 400 37.6 / 26.6, 6144 x 4096 at M = 129 14.7 / 14.4 and M = 180 16.7 / 14.6, 6144 x
+// 5120 at M = 160 21.7 / 17.6.  It leads where 128 x 64 needs twice the rounds
+// (10240 x 4096 at M = 129 17.2 / 19.2), and by little at the most tiles of one
+// round (8192 x 4096 at M = 129 15.5 / 16.4, M = 180 17.4 / 17.0).
 //
 // kTailTiles, K % 128 != 0: four waves.  gemm_tiled, the register-staged kernel
 // these replaced -> the tile the route takes: 4096 x 8000 x 5008 316 -> 168, 2000
@@ -1154,7 +1157,7 @@ static const DmaTile kDmaTiles[] = {
     {256, 256, 64, 128, 2, 3, 11000, 1700, 0}, {256, 192, 64, 96, 2, 3, 10000, 1270, 0},
     {256, 128, 64, 64, 2, 4, 7000, 940, 0},    {128, 192, 32, 96, 2, 4, 5000, 740, 0},
     {128, 128, 32, 64, 4, 4, 3000, 590, 0},    {128, 64, 32, 32, 4, 4, 2500, 440, 0},
-    {64, 128, 32, 32, 4, 4, 2500, 460, 0},     {64, 64, 32, 32, 4, 4, 3000, 280, 460},
+    {64, 128, 32, 32, 4, 4, 2500, 468, 0},     {64, 64, 32, 32, 4, 4, 3000, 280, 460},
 };
 static const DmaTile kTailTiles[] = {
     {256, 256, 128, 128, 2, 3, 11000, 1830, 0}, {256, 128, 128, 64, 2, 4, 7000, 1100, 0},

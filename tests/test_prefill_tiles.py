@@ -45,7 +45,7 @@ def test_lane_offsets_fit_32_bits():
 # (tile, family, m, n, k): eight waves (13), four waves (14), K tails of 16 and
 # 112 bytes, K below one stage
 TILES = [((128, 64), 13, 2049, 515, 1280), ((128, 128), 13, 1025, 2003, 1280), ((128, 192), 13, 1300, 3003, 1280),
-         ((256, 128), 13, 1025, 6003, 1280), ((256, 192), 13, 1300, 6003, 1280), ((64, 128), 13, 129, 6003, 1280),
+         ((256, 128), 13, 1025, 6003, 1280), ((256, 192), 13, 1300, 6003, 1280), ((64, 128), 13, 129, 10003, 1280),
          ((256, 256), 13, 2049, 6003, 1280), ((64, 64), 14, 150, 515, 1280), ((64, 64), 14, 17, 33, 16),
          ((64, 64), 14, 77, 1003, 112), ((64, 64), 14, 257, 515, 1392), ((128, 64), 14, 1025, 2003, 16),
          ((128, 128), 14, 1300, 3003, 144), ((256, 128), 14, 2049, 2003, 1296), ((256, 256), 14, 1300, 6003, 1296)]
@@ -58,7 +58,9 @@ def test_tile_routes(tile, family, m, n, k):
 
 
 @pytest.mark.parametrize("m,n,k,tile", [(300, 4096, 4096, (128, 64)), (700, 2560, 8192, (128, 64)),
-                                        (400, 3584, 8192, (128, 64)), (129, 6144, 4096, (64, 128))])
+                                        (400, 3584, 8192, (128, 64)), (129, 6144, 4096, (128, 64)),
+                                        (180, 6144, 4096, (128, 64)), (129, 8192, 4096, (64, 128)),
+                                        (129, 10240, 4096, (64, 128)), (320, 6144, 4096, (64, 128))])
 def test_measured_tile_choice(m, n, k, tile):
     """Between the two tiles of 8192 outputs: the one that was faster with
     distinct weights (128 x 64 but where it needs more tiles)."""
