@@ -455,7 +455,7 @@ __device__ __forceinline__ void store_blocks(const GemmArgs& a, const v16i (&acc
 // most panels once per tile: 24576 x 4096 at M = 4096, f32, 256 x 192 tiles
 // 484 -> 443 us; strips of 4 / 8 / 16 on 256 x 256 tiles 387 / 397 / 430.
 constexpr uint32_t kStrip = 4;
-// Rotated K (unsplit, K % 128 == 0): stage kt of tile t reads K chunk (kt + t)
+// Rotated K (unsplit, K % 128 == 0, eight waves): stage kt of tile t reads K chunk (kt + t)
 // mod KT, so that the workgroups do not all read the same 128-byte column of
 // their rows at once; the i32 sums are exact in any order.  It pays in a
 // launch of one round whose M tiles are few, and with one column of tiles,
@@ -513,10 +513,10 @@ __global__ __launch_bounds__(64 * NW, (waves_per_simd(NW, (SA * BM + SB * BN) * 
   const uint32_t K = a.k, KT = TAIL ? K / 128 + 1 : K / 128 / splits;
   const size_t kbase = (size_t)split * KT * 128;
   if (raw_i32(EP)) a.out = reinterpret_cast<int32_t*>(a.out) + (size_t)split * a.m * a.n;
-  const bool turned =
-      !TAIL && splits == 1 && T <= kRotateTiles && (tiles_n == 1 || (NW == 8 && a.m <= kRotateRows));
-  const uint32_t rot = turned ? Lt % KT : 0;
+  const bool turned = splits == 1 && T <= kRotateTiles && (tiles_n == 1 || a.m <= kRotateRows);
+  const uint32_t rot = !TAIL && NW == 8 && turned ? Lt % KT : 0;
   auto kc = [&](uint32_t kt) -> size_t {  // byte offset of stage kt
+    if constexpr (TAIL || NW != 8) return (size_t)kt * 128;
     const uint32_t c = kt + rot;
     return (size_t)(c >= KT ? c - KT : c) * 128;
   };
