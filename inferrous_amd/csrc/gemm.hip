@@ -455,19 +455,15 @@ __device__ __forceinline__ void store_blocks(const GemmArgs& a, const v16i (&acc
 // most panels once per tile: 24576 x 4096 at M = 4096, f32, 256 x 192 tiles
 // 484 -> 443 us; strips of 4 / 8 / 16 on 256 x 256 tiles 387 / 397 / 430.
 constexpr uint32_t kStrip = 4;
-// Rotated K (unsplit, K % 128 == 0, eight waves): stage kt of tile t reads K chunk (kt + t)
-// mod KT, so that the workgroups do not all read the same 128-byte column of
-// their rows at once; the i32 sums are exact in any order.  It pays in a
-// launch of one round whose M tiles are few, and with one column of tiles,
-// where every workgroup walks the same weights (K = 16384 puts all their rows
-// on one channel); with several strips it loses the panels that they share.
-// Distinct weights, BF16, in order -> rotated, us: 6144 x 4096 at M = 256 16.4
-// -> 16.1, M = 512 21.6 -> 21.1, 4096 x 4096 at M = 300 16.5 -> 15.9, M = 768
-// 21.3 -> 20.8, 64 x 16384 at M = 22,000 87 -> 69; not taken: 6144 x 4096 at M =
-// 2048 51.8 -> 56.8, 4096 x 4096 at M = 4096 66 -> 69, and on 64 x 64 tiles 4096 x
-// 4096 at M = 129 11.7 -> 11.8.
-constexpr uint32_t kRotateTiles = 256;  // one per CU
-constexpr uint32_t kRotateRows = 768;
+// Rotated K: in a launch of one round over one column of tiles (unsplit, K % 128
+// == 0, eight waves), stage kt of tile t reads K chunk (kt + t) mod KT; the i32 sums
+// are exact in any order.  Every workgroup walks the same weights there, and in
+// step all rows of a stage can lie on one memory channel: 64 x 16384 at M = 22,000
+// 87 -> 69 us.  With more columns the panels shared in step are worth as much:
+// rotated / in order with distinct weights, BF16, 6144 x 4096 at M = 129 14.9 /
+// 13.9, M = 256 16.2 / 16.6, M = 512 21.6 / 21.9, M = 2048 56.8 / 51.8; 6144 x 8192 at
+// M = 256 30.0 / 29.1, 6144 x 2048 10.1 / 10.0; 4096 x 4096 at M = 4096 69 / 66.
+constexpr uint64_t kCus = 256;
 constexpr uint32_t kMaxK = 1u << 23;  // 256 rows of K bytes stay within a 32-bit offset
 
 // TAIL (K % 128 != 0, any N): the last stage is partial.  A lane whose 16-byte
@@ -513,7 +509,7 @@ __global__ __launch_bounds__(64 * NW, (waves_per_simd(NW, (SA * BM + SB * BN) * 
   const uint32_t K = a.k, KT = TAIL ? K / 128 + 1 : K / 128 / splits;
   const size_t kbase = (size_t)split * KT * 128;
   if (raw_i32(EP)) a.out = reinterpret_cast<int32_t*>(a.out) + (size_t)split * a.m * a.n;
-  const bool turned = splits == 1 && T <= kRotateTiles && (tiles_n == 1 || a.m <= kRotateRows);
+  const bool turned = splits == 1 && tiles_n == 1 && T <= kCus;
   const uint32_t rot = !TAIL && NW == 8 && turned ? Lt % KT : 0;
   auto kc = [&](uint32_t kt) -> size_t {  // byte offset of stage kt
     if constexpr (TAIL || NW != 8) return (size_t)kt * 128;
@@ -1164,8 +1160,6 @@ static const DmaTile kTailTiles[] = {
     {128, 128, 64, 64, 2, 3, 5000, 620, 1340},  {128, 64, 64, 32, 3, 4, 4000, 420, 890},
     {64, 64, 32, 32, 4, 4, 3000, 280, 460},
 };
-constexpr uint64_t kCus = 256;
-
 static uint64_t launch_ns(const DmaTile& t, uint64_t tiles, uint64_t stages) {
   const uint64_t at_once = t.pair ? 2 * kCus : kCus, rest = tiles % at_once;
   const uint64_t full = t.fixed + stages * (t.pair ? t.pair : t.stage);

@@ -129,7 +129,7 @@ def test_every_tile(tile, family, m, n, k):
                                    (5000, 60, 1280), (22000, 60, 640), (33000, 61, 256), (300, 2003, 16384)])
 def test_rotated_k(m, n, k):
     """Both sides of gemm_dma's rule for starting each tile at its own K stage
-    (one round of tiles at up to 768 rows, or one column of tiles): the sums."""
+    (one round of tiles in one column): the sums."""
     from inferrous_amd import CudaContext, DeviceBuffer, load
     ctx = CudaContext(0)
     mod, s = load(ctx), ctx.new_stream()
