@@ -1278,22 +1278,32 @@ static bool tall_plan(uint32_t m, uint32_t n, uint32_t k, int& bn, uint32_t& spl
   return true;
 }
 
-// Whether one unsplit launch (64 x 64 or 64 x 128 tiles, gemm_dma) runs a shape of
-// gemm_tall's split plan faster than the split GEMM and its slab epilogue: above
-// 64 rows, up to a K that grows with the slabs (M N values).  Measured on
-// MI355X with residual, split / unsplit us, 4096 columns at K = 2048 / 4096 /
-// 5120 / 6144 / 8192: M = 65 9.3 / 10.9 / 12.0 / 12.7 / 14.3 against 7.7 / 11.5 /
-// 13.8 / 15.8 / 20.2, M = 129 11.6 / 13.3 / 14.7 / 15.3 / 17.5 against 8.1 / 11.7 /
-// 14.3 / 16.1 / 20.4, M = 200 13.6 / 15.3 / 17.4 / 18.1 / 20.2 against 8.2 / 11.9 /
-// 14.6 / 16.4 / 20.8, M = 256 14.2 / 16.7 / 19.0 / 19.5 / 22.4 against 8.5 / 12.6 /
-// 16.3 / 17.5 / 22.2; 6144 columns, M = 100 12.3 / 14.2 / 16.5 / 16.7 / 19.0 against
-// 8.1 / 12.7 / 16.0 / 17.4 / 21.6; 8192 columns, M = 129 19.8 / 25.2 / 28.3 / 30.4 /
-// 35.2 against 9.9 / 16.2 / 20.6 / 22.2 / 26.7.
+// Whether one unsplit launch of gemm_dma's small tiles runs a shape of gemm_tall's
+// split plan faster than the split GEMM and its slab epilogue: above 64 rows, up
+// to a K that grows with the rows and with the slabs.  Always where the split
+// grid takes a second round, and later where only two slabs divide K.
+// Measured on MI355X with distinct weights, BF16, split / unsplit us at K = 2048 /
+// 3072 / 4096 / 5120 / 8192:
+//   1024 cols, M = 65    7.2 /  7.6    8.0 /  9.7    8.9 / 11.7    9.9 / 13.8   12.2 / 19.9
+//              M = 129   8.3 /  7.6    9.5 /  9.6   10.3 / 11.7   11.5 / 13.8   14.2 / 19.9
+//              M = 256   9.4 /  7.7   10.7 /  9.9   11.4 / 11.9   13.5 / 15.0   16.2 / 20.5
+//   4096 cols, M = 65    7.9 /  7.8    8.8 /  9.9    9.6 / 12.0   10.7 / 14.4   13.1 / 20.7
+//              M = 100   8.6 /  7.8    9.7 / 10.1   10.4 / 12.2   12.5 / 15.3   14.2 / 21.1
+//              M = 129  10.0 /  7.8   11.2 /  9.9   12.1 / 12.0   13.4 / 14.4   16.4 / 20.7
+//              M = 193  10.9 /  7.8   12.6 / 10.0   13.7 / 12.1   15.4 / 14.6   18.9 / 21.2
+//              M = 256  13.2 /  8.0   14.7 / 10.4   16.2 / 12.5   17.9 / 16.1   22.2 / 21.8
+//   6144 cols, M = 129  11.3 /  9.3   13.4 / 12.4   14.6 / 14.5   16.3 / 17.3   20.6 / 25.2
+//              M = 256  17.2 / 10.1   19.6 / 13.9   21.5 / 16.2   23.1 / 22.4   28.6 / 29.9
+//   8192 cols, M = 129  17.6 /  9.6   20.9 / 12.7   23.2 / 15.5   26.3 / 20.1   33.3 / 26.6
+// Two slabs, unsplit over split at K = 4352 / 5376 / 7936: M = 65 0.95-0.99 / 0.99-1.02 /
+// 1.04-1.06, M = 129 0.83-0.87 / 0.84-0.89 / 0.90-0.92 (1024 to 4096 columns).
 bool gemm_unsplit_leads(uint32_t m, uint32_t n, uint32_t k) {
   int bn, ma;
   uint32_t splits;
-  if (m <= 64 || !tall_plan(m, n, k, bn, splits, ma) || splits == 1) return false;
-  return k <= std::min<uint64_t>(std::max<uint64_t>((uint64_t)m * n / 104, 3584), 8192);
+  if (m <= 64 || k > 8192 || !tall_plan(m, n, k, bn, splits, ma) || splits == 1) return false;
+  if ((n + bn - 1) / bn * splits > kCus) return true;
+  if (splits == 2) return m > 100 || k <= 5376;
+  return 2000 * k <= 27000 * m + 9 * m * std::min(n, 4096u);
 }
 
 size_t gemm_workspace_bytes(uint32_t m, uint32_t n, uint32_t k) {

@@ -561,6 +561,18 @@ def test_workspace_queries_by_route_and_batch_range():
     assert L.w8a8_linear_workspace_bytes_upto(0, *down) == 0
 
 
+@pytest.mark.parametrize("m,n,k,split", [
+    (65, 1024, 2048, True), (100, 1024, 3072, True), (129, 1024, 2048, False), (256, 1024, 5120, True),
+    (65, 4096, 3072, True), (129, 4096, 4096, False), (129, 4096, 5120, True), (193, 4096, 6144, False),
+    (129, 6144, 4096, False), (129, 6144, 5120, True), (160, 6144, 8192, True), (256, 6144, 6144, False),
+    (129, 5120, 8192, False), (65, 8192, 8192, False), (129, 4096, 8704, True),
+    (129, 4096, 7936, False), (65, 1024, 6400, True), (64, 4096, 8192, True), (129, 24576, 4096, False)])
+def test_auto_splits_where_measured_faster(m, n, k, split):
+    """Above 64 rows AUTO sizes a workspace only where the split pair was the
+    faster one with distinct weights."""
+    assert (_lib.lib().w8a8_linear_workspace_bytes_path(m, n, k, _lib.PATH_AUTO) > 0) == split
+
+
 @pytest.mark.skipif(no_device_status() > 0, reason="validation-order test assumes no GPU")
 def test_sequence_prepare_validation_precedes_device():
     """w8a8_linear_sequence_prepare checks every entry on the host before
