@@ -200,6 +200,8 @@ int w8a8_linear_path(void *stream, const int8_t *q, const float *asc, size_t m,
  * With a workspace of at least w8a8_linear_workspace_bytes(m, n, k) bytes
  * (16-byte aligned), shapes that gain from it are computed split-K: i32
  * partial sums in the workspace, added exactly by an epilogue kernel.
+ * W8A8_PATH_AUTO uses it only where the split launches are faster than one
+ * without; W8A8_PATH_MFMA wherever the shape's plan splits K.
  * Results are identical with or without the workspace; a smaller or NULL
  * workspace selects the unsplit kernels.  Calls sharing one workspace must
  * not overlap. */
@@ -208,8 +210,7 @@ size_t w8a8_linear_workspace_bytes(size_t m, size_t n, uint32_t k);
  * where AUTO runs the dot4 GEMV whatever the workspace (m = 1, and m = 2
  * unless the MFMA route there is the narrow kernel or the unsplit one-M-tile
  * kernel, which need none) or where one unsplit launch is faster than the split
- * pair (above 64 rows at short K; a call that gives a workspace all the same
- * takes the split kernels); the MFMA family's need otherwise.  Size a per-call
+ * pair (above 64 rows at short K); the MFMA family's need otherwise.  Size a per-call
  * workspace with this. */
 size_t w8a8_linear_workspace_bytes_path(size_t m, size_t n, uint32_t k, int path);
 /* The largest w8a8_linear_workspace_bytes(m, n, k) over m = 1 .. max_m.

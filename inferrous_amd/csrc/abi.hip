@@ -99,12 +99,20 @@ static int auto_path(size_t m, size_t n, uint32_t k, size_t workspace_bytes) {
   return W8A8_PATH_MFMA;
 }
 
+// The workspace bytes a call's GEMM may use: AUTO leaves the split plan where one
+// launch without it is faster, whatever the caller holds (one buffer for
+// every batch size, w8a8_linear_workspace_bytes_upto); MFMA takes what it gets.
+static size_t usable_workspace(int path, size_t m, size_t n, uint32_t k, size_t bytes) {
+  return path == W8A8_PATH_AUTO && gemm_unsplit_leads((uint32_t)m, (uint32_t)n, k) ? 0 : bytes;
+}
+
 int run_linear(hipStream_t st, const int8_t* q, const float* asc, size_t m, const int8_t* w,
                const float* ws, size_t n, uint32_t k, void* out, int out_dtype, int path,
                const float* residual, void* combined, void* workspace = nullptr,
                size_t workspace_bytes = 0) {
   if (m == 0 || n == 0) return W8A8_OK;
-  if (path == W8A8_PATH_AUTO) path = auto_path(m, n, k, workspace ? workspace_bytes : 0);
+  workspace_bytes = usable_workspace(path, m, n, k, workspace ? workspace_bytes : 0);
+  if (path == W8A8_PATH_AUTO) path = auto_path(m, n, k, workspace_bytes);
   if (path == W8A8_PATH_DOT4) {
     GemvArgs a{};
     a.q = q;
@@ -133,8 +141,8 @@ int run_linear(hipStream_t st, const int8_t* q, const float* asc, size_t m, cons
   g.out_dtype = out_dtype;
   g.residual = residual;
   g.combined = combined;
-  g.partials = static_cast<int32_t*>(workspace);
-  g.partial_bytes = workspace ? workspace_bytes : 0;
+  g.partials = workspace_bytes ? static_cast<int32_t*>(workspace) : nullptr;
+  g.partial_bytes = workspace_bytes;
   return hip_status(launch_gemm(st, g));
 }
 
@@ -1050,6 +1058,7 @@ int w8a8_diag_linear_route(size_t m, size_t n, uint32_t k, int out_dtype, int re
   if (residual && out_dtype == W8A8_OUT_I32) return W8A8_EARG;
   put_route(route, kRouteNone, 0, 0, 0);
   if (m == 0 || n == 0) return W8A8_OK;
+  workspace_bytes = usable_workspace(path, m, n, k, workspace_bytes);
   if (path == W8A8_PATH_AUTO) path = auto_path(m, n, k, workspace_bytes);
   if (path == W8A8_PATH_DOT4) {
     const uint32_t nn = (uint32_t)n;

@@ -1196,8 +1196,9 @@ static bool staged_shape(uint32_t n, uint32_t k) { return k % 128 == 0 && k <= k
 // for a long K (4096 x 12288 at M = 512: 36 + 8 us for the slab epilogue
 // against 58 unsplit and 44.7 on 128 x 64 tiles).  With more tiles the
 // slabs cost more than the CUs they fill: at M = 4096 288 + 64 us against 196
-// on 256 x 256 tiles.  A single column of tiles (N <= 128) keeps the plan at any
-// M.  gemm_tall's plan covers M <= 256.
+// on 256 x 256 tiles.  A single column of tiles (N <= 128) has the plan at any M for
+// calls that ask for it (W8A8_PATH_MFMA with a workspace); AUTO leaves it there
+// too (gemm_unsplit_leads).  gemm_tall's plan covers M <= 256.
 static bool split_plan(uint32_t m, uint32_t n, uint32_t k, uint32_t& splits) {
   if (m <= 256 || k < 8192 || !staged_shape(n, k) || n % 4 != 0) return false;
   const uint32_t kt = k / 128;
@@ -1297,9 +1298,12 @@ static bool tall_plan(uint32_t m, uint32_t n, uint32_t k, int& bn, uint32_t& spl
 //   8192 cols, M = 129  17.6 /  9.6   20.9 / 12.7   23.2 / 15.5   26.3 / 20.1   33.3 / 26.6
 // Two slabs, unsplit over split at K = 4352 / 5376 / 7936: M = 65 0.95-0.99 / 0.99-1.02 /
 // 1.04-1.06, M = 129 0.83-0.87 / 0.84-0.89 / 0.90-0.92 (1024 to 4096 columns).
+// Above 256 rows: split_plan's single column of tiles past its share of the CUs (64
+// columns, M = 22,000 / 33,000, K = 8192 48 / 83 split, 27 / 57 unsplit).
 bool gemm_unsplit_leads(uint32_t m, uint32_t n, uint32_t k) {
   int bn, ma;
   uint32_t splits;
+  if (m > 256) return split_plan(m, n, k, splits) && (uint64_t)((m + 127) / 128) * 3 > kCus * 2 && n <= 128;
   if (m <= 64 || k > 8192 || !tall_plan(m, n, k, bn, splits, ma) || splits == 1) return false;
   if ((n + bn - 1) / bn * splits > kCus) return true;
   if (splits == 2) return m > 100 || k <= 5376;

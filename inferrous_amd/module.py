@@ -181,7 +181,9 @@ class LoadedModule:
                 self._retired.append(cur)
             self._gemm_ws[_key(stream)] = DeviceBuffer((nbytes + 15) // 16 * 16, np.uint8)
 
-    def _workspace_for(self, stream, m: int, n: int, k: int, path: int):
+    def _workspace_for(self, stream, m: int, n: int, k: int, path: int, split: bool = False):
+        if path == _lib.PATH_MFMA and m > 4 and not split:
+            path = _lib.PATH_AUTO   # the MFMA family too, split only where that is faster
         need = lib().w8a8_linear_workspace_bytes_path(m, n, k, path)
         if not need:
             return None, 0   # none used, or faster without
@@ -192,11 +194,12 @@ class LoadedModule:
         ws = self._gemm_ws.get(_key(stream))
         return (ws.ptr, ws.nbytes) if ws is not None else (None, 0)
 
-    def _linear(self, stream, q, asc, w, ws, width, out, path, residual=None, combined=None) -> None:
+    def _linear(self, stream, q, asc, w, ws, width, out, path, residual=None, combined=None,
+                split: bool = False) -> None:
         m, n, k = _shape(asc, ws, out, width)
         if len(q) < m * k or len(w) < n * k:
             raise ValueError("q or w shorter than M*K / N*K")
-        wp, wb = self._workspace_for(stream, m, n, k, path)
+        wp, wb = self._workspace_for(stream, m, n, k, path, split)
         check(lib().w8a8_linear_ex(_h(stream), q.ptr, asc.ptr, m, w.ptr, ws.ptr, n, k,
                                    None if residual is None else residual.ptr, out.ptr,
                                    None if combined is None else combined.ptr, _dtype_code(out), path,
@@ -221,7 +224,8 @@ class LoadedModule:
         self._linear(stream, q, asc, w, ws, width, out, _lib.PATH_MFMA)
 
     def linear_splitk(self, stream, config, q, asc, w, ws, width, out) -> None:
-        self._linear(stream, q, asc, w, ws, width, out, _lib.PATH_MFMA)
+        """Split K wherever the shape's plan does, also where one launch is faster."""
+        self._linear(stream, q, asc, w, ws, width, out, _lib.PATH_MFMA, split=True)
 
     def linear_tiled(self, stream, config, q, asc, w, ws, width, out) -> None:
         self._linear(stream, q, asc, w, ws, width, out, _lib.PATH_MFMA)

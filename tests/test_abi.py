@@ -117,7 +117,7 @@ def test_diag_gemm_timeline_stamp_count():
     route = np.zeros(20, np.int32)
     for (m, n, k) in [(129, 4096, 4096), (129, 24576, 4096), (24, 4096, 12288), (200, 6100, 4096)]:
         wsb = L.w8a8_linear_workspace_bytes(m, n, k)
-        assert L.w8a8_diag_linear_route(m, n, k, _lib.OUT_BF16, 0, 0, wsb, route.ctypes.data, 20) == 0
+        assert L.w8a8_diag_linear_route(m, n, k, _lib.OUT_BF16, 0, _lib.PATH_MFMA, wsb, route.ctypes.data, 20) == 0
         assert route[0] == 12
         assert L.w8a8_diag_gemm_timeline_stamps(m, n, k, wsb) == 4 * 8 * route[1]
     assert L.w8a8_diag_gemm_timeline_stamps(512, 4096, 4096, 0) == 0      # gemm_dma

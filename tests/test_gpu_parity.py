@@ -683,8 +683,9 @@ def test_linear_split_k_workspace_identical(env, m, n, k, dtype, res):
     equals the call without one and the oracle, bit for bit -- also on a
     second call with the same workspace, which carries nothing between calls.
     Up to M = 16 the narrow kernel takes every K it can split over its waves;
-    K >= 8192 with K % 1024 != 0 still splits there (3 x 4100 x 8448 under
-    AUTO's MFMA route from M = 3, 7 x 1024 x 8448).
+    K >= 8192 with K % 1024 != 0 still splits there (3 x 4100 x 8448, 7 x 1024
+    x 8448).  W8A8_PATH_MFMA, which splits whenever the plan does; AUTO takes
+    one launch for some of these shapes.
     The shapes cover both slab policies with the 16-byte epilogue (M > 200,
     N % 8 == 0) and the 4-column one: streamed (gemm_tall from 3 MiB of
     slabs: 129 x 4096 x 4096 and 64 x 4100 x 12288 on 4 columns, 255 x 4096
@@ -715,7 +716,7 @@ def test_linear_split_k_workspace_identical(env, m, n, k, dtype, res):
         comb = DeviceBuffer.zeroed(s, m * n, dtype) if res else None
         _lib.check(lib.w8a8_linear_ex(s.handle, dq.ptr, da.ptr, m, dw.ptr, dws.ptr, n, k,
                                       dres.ptr if res else None, out.ptr,
-                                      comb.ptr if res else None, dt, _lib.PATH_AUTO, wp, wb))
+                                      comb.ptr if res else None, dt, _lib.PATH_MFMA, wp, wb))
         outs.append((out.to_host_vec(s), comb.to_host_vec(s) if res else None))
     for o, c in outs[1:]:
         assert np.array_equal(o.view(np.uint8), outs[0][0].view(np.uint8))
@@ -755,7 +756,7 @@ def test_split_k_workspace_shared_by_shapes(env):
         dq, da, dw, dws = dev(s, q), dev(s, asc), dev(s, w), dev(s, ws)
         out = DeviceBuffer.zeroed(s, m * n, np.uint16)
         _lib.check(lib.w8a8_linear_ex(s.handle, dq.ptr, da.ptr, m, dw.ptr, dws.ptr, n, k, None, out.ptr, None,
-                                      _lib.OUT_BF16, _lib.PATH_AUTO, work.ptr, need))
+                                      _lib.OUT_BF16, _lib.PATH_MFMA, work.ptr, need))
         _, _, ob = oracle.linear(q, asc, w, ws, k, threads=8)
         assert np.array_equal(out.to_host_vec(s), ob), f"call {i}"
 
@@ -793,7 +794,7 @@ def test_large_row_counts_beyond_grid_y(env):
     # named, so that no buffer is freed before the kernels that read it ran
     dq, da, dw, dws, dres = dev(s, qa), dev(s, asc), dev(s, w), dev(s, ws), dev(s, resid)
     _lib.check(lib.w8a8_linear_ex(s.handle, dq.ptr, da.ptr, m, dw.ptr, dws.ptr, n, k, dres.ptr, out.ptr,
-                                  comb.ptr, _lib.OUT_BF16, _lib.PATH_AUTO, work.ptr, need))
+                                  comb.ptr, _lib.OUT_BF16, _lib.PATH_MFMA, work.ptr, need))
     assert np.array_equal(out.to_host_vec(s), ob)
     assert np.array_equal(comb.to_host_vec(s), (bits(oracle.residual(resid, of)) >> 16).astype(np.uint16))
 

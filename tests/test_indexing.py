@@ -506,9 +506,10 @@ def test_lm_head_argmax():
 def test_prefill_shapes(m, n, k):
     """C4: M = 129 and 512 on the four layer shapes, with and without the
     split-K workspace, plain and with a residual."""
-    for ws in (0, workspace_bytes(m, n, k)):
-        for residual in (False, True):
-            check_linear(m, n, k, residual=residual, workspace=ws)
+    for path in (AUTO, MFMA):
+        for ws in (0, workspace_bytes(m, n, k)):
+            for residual in (False, True):
+                check_linear(m, n, k, residual=residual, path=path, workspace=ws)
 
 
 @pytest.mark.parametrize("m", [130, 131, 135, 136, 140, 159])
@@ -516,7 +517,7 @@ def test_prefill_shapes(m, n, k):
 def test_m129_tails(m, n, k):
     """The rows past a 32-row block and past the 128-row tile: M = 129-135
     and 136-159 (sampled)."""
-    check_linear(m, n, k, workspace=workspace_bytes(m, n, k))
+    check_linear(m, n, k, path=MFMA, workspace=workspace_bytes(m, n, k))
     check_linear(m, n, k, residual=True)
 
 
@@ -536,6 +537,7 @@ def test_other_m_and_n_not_multiple_of_96(m):
     for n, k in [(4000, 4096), (6100, 4096), (24500, 4096), (1000, 12288), (4100, 4096)]:
         for ws in (0, workspace_bytes(m, n, k)):
             check_linear(m, n, k, workspace=ws)
+        check_linear(m, n, k, path=MFMA, workspace=workspace_bytes(m, n, k))
         check_linear(m, n, k, residual=True)
 
 
@@ -578,11 +580,21 @@ def test_seeded_shape_sweep(m, n, k):
     check_linear(m, n, k, I32, path=MFMA, workspace=wsb)
 
 
+@pytest.mark.parametrize("m,n,k", [(129, 8192, 4096), (256, 4096, 4096), (193, 6144, 2048), (33000, 64, 8192)])
+def test_auto_ignores_a_workspace_that_only_slows_it(m, n, k):
+    """The launch follows the shape, not the pointer: with a workspace for the
+    split plan AUTO runs the same route as without one, and MFMA splits."""
+    ws = workspace_bytes(m, n, k)
+    assert ws > 0
+    assert route(m, n, k, workspace=ws) == route(m, n, k) and route(m, n, k)["splits"] == 1
+    assert route(m, n, k, path=MFMA, workspace=ws)["splits"] > 1
+
+
 def test_every_family_is_replayed():
     """The shapes above reach every GEMM and GEMV family."""
     seen = set()
     for (m, n, k, ws) in [(1, 4096, 4096, 0), (1, 4096, 1040, 0), (3, 4096, 4096, 0), (3, 4096, 1040, 0),
-                          (129, 4096, 4096, 1 << 30), (512, 24576, 4096, 0), (100, 4096, 4112, 0)]:
+                          (129, 4096, 12288, 1 << 30), (512, 24576, 4096, 0), (100, 4096, 4112, 0)]:
         seen.add(route(m, n, k, workspace=ws)["family"])
     seen.add(argmax_route(4096, 4096)["family"])
     assert seen == {1, 2, 3, 11, 12, 13, 14, 15}, seen
@@ -646,7 +658,7 @@ def test_checker_catches_planted_mistakes():
     read without its clamp, a store written twice or not at all, a slot
     mapping off by one."""
     m, n, k = 129, 4096, 4096
-    r = route(m, n, k, workspace=workspace_bytes(m, n, k))
+    r = route(m, n, k, path=MFMA, workspace=workspace_bytes(m, n, k))
     assert r["family"] == 12  # gemm_tall, 160-row tile, split K
     lane = np.arange(64)
     row = 8 * (0 + 8 * 2) + (lane >> 3)  # wave 0's third activation row group: rows 128-135
