@@ -18,7 +18,7 @@
 //     16 x i32 result of lane l holds rows 8*(v/4)+4*(l/32)+v%4, column l%32.
 //
 // Kernels:
-//  * gemm_dma: the prefill GEMM, and every shape above 16 rows that no plan
+//  * gemm_dma: the prefill GEMM, and every shape above 16 rows that no kernel
 //    below takes; built on v_mfma_i32_32x32x32_i8 (on gfx950 the 16x16x64 int8
 //    form issues at half its rate), eight waves per workgroup (two per SIMD,
 //    so one wave's LDS reads overlap the other's MFMAs; four on the 64 x 64
@@ -45,9 +45,9 @@
 //    loop has no workgroup barrier and no split-K slabs leave the CU.  The S
 //    partial 16 x 16 tiles are summed through LDS (exact) and stored by the
 //    fused epilogue.
-//  * gemm_skinny (M <= 16 where gemm_narrow and gemm_tall do not run: k not in
-//    their stages, or a split-K plan without a workspace; HBM-bound, 16x16x64
-//    MFMA): one workgroup owns 16 weight rows; its S waves split K and stream
+//  * gemm_skinny (M <= 16, and up to 64 on narrow n, where gemm_narrow and
+//    gemm_tall do not run: k not in their stages, or a split-K plan without a
+//    workspace; HBM-bound, 16x16x64 MFMA): one workgroup owns 16 weight rows; its S waves split K and stream
 //    their weight fragments straight from HBM into MFMA B operands (no LDS
 //    round trip), activation fragments come from L1/L2.  Partial i32 tiles
 //    are summed through LDS -- exact.
@@ -1451,6 +1451,24 @@ static hipError_t launch_tall_timed(hipStream_t st, const GemmArgs& a, uint32_t 
 
 // ---------------------------------------------------------------- dispatch
 // The route of one GEMM call (see GemmRoute).
+// Where no plan runs, whether gemm_skinny's K split over a workgroup's waves beats
+// gemm_dma's small tiles, which walk K in one piece: always up to 16 rows; with up to
+// one 16-column workgroup per CU to 32 rows, and to 64 with a K tail (whose rows
+// cross cache lines, which costs the DMA more) or a short K; with twice the
+// columns at the shortest K.  Measured on MI355X with distinct weights, BF16, M x N x
+// K, gemm_skinny / gemm_dma us: 17 x 1024 x 8208 16.4 / 21.3, 32 x 512 x 16016 37 / 44,
+// 32 x 4096 x 8192 15.8 / 20.6, 33 x 4096 x 2064 8.5 / 8.8, 48 x 1024 x 4112 13.4 / 16.1,
+// 64 x 1024 x 12304 41 / 50, 64 x 4096 x 16016 57 / 66, 48 x 4096 x 384 3.8 / 5.1, 64 x 4096 x
+// 384 4.2 / 5.0, 24 x 6144 x 1040 6.2 / 6.2, 32 x 8192 x 528 4.5 / 4.9, 48 x 6144 x 384 4.6 /
+// 5.2; not taken: 33 x 1024 x 8192 23.3 / 19.8, 64 x 4096 x 16384 43.8 / 39.0, 48 x 4096 x
+// 1152 6.5 / 6.1, 64 x 4096 x 640 5.4 / 5.0, 32 x 6144 x 8192 28 / 21, 32 x 6144 x 1040 6.9 / 6.3.
+static bool skinny_leads(uint32_t m, uint32_t n, uint32_t k) {
+  if (m <= 16) return true;
+  if (m > 64 || n > 32 * kCus) return false;
+  if (n <= 16 * kCus) return m <= 32 || k % 128 != 0 || k <= (m <= 48 ? 896u : 384u);
+  return k <= (m <= 24 ? 1040u : m <= 32 ? 640u : m <= 48 ? 384u : 0u);
+}
+
 GemmRoute gemm_route(const GemmArgs& a) {
   GemmRoute r{};
   r.splits = 1;
@@ -1512,11 +1530,11 @@ GemmRoute gemm_route(const GemmArgs& a) {
       return r;
     }
   }
-  if (a.m <= 16 && !wide) {
+  if (!wide && skinny_leads(a.m, a.n, a.k)) {
     r.family = kRouteSkinny;
-    r.mt = 1;
+    r.mt = a.m <= 16 ? 1 : a.m <= 32 ? 2 : 4;
     r.s = 4;
-    r.u = 4;
+    r.u = a.m <= 32 ? 4 : 2;
     r.grid_x = (a.n + 15) / 16;
     r.block = 64 * r.s;
     return r;
@@ -1615,7 +1633,9 @@ hipError_t launch_gemm(hipStream_t st, const GemmArgs& a) {
     case kRouteNarrow:
       return launch_narrow<1>(st, a, NoGroup{}, r);
     case kRouteSkinny:
-      hipLaunchKernelGGL((gemm_skinny<1, 4, 4>), dim3(r.grid_x, 1), dim3(r.block), 0, st, a);
+      if (r.mt == 1) hipLaunchKernelGGL((gemm_skinny<1, 4, 4>), dim3(r.grid_x, 1), dim3(r.block), 0, st, a);
+      else if (r.mt == 2) hipLaunchKernelGGL((gemm_skinny<2, 4, 4>), dim3(r.grid_x, 1), dim3(r.block), 0, st, a);
+      else hipLaunchKernelGGL((gemm_skinny<4, 4, 2>), dim3(r.grid_x, 1), dim3(r.block), 0, st, a);
       return hipGetLastError();
     case kRouteDma:
       if (r.splits > 1) return launch_split<128, 128, 32, 64, 4, 4>(st, a, r.splits);

@@ -985,3 +985,30 @@ def test_linear_split_k_graph_replay(env):
         g.launch()
         s.synchronize()
         assert np.array_equal(bits(out.to_host_vec(s)), bits(want)), f"replay {rep}"
+
+
+@pytest.mark.parametrize("m", [16, 17, 31, 32, 33, 48, 63, 64])
+@pytest.mark.parametrize("n,k", [(64, 16), (333, 528), (1000, 4112), (4096, 1040), (17, 8208), (600, 4224)])
+def test_skinny_row_blocks(env, m, n, k):
+    """gemm_skinny at every count of 16-row blocks (one, two and four), K
+    below and past a wave's share, rows and columns that do not fill the last
+    block, guard values past the output untouched (33 to 64 rows of a K of
+    whole stages run gemm_dma's small tiles)."""
+    ctx, mod, s = env
+    print(f"skinny m={m} n={n} k={k}", flush=True)
+    rng = np.random.default_rng(m * 13 + n)
+    q = rng.integers(-127, 128, (m, k), dtype=np.int8)
+    w = rng.integers(-127, 128, (n, k), dtype=np.int8)
+    asc, ws = (rng.random(m) / 64).astype(F32), (rng.random(n) / 64).astype(F32)
+    res = oracle.bf16_rne(rng.standard_normal(m * n).astype(F32))
+    acc, of, ob = oracle.linear(q, asc, w, ws, k, threads=8)
+    dq, da, dw, dws, dres = dev(s, q), dev(s, asc), dev(s, w), dev(s, ws), dev(s, res)
+    out = dev(s, np.full(m * n + 64, 7, np.uint16))
+    mod.linear_mfma(s, None, dq, da, dw, dws, k, DeviceBuffer.view_of(out, 0, m * n))
+    got = out.to_host_vec(s)
+    assert np.array_equal(got[:m * n], ob) and (got[m * n:] == 7).all()
+    f, c = DeviceBuffer.zeroed(s, m * n, np.float32), dev(s, np.full(m * n + 64, 7, F32))
+    mod.linear_residual(s, None, dq, da, dw, dws, k, dres, f, DeviceBuffer.view_of(c, 0, m * n))
+    assert np.array_equal(bits(f.to_host_vec(s)), bits(of))
+    got = c.to_host_vec(s)
+    assert np.array_equal(bits(got[:m * n]), bits(oracle.residual(res, of))) and (got[m * n:] == 7).all()

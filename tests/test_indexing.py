@@ -580,6 +580,18 @@ def test_seeded_shape_sweep(m, n, k):
     check_linear(m, n, k, I32, path=MFMA, workspace=wsb)
 
 
+@pytest.mark.parametrize("m,n,k,skinny", [
+    (17, 1024, 8192, True), (32, 512, 16000, True), (32, 4096, 8192, True), (32, 4100, 8192, False),
+    (33, 1024, 8192, False), (64, 1024, 12304, True), (64, 4096, 2064, True), (64, 4100, 2064, False),
+    (65, 1024, 12304, False), (24, 8192, 1040, True), (25, 8192, 1040, False), (32, 8192, 528, True),
+    (24, 8208, 528, False), (33, 8192, 528, False), (48, 8192, 384, True), (49, 8192, 384, False),
+    (48, 4096, 896, True), (48, 4096, 1152, False), (64, 4096, 384, True), (64, 4096, 640, False)])
+def test_k_split_over_waves_on_narrow_n(m, n, k, skinny):
+    """Where no plan runs (K tails, no workspace): gemm_skinny up to one
+    workgroup per CU, gemm_dma's small tiles beyond."""
+    assert (check_linear(m, n, k, path=MFMA)["family"] == 11) == skinny
+
+
 @pytest.mark.parametrize("m,n,k", [(129, 8192, 4096), (256, 4096, 4096), (193, 6144, 2048), (33000, 64, 8192)])
 def test_auto_ignores_a_workspace_that_only_slows_it(m, n, k):
     """The launch follows the shape, not the pointer: with a workspace for the

@@ -46,7 +46,7 @@ def test_lane_offsets_fit_32_bits():
 # 112 bytes, K below one stage
 TILES = [((128, 64), 13, 2049, 515, 1280), ((128, 128), 13, 1025, 2003, 1280), ((128, 192), 13, 1300, 3003, 1280),
          ((256, 128), 13, 1025, 6003, 1280), ((256, 192), 13, 1300, 6003, 1280), ((64, 128), 13, 129, 10003, 1280),
-         ((256, 256), 13, 2049, 6003, 1280), ((64, 64), 14, 150, 515, 1280), ((64, 64), 14, 17, 33, 16),
+         ((256, 256), 13, 2049, 6003, 1280), ((64, 64), 14, 150, 515, 1280), ((64, 64), 14, 65, 33, 16),
          ((64, 64), 14, 77, 1003, 112), ((64, 64), 14, 257, 515, 1392), ((128, 64), 14, 1025, 2003, 16),
          ((128, 128), 14, 1300, 3003, 144), ((256, 128), 14, 2049, 2003, 1296), ((256, 256), 14, 1300, 6003, 1296)]
 
