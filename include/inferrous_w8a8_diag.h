@@ -67,7 +67,7 @@ int w8a8_diag_gemm_timeline(void *stream, const int8_t *q, const float *asc,
  *   [0] family: 0 none (m or n is 0), 1 gemv_m1_one, 2 gemv_m1, 3 gemv_mt,
  *       11 gemm_skinny, 12 gemm_tall, 13 gemm_dma, 14 gemm_dma with four waves, 15 gemm_narrow
  *   [1] grid x  [2] grid y  [3] threads per workgroup
- *   [4] BM  [5] BN  [6] WM  [7] WN  [8] SA (gemm_narrow: ring stages)  [9] SB
+ *   [4] BM  [5] BN (grouped: also of gemm_narrow)  [6] WM  [7] WN  [8] SA (gemm_narrow: ring stages)  [9] SB
  *   [10] MA (gemm_tall's M tile)
  *   [11] MT (skinny, narrow: 16-row tiles; gemv_mt: activation rows per pass)
  *   [12] S (skinny, narrow: waves)  [13] U (skinny: unroll; narrow: live
@@ -91,6 +91,13 @@ int w8a8_diag_linear_route(size_t m, size_t n, uint32_t k, int out_dtype,
  * selection's finalize launch follows it). */
 int w8a8_diag_argmax_route(size_t n, uint32_t k, int32_t *route,
                            size_t route_len);
+
+/* The route of w8a8_linear_grouped for m rows and count (1..4) matrices of n[i]
+ * columns (host array; empty ones are left out): [5] is the GEMM's columns per
+ * tile, matrix i's tiles following matrix i - 1's; family 3 (or 2, m = 1) is
+ * the one dot4 launch, 0 one launch per matrix. */
+int w8a8_diag_grouped_route(size_t m, uint32_t k, int count, const size_t *n,
+                            int32_t *route, size_t route_len);
 
 #ifdef __cplusplus
 }

@@ -118,6 +118,7 @@ DIAG_SIGNATURES: dict[str, tuple] = {
     "w8a8_diag_gemm_timeline_stamps": (S, [S, S, U32, S]),
     "w8a8_diag_gemm_timeline": (I, [P, P, P, S, P, P, S, U32, P, P, S, P, S]),
     "w8a8_diag_argmax_route": (I, [S, U32, P, S]),
+    "w8a8_diag_grouped_route": (I, [S, U32, I, P, P, S]),
 }
 
 

@@ -147,6 +147,14 @@ int run_linear(hipStream_t st, const int8_t* q, const float* asc, size_t m, cons
 }
 
 
+// The GEMM launch of a grouped call (family none: one dot4 launch up to kDot4MaxM
+// rows, one launch per matrix above).
+static GemmRoute grouped_gemm(size_t m, uint32_t k, const GemmGroup& g) {
+  if (m <= 1) return GemmRoute{};
+  const GemmRoute r = gemm_group_route((uint32_t)m, k, g.n, g.count);
+  return m > kDot4MaxM || r.family == kRouteNarrow || r.bn == 96 ? r : GemmRoute{};
+}
+
 int check_argmax(const int8_t* q, const float* asc, const int8_t* w, const float* ws, size_t n,
                  uint32_t k, const uint32_t* token, const void* logits, int logits_dtype) {
   if (logits && logits_dtype != W8A8_OUT_F32 && logits_dtype != W8A8_OUT_BF16) return W8A8_EARG;
@@ -619,9 +627,7 @@ int w8a8_linear_grouped(void* stream, const int8_t* q, const float* asc, size_t 
     g.n[g.count++] = (uint32_t)n[i];
   }
   if (g.count == 0) return W8A8_OK;
-  const GemmRoute r = m > 1 ? gemm_group_route((uint32_t)m, k, g.n, g.count) : GemmRoute{};
-  const bool gemm = r.family != kRouteNone && (m > kDot4MaxM || r.family == kRouteNarrow || r.bn == 96);
-  if (gemm) {
+  if (grouped_gemm(m, k, g).family != kRouteNone) {
     GemmArgs a{};
     a.q = q;
     a.asc = asc;
@@ -1048,6 +1054,23 @@ static void put_gemv_route(int32_t* r, const GemvRoute& g) {
   r[19] = g.waves;
 }
 
+static void put_gemm_route(int32_t* r, const GemmRoute& g) {
+  put_route(r, g.family, g.grid_x, g.grid_y, g.block);
+  r[4] = g.bm;
+  r[5] = g.bn;
+  r[6] = g.wm;
+  r[7] = g.wn;
+  r[8] = g.sa;
+  r[9] = g.sb;
+  r[10] = g.ma;
+  r[11] = g.mt;
+  r[12] = g.s;
+  r[13] = g.u;
+  r[14] = (int32_t)g.splits;
+  r[15] = g.nt_slabs;
+  r[16] = g.epi_cols;
+}
+
 int w8a8_diag_linear_route(size_t m, size_t n, uint32_t k, int out_dtype, int residual, int path,
                            size_t workspace_bytes, int32_t* route, size_t route_len) {
   if (!route) return W8A8_ENULL;
@@ -1076,21 +1099,7 @@ int w8a8_diag_linear_route(size_t m, size_t n, uint32_t k, int out_dtype, int re
   a.residual = residual ? kDummy : nullptr;
   a.partials = workspace_bytes ? (int32_t*)kDummy : nullptr;
   a.partial_bytes = workspace_bytes;
-  const GemmRoute g = gemm_route(a);
-  put_route(route, g.family, g.grid_x, g.grid_y, g.block);
-  route[4] = g.bm;
-  route[5] = g.bn;
-  route[6] = g.wm;
-  route[7] = g.wn;
-  route[8] = g.sa;
-  route[9] = g.sb;
-  route[10] = g.ma;
-  route[11] = g.mt;
-  route[12] = g.s;
-  route[13] = g.u;
-  route[14] = (int32_t)g.splits;
-  route[15] = g.nt_slabs;
-  route[16] = g.epi_cols;
+  put_gemm_route(route, gemm_route(a));
   return W8A8_OK;
 }
 
@@ -1102,6 +1111,24 @@ int w8a8_diag_argmax_route(size_t n, uint32_t k, int32_t* route, size_t route_le
   if (n == 0) return W8A8_OK;
   const uint32_t nn = (uint32_t)n;
   put_gemv_route(route, gemv_route(1, k, &nn, 1, true));
+  return W8A8_OK;
+}
+
+int w8a8_diag_grouped_route(size_t m, uint32_t k, int count, const size_t* n, int32_t* route, size_t route_len) {
+  if (!route || !n) return W8A8_ENULL;
+  if (route_len < W8A8_DIAG_ROUTE_LEN) return W8A8_EWORKSPACE;
+  if (count < 1 || count > kMaxGroup) return W8A8_EARG;
+  if (k == 0 || k % 16 != 0 || m > kU32Max) return W8A8_ESHAPE;
+  put_route(route, kRouteNone, 0, 0, 0);
+  GemmGroup g{};
+  for (int i = 0; i < count; ++i) {
+    if (n[i] > kU32Max) return W8A8_ESHAPE;
+    if (n[i] > 0) g.n[g.count++] = (uint32_t)n[i];
+  }
+  if (m == 0 || g.count == 0) return W8A8_OK;
+  const GemmRoute r = grouped_gemm(m, k, g);
+  if (r.family != kRouteNone) put_gemm_route(route, r);
+  else if (m <= kDot4MaxM) put_gemv_route(route, gemv_route((uint32_t)m, k, g.n, g.count, false));
   return W8A8_OK;
 }
 

@@ -11,7 +11,7 @@ split-K launch) must be written exactly once.  K loops are checked at their
 extreme iterations: each address is affine in the loop counter.
 
 The replay restates the index expressions of the kernels, each function
-citing the source lines it follows; the table in the design notes states the
+naming the kernel it follows; the table in the design notes states the
 same bounds in words.  Shapes: the benchmark configurations (C1-C5: the
 decode shapes at M = 1, the lm_head, M = 129 and 512, the ragged M = 4 / 16 /
 64), the M = 129 tails (M = 129-135 and 136-159, sampled), N not a multiple
@@ -83,13 +83,13 @@ def xcd_slot(b, G):
 
 
 def mfma32_rows_cols(lane, v):
-    """Row / column of value v of lane l in a 32 x 32 i32 MFMA block (gemm.hip:382-384)."""
+    """Row / column of value v of lane l in a 32 x 32 i32 MFMA block (gemm.hip)."""
     return (v >> 2) * 8 + (lane >> 5) * 4 + (v & 3), lane & 31
 
 
 def frag_offsets():
     """gemm_dma / gemm_tall fragment reads: lane l, sub-step i -> byte offset
-    inside a 32-row block of 128-byte LDS rows (gemm.hip:559-562, :829-832)."""
+    inside a 32-row block of 128-byte LDS rows (gemm.hip)."""
     lane = np.arange(64)
     fr, fh = lane & 31, lane >> 5
     return np.stack([fr * 128 + (((2 * i + fh) ^ ((fr >> 1) & 7)) * 16) for i in range(4)])  # [4, 64]
@@ -99,7 +99,7 @@ def frag_offsets():
 def store_blocks(m, n, row0, col0, FM, FN):
     """(rows, cols) that store_blocks writes for wave tiles with top-left
     corners (row0, col0) (broadcast arrays), guarded by r < m, c < n
-    (gemm.hip:389-460).  Its epilogue loads are clamped (min(r, m - 1),
+    (gemm.hip).  Its epilogue loads are clamped (min(r, m - 1),
     min(c, n - 1)), hence always in bounds."""
     lane = np.arange(64)[:, None]
     v = np.arange(16)[None, :]
@@ -113,71 +113,122 @@ def store_blocks(m, n, row0, col0, FM, FN):
     return rows[keep].astype(np.int64), cols[keep].astype(np.int64)
 
 
-def check_dma(m, n, k, r, residual):
-    """gemm_dma (gemm.hip:483-629) over its grid: DMA sources, LDS ring slots,
+STRIP, CUS = 4, 256                    # kStrip, kCus (gemm.hip)
+MAX_K, MAX_COLS = 1 << 23, 1 << 26     # kMaxK, kMaxCols
+KERNEL_TILES = {13: 8, 14: 4}          # waves per workgroup of gemm_dma's families
+
+
+def own_tile(ns, bn):
+    """Column tiles of the matrices ns (one for a single projection): per tile
+    the matrix that own_tile (gemm.hip) picks and the tile's index within it,
+    by the kernel's comparisons against the launcher's tbegin."""
+    tbegin = np.concatenate([[0], np.cumsum([-(-n // bn) for n in ns])])
+    tbegin = np.concatenate([tbegin, np.full(5 - len(tbegin), tbegin[-1])])  # kMaxGroup + 1 entries
+    t = np.arange(tbegin[-1])
+    mat, first = np.zeros_like(t), np.zeros_like(t)
+    for i in range(1, 4):
+        mat = np.where(t >= tbegin[i], i, mat)
+        first = np.where(t >= tbegin[i], tbegin[i], first)
+    return mat, t - first
+
+
+def check_dma(m, ns, k, r, residual):
+    """gemm_dma over its grid, eight waves (family 13) or four (14), with or
+    without a K tail, one matrix or several: the strip numbering, the DMA
+    sources of every stage, the LDS ring slots, the rotated K order, the
     fragment reads, the stores of store_blocks."""
+    ns = [ns] if isinstance(ns, int) else ns
     BM, BN, WM, WN, SA, SB, splits = r["bm"], r["bn"], r["wm"], r["wn"], r["sa"], r["sb"], r["splits"]
-    tm, tn = -(-m // BM), -(-n // BN)
+    NW = KERNEL_TILES[r["family"]]
+    tail = not (k % 128 == 0 and k <= MAX_K and sum(ns) <= MAX_COLS)
+    mat, local = own_tile(ns, BN)
+    tm, tn = -(-m // BM), len(mat)
     T, G = tm * tn, tm * tn * splits
-    assert r["grid_x"] == G and r["block"] == 512
-    assert k % 128 == 0 and (k // 128) % splits == 0
-    KT = k // 128 // splits
-    LA, LB = BM // 64, BN // 64
+    assert r["grid_x"] == G and r["block"] == 64 * NW and (BM // WM) * (BN // WN) == NW
+    assert len(ns) == 1 or (splits == 1 and not tail)
+    assert not tail or (splits == 1 and NW == 4)
+    KT = k // 128 + 1 if tail else k // 128 // splits
+    assert tail or KT * splits * 128 == k
+    LA, LB = BM // 8 // NW, BN // 8 // NW
     ASL, BSL = BM * 128, BN * 128
     assert SA * ASL + SB * BSL <= 160 * 1024
     Lt = xcd_slot(np.arange(G), G)
     split, Lt = Lt // T, Lt % T
-    m0, n0 = (Lt % tm) * BM, (Lt // tm) * BN
-    wave, lane = np.arange(8)[:, None], np.arange(64)[None, :]
+    s0 = Lt // (STRIP * tn) * STRIP
+    inside = Lt % (STRIP * tn)
+    sm = np.minimum(STRIP, tm - s0)
+    m0, tile = (s0 + inside % sm) * BM, inside // sm
+    assert len({*zip(split.tolist(), m0.tolist(), tile.tolist())}) == G
+    rotated = not tail and NW == 8 and splits == 1 and tn == 1 and T <= CUS
+    for rot in {0, (T - 1) % KT if rotated else 0}:  # every chunk once, whatever the start
+        assert np.array_equal(np.sort([kt + rot - (KT if kt + rot >= KT else 0) for kt in range(KT)]), np.arange(KT))
     kbase = split * KT * 128
+    wave, lane = np.arange(NW)[:, None], np.arange(64)[None, :]
     chunk = lambda row: ((lane & 7) ^ ((row >> 1) & 7)) * 16  # noqa: E731
-    for j in range(LA):
-        row = 8 * (wave * LA + j) + (lane >> 3)                              # [8, 64]
-        g = m0[:, None, None] + row
-        src = np.where(g < m, g, 0) * k + kbase[:, None, None] + chunk(row)
-        within("gemm_dma A", src, src + (KT - 1) * 128 + 16, m * k)
-        dst = (wave * LA + j) * 1024 + lane * 16
-        within("gemm_dma A ring slot", dst, dst + 16, ASL)
-    for j in range(LB):
-        row = 8 * (wave * LB + j) + (lane >> 3)
-        g = n0[:, None, None] + row
-        src = np.where(g < n, g, 0) * k + kbase[:, None, None] + chunk(row)
-        within("gemm_dma B", src, src + (KT - 1) * 128 + 16, n * k)
-        dst = (wave * LB + j) * 1024 + lane * 16
-        within("gemm_dma B ring slot", dst, dst + 16, BSL)
+    slots = {"A": [], "B": []}
+    for name, L, first, rows, pick in (("A", LA, m0, [m], np.zeros(G, int)), ("B", LB, local[tile] * BN, ns, mat[tile])):
+        for j in range(L):
+            row = 8 * (wave * L + j) + (lane >> 3)                               # [NW, 64]
+            slots[name].append((wave * L + j) * 1024 + lane * 16)
+            for i, size in enumerate(rows):
+                f, kb = first[pick == i], kbase[pick == i]
+                if f.size == 0:
+                    continue
+                assert f.max() < size  # the tile's first row exists: it stands in for rows past the end
+                src = np.where(f[:, None, None] + row < size, row, 0) * k            # lane offset
+                if not tail:
+                    assert src.max() + chunk(row).max() < 1 << 32                    # held in 32 bits
+                    at = f[:, None, None] * k + kb[:, None, None] + src + chunk(row)
+                    within(f"gemm_dma {name}", at, at + (KT - 1) * 128 + 16, size * k)
+                    continue
+                for kt in (range(KT) if KT < 4 else (0, KT - 2, KT - 1)):
+                    kk = kt * 128 + chunk(row)
+                    at = f[:, None, None] * k + src + np.where(kk < k, kk, 0)  # activations past K: kZeroChunk
+                    if name == "A":
+                        at = at[:, kk < k]
+                    within(f"gemm_dma {name} tail", at, at + 16, size * k)
+    for name, size in (("A", ASL), ("B", BSL)):
+        written_once(f"gemm_dma {name} ring slot", np.concatenate([s.ravel() for s in slots[name]]) // 16, size // 16)
     off = frag_offsets()
-    wm0, wn0 = (np.arange(8) // (BN // WN)) * WM, (np.arange(8) % (BN // WN)) * WN
+    wm0, wn0 = (np.arange(NW) // (BN // WN)) * WM, (np.arange(NW) % (BN // WN)) * WN
     for f in range(WM // 32):
         a = (wm0 + 32 * f)[:, None, None] * 128 + off[None]
         within("gemm_dma A fragments", a, a + 16, ASL)
     for f in range(WN // 32):
         b = (wn0 + 32 * f)[:, None, None] * 128 + off[None]
         within("gemm_dma B fragments", b, b + 16, BSL)
-    rows, cols = store_blocks(m, n, (m0[:, None] + wm0[None, :]), (n0[:, None] + wn0[None, :]), WM // 32, WN // 32)
-    if splits == 1:
-        written_once("gemm_dma out", rows * n + cols, m * n)
-    else:
-        # slab index of each store: repeat the per-workgroup split over its stores
-        per_wg = [store_blocks(m, n, m0[w] + wm0, n0[w] + wn0, WM // 32, WN // 32) for w in range(G)]
-        idx = np.concatenate([split[w] * m * n + rr * n + cc for w, (rr, cc) in enumerate(per_wg)])
-        written_once("gemm_dma slabs", idx, splits * m * n)
-        check_epilogue(m, n, r, residual)
+    for i, n in enumerate(ns):
+        sel = np.flatnonzero(mat[tile] == i)
+        n0 = local[tile[sel]] * BN
+        assert tail or (4 * n + 31) * 4 < 1 << 32  # store_blocks' 32-bit lane offset
+        rows, cols = store_blocks(m, n, m0[sel][:, None] + wm0[None, :], n0[:, None] + wn0[None, :], WM // 32, WN // 32)
+        if splits == 1:
+            written_once("gemm_dma out", rows * n + cols, m * n)
+        else:
+            # slab index of each store: repeat the per-workgroup split over its stores
+            per_wg = [store_blocks(m, n, m0[w] + wm0, n0[w] + wn0, WM // 32, WN // 32) for w in range(G)]
+            idx = np.concatenate([split[w] * m * n + rr * n + cc for w, (rr, cc) in enumerate(per_wg)])
+            written_once("gemm_dma slabs", idx, splits * m * n)
+            check_epilogue(m, n, r, residual)
 
 
-def check_tall(m, n, k, r, residual):
-    """gemm_tall (gemm.hip:746-945): per-wave DMA instruction dealing, the
+def check_tall(m, ns, k, r, residual):
+    """gemm_tall, one matrix or several: per-wave DMA instruction dealing, the
     rings, the two compute mappings, the stores."""
+    ns = [ns] if isinstance(ns, int) else ns
     BN, SA, SB, MA, splits = r["bn"], r["sa"], r["sb"], r["ma"], r["splits"]
     FN, ASL, BSL, NB = BN // 32, MA * 128, BN * 128, BN // 8
     kMaxA, kMaxB = (MA // 8 + 7) // 8, (NB + 7) // 8
     assert SA * ASL + SB * BSL <= 160 * 1024 and m <= MA
-    tn = -(-n // BN)
+    mat, local = own_tile(ns, BN)
+    tn = len(mat)
     G = tn * splits
-    assert r["grid_x"] == G
+    assert r["grid_x"] == G and (len(ns) == 1 or splits == 1)
     KT = k // 128 // splits
     assert k % 128 == 0 and KT * splits * 128 == k
     Lt = xcd_slot(np.arange(G), G)
-    split, n0 = Lt // tn, (Lt % tn) * BN
+    split, pick, n0 = Lt // tn, mat[Lt % tn], local[Lt % tn] * BN
+    width = np.asarray(ns)[pick]  # each workgroup's matrix: its columns
     kbase = split * KT * 128
     NA = -(-m // 8)
     for wave in range(8):
@@ -193,8 +244,9 @@ def check_tall(m, n, k, r, residual):
             within("gemm_tall A ring slot", dst, dst + 16, ASL)
         for j in range(nb):
             br = 8 * (wave + 8 * j) + (lane >> 3)
-            src = np.minimum(n0[:, None] + br, n - 1) * k + kbase[:, None] + ((lane & 7) ^ ((br >> 1) & 7)) * 16
-            within("gemm_tall B", src, src + (KT - 1) * 128 + 16, n * k)
+            src = (np.minimum(n0[:, None] + br, width[:, None] - 1) * k + kbase[:, None]
+                   + ((lane & 7) ^ ((br >> 1) & 7)) * 16)
+            assert src.min() >= 0 and (src + (KT - 1) * 128 + 16 <= (width * k)[:, None]).all(), "gemm_tall B"
             dst = 1024 * (wave + 8 * j) + lane * 16
             within("gemm_tall B ring slot", dst, dst + 16, BSL)
     off = frag_offsets()
@@ -219,18 +271,19 @@ def check_tall(m, n, k, r, residual):
                 b = 32 * jj * 128 + off
                 within("gemm_tall B fragments", b, b + 16, BSL)
             stores.append((32 * wave + 0 * n0, n0, 1, FN))
-    idx = []
-    for w in range(G):
-        for (row0, col0, fm, fn) in stores:
-            rr, cc = store_blocks(m, n, row0[w], col0[w], fm, fn)
-            idx.append(split[w] * m * n + rr * n + cc)
-    written_once("gemm_tall slabs" if splits > 1 else "gemm_tall out", np.concatenate(idx), splits * m * n)
+    for i, n in enumerate(ns):
+        idx = []
+        for w in np.flatnonzero(pick == i):
+            for (row0, col0, fm, fn) in stores:
+                rr, cc = store_blocks(m, n, row0[w], col0[w], fm, fn)
+                idx.append(split[w] * m * n + rr * n + cc)
+        written_once("gemm_tall slabs" if splits > 1 else "gemm_tall out", np.concatenate(idx), splits * m * n)
     if splits > 1:
-        check_epilogue(m, n, r, residual)
+        check_epilogue(m, ns[0], r, residual)
 
 
 def check_epilogue(m, n, r, residual):
-    """splitk_epilogue / splitk_epilogue8 (gemm.hip:960-1093): grid
+    """splitk_epilogue / splitk_epilogue8 (gemm.hip): grid
     (ceil(n / cols / 256), min(m, 65535)), thread columns c .. c + cols - 1,
     rows blockIdx.y, + gridDim.y, ...; slab index clamped to splits - 1."""
     cols, splits = r["epi_cols"], r["splits"]
@@ -250,7 +303,7 @@ def check_epilogue(m, n, r, residual):
 
 
 def check_skinny(m, n, k, r):
-    """gemm_skinny (gemm.hip:92-144): grid (ceil(n / 16), 1), S waves split K in
+    """gemm_skinny (gemm.hip): grid (ceil(n / 16), 1), S waves split K in
     64-byte steps; loads guarded by kk + koff < K (16-byte reads, K % 16 == 0)."""
     MT, S, U = r["mt"], r["s"], r["u"]
     assert r["grid_x"] == -(-n // 16) and r["grid_y"] == 1 and 16 * MT >= m and k % 16 == 0
@@ -281,26 +334,31 @@ def check_skinny(m, n, k, r):
     written_once("gemm_skinny out", rr[keep] * n + cc[keep], m * n)
 
 
-def check_narrow(m, n, k, r):
-    """gemm_narrow (gemm.hip:268-380, plan :1125): grid ceil(n / 16) x 64 S
-    threads; wave w sums ST = K / (128 S) of the 128-byte K chunks through
-    its own R-stage ring: at S = 4 stage s reads chunk w ST + s, at S = 8
-    chunk ((s + b) mod ST) S + w for workgroup b; the chunks of all waves
-    and stages of a workgroup must be every chunk of K exactly once.  DMA
-    instruction j < 2 + LAL fills rows 8j .. 8j + 7 of a stage (lane l: row
-    8j + l / 8, 16-byte piece (l % 8) ^ (row % 8)); rows 0-15 are weight
-    rows n0 + row clamped to n - 1, rows 16.. activation rows row - 16,
-    loaded only below M."""
+def check_narrow(m, ns, k, r):
+    """gemm_narrow, one matrix or several: ceil(n / (16 NB)) workgroups of 64 S
+    threads per matrix (NB = 2 for groups only); wave w sums ST = K / (128 S) of
+    the 128-byte K chunks through its own R-stage ring: at S = 4 stage s reads
+    chunk w ST + s, at S = 8 chunk ((s + b) mod ST) S + w for workgroup b; the
+    chunks of all waves and stages of a workgroup must be every chunk of K
+    exactly once.  DMA instruction j < 2 NB + LAL fills rows 8j .. 8j + 7 of a
+    stage (lane l: row 8j + l / 8, 16-byte piece (l % 8) ^ (row % 8)); rows below
+    16 NB are weight rows n0 + row clamped to n - 1, the others activation rows
+    row - 16 NB, loaded only below M."""
+    single = isinstance(ns, int)
+    ns = [ns] if single else ns
     MB, S, LAL, R = r["mt"], r["s"], r["u"], r["sa"]
-    assert r["grid_x"] == -(-n // 16) and r["grid_y"] == 1 and r["block"] == 64 * S and r["splits"] == 1
+    NB = 1 if single else r["bn"] // 16
+    mat, local = own_tile(ns, 16 * NB)
+    assert r["grid_x"] == len(mat) and r["grid_y"] == 1 and r["block"] == 64 * S and r["splits"] == 1
     assert k % (128 * S) == 0 and 16 * MB >= m
     # every row below M has its DMA instruction, and every issued instruction has a live lane
     assert 8 * LAL >= m and 8 * (LAL - 1) < m, (m, LAL)
-    ROWS, L = 16 * (1 + MB), 2 + LAL
+    ROWS, L = 16 * (NB + MB), 2 * NB + LAL
     STAGE, RING = ROWS * 128, R * ROWS * 128
-    assert L <= ROWS // 8 and S * RING <= 160 * 1024
+    assert L <= ROWS // 8 and S * RING <= 160 * 1024 and (R - 1) * L < 64
     ST = k // (128 * S)
-    n0 = np.arange(r["grid_x"])[:, None] * 16
+    n0 = (local * 16 * NB)[:, None]
+    width = np.asarray(ns)[mat][:, None]
     lane = np.arange(64)
     b = np.arange(r["grid_x"])
 
@@ -321,11 +379,11 @@ def check_narrow(m, n, k, r):
                 row = 8 * j + (lane >> 3)
                 chunk = ((lane & 7) ^ (row & 7)) * 16
                 koff = kchunk(wave, st)[:, None] * 128 + chunk
-                if j < 2:
-                    src = np.minimum(n0 + row, n - 1) * k + koff
-                    within("gemm_narrow W", src, src + 16, n * k)
+                if j < 2 * NB:
+                    src = np.minimum(n0 + row, width - 1) * k + koff
+                    assert src.min() >= 0 and (src + 16 <= width * k).all(), "gemm_narrow W"
                 else:
-                    g = row - 16
+                    g = row - 16 * NB
                     live = g < m
                     src = (g * k + koff)[:, live]
                     within("gemm_narrow A", src, src + 16, m * k)
@@ -334,78 +392,30 @@ def check_narrow(m, n, k, r):
     fr, fq = lane & 15, lane >> 4
     for h in range(2):
         c = 4 * h + fq
-        b = fr * 128 + ((c ^ (fr & 7)) * 16)
-        within("gemm_narrow B fragments", b, b + 16, STAGE)
-        for t in range(MB):
-            row = 16 + 16 * t + fr
+        for block in range(NB + MB):  # NB weight blocks, then MB activation blocks
+            row = 16 * block + fr
             a = row * 128 + ((c ^ (row & 7)) * 16)
-            within("gemm_narrow A fragments", a, a + 16, STAGE)
-    red = ((np.arange(S)[:, None, None, None] * MB + np.arange(MB)[:, None, None]) * 4
-           + np.arange(4)[:, None]) * 64 + lane
+            within("gemm_narrow fragments", a, a + 16, STAGE)
+    # reduction slot of value v of block (t, u) of a wave, and its reader: index i of every wave
+    t, u, v = np.meshgrid(np.arange(MB), np.arange(NB), np.arange(4), indexing="ij")
+    red = (((np.arange(S)[:, None, None, None, None] * MB + t[..., None]) * NB + u[..., None]) * 4 + v[..., None]) * 64 \
+        + lane
+    written_once("gemm_narrow reduction", red, S * MB * NB * 256)
     within("gemm_narrow reduction", red * 4, red * 4 + 4, S * RING)
-    # epilogue: index i = tid, tid + 64 S, ... < MB * 256 -> (t, v, l)
-    i = np.arange(MB * 4 * 64)
-    l, v, t = i & 63, (i >> 6) & 3, i >> 8
-    rr = 16 * t + 4 * (l >> 4) + v
-    cc = n0 + (l & 15)
-    rr = np.broadcast_to(rr, cc.shape)
-    keep = (rr < m) & (cc < n)
-    written_once("gemm_narrow out", rr[keep] * n + cc[keep], m * n)
-
-
-def check_tiled(m, n, k, r):
-    """gemm_tiled (gemm.hip:147-241): guarded 16-byte loads (gm < M, kk < K),
-    LDS rows of PITCH = 144 bytes, XCD-aware tile numbering."""
-    BM, BN, WM, WN = r["bm"], r["bn"], r["wm"], r["wn"]
-    PITCH = 144
-    tm, tn = -(-m // BM), -(-n // BN)
-    T = tm * tn
-    assert r["grid_x"] == T and k % 16 == 0
-    L = xcd_slot(np.arange(T), T)
-    m0, n0 = (L % tm) * BM, (L // tm) * BN
-    tid = np.arange(256)
-    KT = -(-k // 128)
-    for i in range(BM * 8 // 256):
-        idd = tid + i * 256
-        row, kc = idd >> 3, idd & 7
-        within("gemm_tiled A slot", row * PITCH + kc * 16, row * PITCH + kc * 16 + 16, BM * PITCH)
-        for kt in {0, KT - 1}:
-            gm, kk = m0[:, None] + row, kt * 128 + kc * 16
-            ok = (gm < m) & (kk < k)
-            src = (gm * k + kk)[ok]
-            within("gemm_tiled A", src, src + 16, m * k)
-    for i in range(BN * 8 // 256):
-        idd = tid + i * 256
-        row, kc = idd >> 3, idd & 7
-        for kt in {0, KT - 1}:
-            gn, kk = n0[:, None] + row, kt * 128 + kc * 16
-            ok = (gn < n) & (kk < k)
-            src = (gn * k + kk)[ok]
-            within("gemm_tiled B", src, src + 16, n * k)
-    lane = np.arange(64)
-    frow, fk = lane & 15, (lane >> 4) * 16
-    wave = np.arange(4)
-    wm0, wn0 = (wave // (BN // WN)) * WM, (wave % (BN // WN)) * WN
-    for ks in range(2):
-        for ii in range(WM // 16):
-            a = (wm0[:, None] + ii * 16 + frow) * PITCH + ks * 64 + fk
-            within("gemm_tiled A fragments", a, a + 16, BM * PITCH)
-    rows, cols = [], []
-    for ii in range(WM // 16):
-        for jj in range(WN // 16):
-            for v in range(4):
-                rr = m0[:, None, None] + wm0[None, :, None] + ii * 16 + 4 * (lane >> 4) + v
-                cc = n0[:, None, None] + wn0[None, :, None] + jj * 16 + (lane & 15)
-                rr, cc = np.broadcast_arrays(rr, cc)
-                keep = (rr < m) & (cc < n)
-                rows.append(rr[keep])
-                cols.append(cc[keep])
-    written_once("gemm_tiled out", np.concatenate(rows) * n + np.concatenate(cols), m * n)
+    i = np.arange(MB * NB * 4 * 64)
+    l, v, u, t = i & 63, (i >> 6) & 3, (i >> 8) % NB, (i >> 8) // NB
+    assert np.array_equal(((t * NB + u) * 4 + v) * 64 + l, i)
+    for x, n in enumerate(ns):
+        rr = 16 * t + 4 * (l >> 4) + v
+        cc = n0[mat == x] + 16 * u + (l & 15)
+        rr = np.broadcast_to(rr, cc.shape)
+        keep = (rr < m) & (cc < n)
+        written_once("gemm_narrow out", rr[keep] * n + cc[keep], m * n)
 
 
 # ------------------------------------------------------------------ GEMV routes
 def check_gemv_m1(m, n, k, r, residual, argmax=False):
-    """gemv_m1_one / gemv_m1 (gemv.hip:205-325): wave g owns rows R g ..
+    """gemv_m1_one / gemv_m1 (gemv.hip): wave g owns rows R g ..
     R g + R - 1; loads clamped to n - 1; lanes < R store rows < n."""
     R, KC, W = r["rows"], r["kc"], r["waves"]
     assert m == 1 and k == KC * 1024
@@ -430,7 +440,7 @@ def check_gemv_m1(m, n, k, r, residual, argmax=False):
 
 
 def check_gemv_mt(m, n, k, r, residual):
-    """gemv_mt (gemv.hip:348-423): 4-row groups, MT activation rows per pass
+    """gemv_mt (gemv.hip): 4-row groups, MT activation rows per pass
     (blockIdx.y), 1 KiB chunks with rotation, loads guarded by kk < K."""
     MT, R = r["mt"], 4
     groups = -(-n // R)
@@ -471,14 +481,37 @@ def check_linear(m, n, k, dtype=BF16, residual=False, path=AUTO, workspace=0):
         check_skinny(m, n, k, r)
     elif fam == 12:
         check_tall(m, n, k, r, residual)
-    elif fam == 13:
+    elif fam in KERNEL_TILES:
         check_dma(m, n, k, r, residual)
-    elif fam == 14:
-        check_tiled(m, n, k, r)
     elif fam == 15:
         check_narrow(m, n, k, r)
     else:
         raise AssertionError(f"no route for {(m, n, k)}: {r}")
+    return r
+
+
+def grouped_route(m, ns, k):
+    r, n = np.zeros(ROUTE_LEN, np.int32), np.asarray(ns, np.uint64)
+    assert _lib.lib().w8a8_diag_grouped_route(m, k, len(ns), n.ctypes.data, r.ctypes.data, ROUTE_LEN) == 0
+    keys = ("family grid_x grid_y block bm bn wm wn sa sb ma mt s u splits nt epi_cols rows kc waves").split()
+    return dict(zip(keys, (int(v) for v in r)))
+
+
+def check_grouped(m, ns, k):
+    """The one launch over the matrices that have columns, or each matrix's own."""
+    r, ns = grouped_route(m, ns, k), [n for n in ns if n]
+    if r["family"] == 15:
+        check_narrow(m, ns, k, r)
+    elif r["family"] == 12:
+        check_tall(m, ns, k, r, False)
+    elif r["family"] in KERNEL_TILES:
+        check_dma(m, ns, k, r, False)
+    elif r["family"] == 0:
+        assert m > 4
+        for n in ns:
+            check_linear(m, n, k, path=MFMA)
+    else:
+        assert r["family"] in (2, 3) and m <= 4  # the dot4 launch: each matrix's row groups, as for one
     return r
 
 
@@ -544,7 +577,7 @@ def test_other_m_and_n_not_multiple_of_96(m):
 @pytest.mark.parametrize("m,n,k", [(100, 4096, 4112), (300, 1000, 1040), (65, 777, 2064), (1, 5000, 1040),
                                    (3, 333, 48)])
 def test_k_not_multiple_of_128(m, n, k):
-    """gemm_tiled (K % 128 != 0 at M > 64), gemm_skinny and gemv_mt at odd K."""
+    """gemm_dma with a K tail, gemm_skinny and gemv_mt at odd K."""
     check_linear(m, n, k)
     check_linear(m, n, k, path=DOT4)
 
@@ -552,12 +585,12 @@ def test_k_not_multiple_of_128(m, n, k):
 @pytest.mark.parametrize("n,k", [(4096, 4096), (6144, 4096), (4096, 12288), (1000, 512), (4100, 8192), (333, 2048),
                                  (17, 12288)])
 def test_narrow_every_m(n, k):
-    """gemm_narrow at every M it takes (1-16, and 17-32 at K <= 4096 on
-    N <= 4096): both wave counts (K below and from 8192), one to four live
+    """gemm_narrow at every M it takes (1-16, and 17-64 at K <= 4096 on
+    N <= 4096): both wave counts (K below and from 8192), one to eight live
     activation loads per stage, N not a multiple of 16, a one-stage slice
     (K = 512)."""
     took = 0
-    for m in range(1, 33):
+    for m in [*range(1, 34), 40, 41, 47, 48, 49, 56, 57, 63, 64]:
         for path in (AUTO, MFMA):
             r = check_linear(m, n, k, path=path, workspace=workspace_bytes(m, n, k))
             if path == MFMA and m <= 16:
@@ -602,6 +635,40 @@ def test_auto_ignores_a_workspace_that_only_slows_it(m, n, k):
     assert route(m, n, k, path=MFMA, workspace=ws)["splits"] > 1
 
 
+GROUPS = [(200, 33, 1), (64, 0, 96, 31), (4096, 1024, 1024), (4100, 33, 1, 7), (12288, 12288), (10000, 11600, 5)]
+
+
+@pytest.mark.parametrize("m", [2, 4, 5, 16, 17, 32, 33, 48, 64, 65, 129, 160, 161, 256, 257, 512])
+@pytest.mark.parametrize("ns", GROUPS)
+def test_grouped_launches(m, ns):
+    """Sibling projections: one GEMM launch over the matrices' column tiles,
+    each tile inside its own matrix; every route and both gemm_narrow widths."""
+    for k in (512, 1024, 4096, 8192):
+        check_grouped(m, ns, k)
+
+
+def test_every_grouped_route_is_replayed():
+    """gemm_narrow on 16 and 32 columns, the one-M-tile kernel, gemm_dma with
+    eight and four waves, the dot4 launch, and one launch per matrix."""
+    seen = {(r["family"], r["bn"] if r["family"] == 15 else 0)
+            for r in (check_grouped(m, ns, k) for m, ns, k in [
+                (16, (200, 33), 512), (64, (4096, 1024, 1024), 4096), (129, (12288, 12288), 4096),
+                (512, (4096, 1024, 1024), 4096), (100, (300, 40), 4096), (2, (300, 40), 1040), (70, (100, 33), 1040)])}
+    assert seen == {(15, 16), (15, 32), (12, 0), (13, 0), (14, 0), (3, 0), (0, 0)}, seen
+
+
+@pytest.mark.parametrize("tile,family,m,n,k", [((64, 64), 14, 150, 515, 1280), ((64, 64), 14, 65, 33, 16),
+                                               ((64, 64), 14, 257, 515, 1392), ((128, 64), 14, 1025, 2003, 16),
+                                               ((128, 128), 14, 1300, 3003, 144), ((256, 128), 14, 2049, 2003, 1296),
+                                               ((256, 256), 13, 2049, 6003, 1280), ((64, 128), 13, 129, 10003, 1280),
+                                               ((128, 64), 13, 22000, 60, 640), ((256, 256), 14, 1300, 6003, 1296)])
+def test_every_dma_tile(tile, family, m, n, k):
+    """gemm_dma's tiles, several strips of M tiles, ragged edges, K tails of
+    16 bytes and more, one column of tiles (rotated K)."""
+    r = check_linear(m, n, k)
+    assert (r["family"], r["bm"], r["bn"]) == (family, *tile)
+
+
 def test_every_family_is_replayed():
     """The shapes above reach every GEMM and GEMV family."""
     seen = set()
@@ -614,8 +681,7 @@ def test_every_family_is_replayed():
 
 # ------------------------------------------------------------------ folded producers
 def check_rows_split(n, NS, RS, K):
-    """gemv_m1_split / gemv_rowtail_split streaming waves (gemv.hip:690-757,
-    :856-965): row r of wave wv of workgroup b is (r NS + wv) G + slot(b),
+    """gemv_m1_split / gemv_rowtail_split streaming waves (gemv.hip): row r of wave wv of workgroup b is (r NS + wv) G + slot(b),
     loads clamped to n - 1, stores guarded by row < n."""
     G = -(-n // (NS * RS))
     b, wv, rr = np.meshgrid(np.arange(G), np.arange(NS), np.arange(RS), indexing="ij")
@@ -628,7 +694,7 @@ def check_rows_split(n, NS, RS, K):
 
 
 def check_swiglu_split(n, NS=12, CS=4):
-    """gemv_swiglu_split (gemv.hip:763-842): coordinate k of wave wv of
+    """gemv_swiglu_split (gemv.hip): coordinate k of wave wv of
     workgroup b is (k NS + wv) G + slot(b)."""
     G = -(-n // (NS * CS))
     b, wv, kk = np.meshgrid(np.arange(G), np.arange(NS), np.arange(CS), indexing="ij")
@@ -711,3 +777,19 @@ def test_checker_catches_planted_mistakes():
     bad = dict(route(9, n, k, path=MFMA), u=1)
     with pytest.raises(AssertionError):
         check_narrow(9, n, k, bad)
+    # gemm_dma: a four-wave tile dealt as if to eight waves, a tile count of another tile, and a
+    # tail read that takes the weights' chunk past K
+    r = route(150, 515, 1280)
+    with pytest.raises(AssertionError):
+        check_dma(150, 515, 1280, dict(r, family=13, block=512), False)
+    with pytest.raises(AssertionError):
+        check_dma(150, 515, 1280, dict(r, bn=128), False)
+    k = 1040
+    past = (514 * k) + 8 * 128 + ((lane & 7) ^ 0) * 16  # stage 8 of the last row, unclamped
+    with pytest.raises(AssertionError, match="past the buffer"):
+        within("unclamped tail", past, past + 16, 515 * k)
+    # grouped: a tile given to the next matrix
+    mat, local = own_tile([200, 33], 64)
+    assert mat.tolist() == [0, 0, 0, 0, 1] and local.tolist() == [0, 1, 2, 3, 0]
+    with pytest.raises(AssertionError):
+        check_narrow(2, [200, 33], 512, dict(grouped_route(2, [200, 33], 512), bn=32))
