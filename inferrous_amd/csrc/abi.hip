@@ -77,8 +77,9 @@ int check_linear(const int8_t* q, const float* asc, size_t m, const int8_t* w, c
 // MFMA routes at m = 2 (gemm_skinny at K not a multiple of 512, split-K) were
 // not measured to lead and keep the GEMV.  A split-K route needs the
 // caller's workspace; without it m = 3 and 4 keep the dot4 GEMV.  The grouped
-// projections take one GEMM launch from m = 2 where their route is gemm_narrow
-// or the 96-column tiles, and keep one dot4 launch up to m = 4 otherwise.
+// projections take one GEMM launch from m = 2 where their route is the 96-column
+// tiles or gemm_narrow leads (narrow_group_leads), and keep one dot4 launch up
+// to m = 4 otherwise.
 constexpr size_t kDot4MaxM = 4;
 constexpr size_t kDot4AutoMaxM = 2;
 constexpr size_t kRowtailWidthAbi = 12288;  // the down projection's K (the MLP width)
@@ -147,12 +148,32 @@ int run_linear(hipStream_t st, const int8_t* q, const float* asc, size_t m, cons
 }
 
 
+// Whether gemm_narrow runs a group of up to kDot4MaxM rows faster than the one dot4
+// launch.  gemm_narrow's K = 8192 form takes a CU per workgroup, so a second
+// round of them loses; below, it loses at two or three rounds of short stages.
+// Measured on MI355X with distinct weights, BF16, dot4 / gemm_narrow us, columns
+// together x K: M = 2 6144 x 4096 7.3 / 7.3, 4096 x 2048 4.2 / 4.3, 8192 x 3072 6.6 / 7.1,
+// 12288 x 4096 10.5 / 11.8, 3072 x 8192 7.6 / 7.2, 6144 x 8192 11.6 / 13.2, 16384 x 8192
+// 21.6 / 27.7; M = 3 8192 x 2048 6.0 / 5.8, 12288 x 2048 7.4 / 8.1, 12288 x 4096 12.8 / 11.8,
+// 4096 x 12288 13.8 / 11.1, 6144 x 8192 12.9 / 13.4; M = 4 6144 x 12288 19.3 / 18.6, 8192 x
+// 8192 14.8 / 15.8.  At K = 16384 every weight row starts on one memory channel: M = 3
+// 3072 columns 15.9 / 16.0, 8192 25 / 36.
+static bool narrow_group_leads(size_t m, uint32_t k, uint32_t workgroups) {
+  if (k >= 8192) {
+    const uint32_t most = k % 16384 == 0 ? 64u * (uint32_t)(m - 1) : m == 4 ? 384u : m == 3 || k > 8192 ? 256u : 192u;
+    return workgroups <= most;
+  }
+  if (workgroups <= (m == 2 ? 256u : 512u)) return true;
+  return (m > 2 || workgroups <= 512u) && (k <= (m == 2 ? 1024u : 512u) || k >= 4096);
+}
+
 // The GEMM launch of a grouped call (family none: one dot4 launch up to kDot4MaxM
 // rows, one launch per matrix above).
 static GemmRoute grouped_gemm(size_t m, uint32_t k, const GemmGroup& g) {
   if (m <= 1) return GemmRoute{};
   const GemmRoute r = gemm_group_route((uint32_t)m, k, g.n, g.count);
-  return m > kDot4MaxM || r.family == kRouteNarrow || r.bn == 96 ? r : GemmRoute{};
+  if (m > kDot4MaxM || r.bn == 96) return r;
+  return r.family == kRouteNarrow && narrow_group_leads(m, k, r.grid_x) ? r : GemmRoute{};
 }
 
 int check_argmax(const int8_t* q, const float* asc, const int8_t* w, const float* ws, size_t n,

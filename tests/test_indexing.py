@@ -657,6 +657,19 @@ def test_every_grouped_route_is_replayed():
     assert seen == {(15, 16), (15, 32), (12, 0), (13, 0), (14, 0), (3, 0), (0, 0)}, seen
 
 
+@pytest.mark.parametrize("m,ns,k,gemm", [
+    (2, (4096, 1024, 1024), 4096, True), (2, (8192, 2048, 2048), 4096, False), (2, (8192, 8192), 1024, False),
+    (2, (2048, 1024, 1024), 2048, True), (2, (4096, 2048, 2048), 3072, False), (2, (12288, 12288), 4096, True),
+    (2, (2048, 512, 512), 12288, True), (2, (4096, 1024, 1024), 8192, False), (2, (1024, 512, 512), 16384, False),
+    (3, (2048, 1024, 1024), 12288, True), (3, (8192, 8192), 8192, False), (3, (8192, 2048, 2048), 2048, False),
+    (3, (4096, 4096), 2048, True), (4, (4096, 1024, 1024), 9216, True), (4, (4096, 4096), 16384, False),
+    (4, (8192, 8192), 4096, True), (4, (8192, 8192), 2048, False), (4, (100, 33), 1040, False)])
+def test_grouped_gemm_or_dot4(m, ns, k, gemm):
+    """Two to four rows of siblings: the launch that was faster with distinct
+    weights, gemm_narrow (or the 96-column tiles) or one dot4 GEMV."""
+    assert (check_grouped(m, ns, k)["family"] >= 11) == gemm
+
+
 @pytest.mark.parametrize("tile,family,m,n,k", [((64, 64), 14, 150, 515, 1280), ((64, 64), 14, 65, 33, 16),
                                                ((64, 64), 14, 257, 515, 1392), ((128, 64), 14, 1025, 2003, 16),
                                                ((128, 128), 14, 1300, 3003, 144), ((256, 128), 14, 2049, 2003, 1296),
@@ -681,7 +694,8 @@ def test_every_family_is_replayed():
 
 # ------------------------------------------------------------------ folded producers
 def check_rows_split(n, NS, RS, K):
-    """gemv_m1_split / gemv_rowtail_split streaming waves (gemv.hip): row r of wave wv of workgroup b is (r NS + wv) G + slot(b),
+    """gemv_m1_split / gemv_rowtail_split streaming waves (gemv.hip): row r of
+    wave wv of workgroup b is (r NS + wv) G + slot(b),
     loads clamped to n - 1, stores guarded by row < n."""
     G = -(-n // (NS * RS))
     b, wv, rr = np.meshgrid(np.arange(G), np.arange(NS), np.arange(RS), indexing="ij")
