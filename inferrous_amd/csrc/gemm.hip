@@ -1207,12 +1207,13 @@ static bool split_plan(uint32_t m, uint32_t n, uint32_t k, uint32_t& splits) {
   return kt % splits == 0 && kt / splits >= 4 && (tiles * 3 <= kCus * 2 || n <= 128);
 }
 
-// gemm_narrow's plan: S = 4 waves below K = 8192 and 8 from there (each wave
-// keeps eight or more 128-byte stages), R-deep rings, MB 16-row blocks, LAL
+// gemm_narrow's plan: S = 4 waves below K = 8192 and 8 from there (a wave
+// walks K / (128 S) stages of 128 bytes), R-deep rings, MB 16-row blocks, LAL
 // = ceil(M / 8) activation DMA loads per stage.  It takes M <= 16 on the
 // narrow shapes, and M <= 64 where one workgroup per 16 columns fits the
-// CUs once at K <= 4096 (o at M = 48 / 64 6.6 / 7.6 us against gemm_tall split
-// K's 8.9 / 8.8); the wide shapes (n / 96 >= 224 tiles) keep
+// CUs once at K <= 4096 (4096 x 2048 at M = 40 / 64 5.5 / 6.2 us against gemm_tall
+// split K's 7.9 / 7.3, 4096 x 4096 at M = 40 7.8 / 9.3; past 48 rows there see
+// split_leads_narrow); the wide shapes (n / 96 >= 224 tiles) keep
 // gemm_tall's unsplit 96-column tiles.  Measured on MI355X, graphs of 36
 // distinct-weight launches, random operands, against the routes it
 // replaced (gemm_tall split-K 4 with its slab epilogue launch, gemm_skinny),
@@ -1239,6 +1240,20 @@ static bool narrow_plan(uint32_t m, uint32_t n, uint32_t k, int& S, int& R, int&
   return true;
 }
 
+static bool tall_plan(uint32_t m, uint32_t n, uint32_t k, int& bn, uint32_t& splits, int& ma);
+
+// Whether, with a workspace, gemm_tall's split K beats gemm_narrow on a shape of
+// narrow_plan: four 16-row blocks at the longest K, whose rings are three deep, and
+// which pull 64 activation rows over all of K into every CU.  Measured on MI355X
+// with distinct weights, gemm_narrow / split us, 4096 columns x K = 4096, BF16 and f32
+// with the residual: M = 48 8.3 / 8.6 and 9.2 / 9.2, M = 52 level and 9.8 / 9.1, M = 64
+// 9.0 / 8.7 and 10.3 / 9.3; 1024 columns M = 56 8.0 / 7.7, M = 64 8.2 / 7.9, 2560 columns M =
+// 64 level; at K = 3584 level or slower.
+static bool split_leads_narrow(uint32_t m, uint32_t n, uint32_t k) {
+  int bn, ma;
+  uint32_t splits;
+  return m > (n > 3900 ? 48u : n > 3500 ? 52u : 56u) && k > 3584 && tall_plan(m, n, k, bn, splits, ma) && splits > 1;
+}
 
 // gemm_tall plan for 1 <= m <= 256 (measured on MI355X on the Qwen3-8B
 // projection shapes at M = 16, 64, 65, 80, 100, 128 and 129): 96-column
@@ -1316,7 +1331,7 @@ size_t gemm_workspace_bytes(uint32_t m, uint32_t n, uint32_t k) {
   int ma;
   {
     int S, R, MB, LAL;
-    if (narrow_plan(m, n, k, S, R, MB, LAL)) return 0;
+    if (narrow_plan(m, n, k, S, R, MB, LAL) && !split_leads_narrow(m, n, k)) return 0;
   }
   if (tall_plan(m, n, k, tile, splits, ma)) return splits > 1 ? (size_t)splits * m * n * sizeof(int32_t) : 0;
   if (!split_plan(m, n, k, splits)) return 0;
@@ -1478,7 +1493,9 @@ GemmRoute gemm_route(const GemmArgs& a) {
   if (a.m == 0 || a.n == 0) return r;
   {
     int S, R, MB, LAL;
-    if (narrow_plan(a.m, a.n, a.k, S, R, MB, LAL)) {
+    const size_t slabs = 4 * (size_t)a.m * a.n * sizeof(int32_t);
+    const bool split = a.partials && a.partial_bytes >= slabs && split_leads_narrow(a.m, a.n, a.k);
+    if (!split && narrow_plan(a.m, a.n, a.k, S, R, MB, LAL)) {
       r.family = kRouteNarrow;
       r.mt = MB;
       r.s = S;

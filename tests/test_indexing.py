@@ -635,6 +635,19 @@ def test_auto_ignores_a_workspace_that_only_slows_it(m, n, k):
     assert route(m, n, k, path=MFMA, workspace=ws)["splits"] > 1
 
 
+@pytest.mark.parametrize("m,n,k,split", [(64, 4096, 4096, True), (49, 4096, 4096, True), (48, 4096, 4096, False),
+                                         (53, 3584, 4096, True), (52, 3584, 4096, False),
+                                         (57, 1024, 4096, True), (56, 1024, 4096, False), (64, 4096, 3584, False),
+                                         (64, 4095, 4096, False), (40, 4096, 4096, False)])
+def test_split_k_past_the_narrow_kernel(m, n, k, split):
+    """At the most rows and the longest K of gemm_narrow a workspace gives
+    split K, which is faster there; without one the shape stays narrow."""
+    assert (workspace_bytes(m, n, k) > 0) == split
+    r = check_linear(m, n, k, workspace=workspace_bytes(m, n, k))
+    assert r["family"] == (12 if split else 15) and r["splits"] == (4 if split else 1)
+    assert check_linear(m, n, k)["family"] == 15
+
+
 GROUPS = [(200, 33, 1), (64, 0, 96, 31), (4096, 1024, 1024), (4100, 33, 1, 7), (12288, 12288), (10000, 11600, 5)]
 
 
