@@ -1122,8 +1122,8 @@ __global__ __launch_bounds__(256) void splitk_epilogue8(GemmArgs a, const int32_
 // ones the other way about.  A round that leaves CUs idle runs up to a
 // quarter faster (L2 and power are shared).
 //
-// kDmaTiles, K % 128 == 0: eight waves, and four on 64 x 64.  Measured on MI355X with random operands, us per
-// launch (256 x 256 / 256 x 192 / 256 x 128 / 128 x 192 / 128 x 128 / 128 x 64):
+// kDmaTiles, K % 128 == 0: eight waves, and four on 64 x 64.  Measured on MI355X
+// with random operands, us per launch (256 x 256 / 256 x 192 / 256 x 128 / 128 x 192 / 128 x 128 / 128 x 64):
 // 24576 x 4096 f32 at M = 4096 393 / 417 / 439 / 488 / 537 / -; 6144 x 4096 BF16
 // at M = 4096 112 / 97.7 / 103 / 113 / 126 / -, at M = 1024 - / - / 30.3 / 28.1 /
 // 38.2 / 39.4, at M = 512 - / - / - / 23.5 / 19.4 / 25.5; 4096 x 4096 f32 with the
@@ -1132,10 +1132,9 @@ __global__ __launch_bounds__(256) void splitk_epilogue8(GemmArgs a, const int32_
 // likewise at M = 4096 196 / - / 211 / - / 257 / -, at M = 512 - / - / 84 / 72 / 58 /
 // 44.7.
 //
-// 6144 x 4096 f32 at M = 129: 64 x 128 12.5, 64 x 64 16.5 (gemm_tall's split K with
-// its slab epilogue 16.4); 4096 x 4096 with the residual at M = 129 64 x 64 11.5
-// (split 13.6), at M = 256 12.7 (17.2).  Four-wave tiles of 128 x 64 and 128 x 32
-// were within 1 us of those on these shapes, and slower where they mattered.
+// With distinct weights, f32 and the residual, 4096 x 4096 on 64 x 64 at M = 129 12.8
+// (split K with its slab epilogue 13.6), at M = 256 13.4 (17.4).  Four-wave tiles of
+// 128 x 64 and 128 x 32 were within 1 us of those, and slower where they mattered.
 // 64 x 128 costs more than 128 x 64 although it moves as much: with distinct
 // weights, BF16, 64 x 128 / 128 x 64, 4096 columns at M = 300, K = 4096 15.8 / 14.1
 // and K = 8192 28.2 / 24.8, 2560 x 8192 at M = 700 41.2 / 28.2, 3584 x 8192 at M =
@@ -1144,11 +1143,12 @@ __global__ __launch_bounds__(256) void splitk_epilogue8(GemmArgs a, const int32_
 // (10240 x 4096 at M = 129 17.2 / 19.2), and by little at the most tiles of one
 // round (8192 x 4096 at M = 129 15.5 / 16.4, M = 180 17.4 / 17.0).
 //
-// kTailTiles, K % 128 != 0: four waves.  gemm_tiled, the register-staged kernel
-// these replaced -> the tile the route takes: 4096 x 8000 x 5008 316 -> 168, 2000
-// x 8000 x 5008 145 -> 89, 1024 x 4096 x 4112 52 -> 26, 512 x 6000 x 4112 52 -> 30,
-// 300 x 3000 x 2000 28 -> 9.2, 77 x 5003 x 2000 27.7 -> 8.7, and gemm_skinny: 64 x
-// 4096 x 4112 16.0 -> 11.9, 30 x 12000 x 4112 28.6 -> 15.8 (M x N x K).
+// kTailTiles, K % 128 != 0: four waves.  The register-staged kernel that
+// these replaced -> the tile the route takes, distinct weights, BF16, M x N x K: 4096 x
+// 8000 x 5008 294 -> 163, 2000 x 8000 x 5008 139 -> 87, 1024 x 4096 x 4112 54 -> 30, 512 x
+// 6000 x 4112 56 -> 32, 300 x 3000 x 2000 31 -> 10.3, 129 x 4096 x 4112 50 -> 13.2, 77 x
+// 5003 x 2000 32 -> 9.0; and gemm_skinny on wider N (skinny_leads): 32 x 12000 x 4112
+// 29.6 -> 16.0, 64 x 8192 x 4112 29.0 -> 20.0.
 struct DmaTile {
   int bm, bn, wm, wn, sa, sb;
   uint32_t fixed, stage, pair;  // pair 0: one workgroup per CU
@@ -1693,17 +1693,13 @@ static hipError_t launch_dma_group(hipStream_t st, const GemmArgs& a, const Gemm
   return hipGetLastError();
 }
 
-// The grouped route: the single projection's plans on the siblings' columns
-// together, so a group fills the chip where its matrices alone would not, and
-// pays one launch.  Groups have no workspace, so narrow groups of 17 to 256
-// rows take 32-column one-M-tile workgroups where a single projection would
-// split K.  Measured on MI355X, one launch per matrix -> one launch, per
-// dispatch: gate and up (12288 x 4096 each) at M = 4 24.3 (dot4) -> 18.3 us, at
-// M = 32 2 x 23.1 -> 18.2, at M = 129 2 x 33 -> 30.1, at M = 512 2 x 33.0 ->
-// 58.2; q, k and v (4096 + 1024 + 1024) at M = 4 8.7 (dot4) -> 8.1, at M = 129
-// 14.2 + 2 x 14 -> 20.9, at M = 512 3 x 16.5 -> 24.6, at M = 4096 99 + 2 x 42
-// -> 149.  gate and up at M = 4096 (several rounds of tiles either way) are
-// level.
+// The grouped route: the single projection's unsplit routes on the siblings'
+// columns together (groups have no workspace), so a group fills the chip where
+// its matrices alone would not, and pays one launch.  Measured on MI355X with
+// distinct weights, BF16, one launch per matrix (dot4 up to M = 4) -> this, us: gate
+// and up (12288 x 4096 each) at M = 4 20.8 -> 17.4, M = 32 46.4 -> 17.4, M = 129 57.3 ->
+// 28.0, M = 512 66.0 -> 52.1, M = 4096 435 -> 367; q, k and v (4096 + 1024 + 1024) at M = 4 8.8
+// -> 7.5, M = 32 19.3 -> 9.6, M = 129 44.8 -> 14.9, M = 512 47.6 -> 22.4, M = 4096 173 -> 104.
 GemmRoute gemm_group_route(uint32_t m, uint32_t k, const uint32_t* n, int count) {
   GemmRoute r{};
   r.splits = 1;
