@@ -1251,12 +1251,14 @@ static bool tall_plan(uint32_t m, uint32_t n, uint32_t k, int& bn, uint32_t& spl
 // which pull 64 activation rows over all of K into every CU.  Measured on MI355X
 // with distinct weights, gemm_narrow / split us, 4096 columns x K = 4096, BF16 and f32
 // with the residual: M = 48 8.3 / 8.6 and 9.2 / 9.2, M = 52 level and 9.8 / 9.1, M = 64
-// 9.0 / 8.7 and 10.3 / 9.3; 1024 columns M = 56 8.0 / 7.7, M = 64 8.2 / 7.9, 2560 columns M =
-// 64 level; at K = 3584 level or slower.
+// 9.0 / 8.7 and 10.3 / 9.3; 512 columns M = 56 7.9 / 7.4, 1024 M = 56 7.9 / 7.6, M = 64 8.2 / 7.9; not 2048
+// columns at M = 57 8.2 / 8.4, 3000 at M = 64 8.7 / 9.2 (split K's 64-column tiles fill the CUs
+// less well there); at K = 3584 level or slower.
 static bool split_leads_narrow(uint32_t m, uint32_t n, uint32_t k) {
   int bn, ma;
   uint32_t splits;
-  return m > (n > 3900 ? 48u : n > 3500 ? 52u : 56u) && k > 3584 && tall_plan(m, n, k, bn, splits, ma) && splits > 1;
+  if (n > 1536 && n <= 3050) return false;
+  return m > (n > 3900 ? 48u : n > 3500 || n <= 1024 ? 52u : 56u) && k > 3584 && tall_plan(m, n, k, bn, splits, ma) && splits > 1;
 }
 
 // gemm_tall plan for 1 <= m <= 256 (measured on MI355X on the Qwen3-8B
@@ -1318,7 +1320,8 @@ static bool tall_plan(uint32_t m, uint32_t n, uint32_t k, int& bn, uint32_t& spl
 // Two slabs, unsplit over split at K = 4352 / 5376 / 7936: M = 65 0.95-0.99 / 0.99-1.02 /
 // 1.04-1.06, M = 129 0.83-0.87 / 0.84-0.89 / 0.90-0.92 (1024 to 4096 columns).
 // Above 256 rows: split_plan's single column of tiles past its share of the CUs (64
-// columns, M = 22,000 / 33,000, K = 8192 48 / 83 split, 27 / 57 unsplit).
+// columns, M = 22,000 / 33,000, K = 8192 48 / 83 split, 27 / 57 unsplit; within it the pair is
+// level at K = 8192 and leads beyond, M = 300 to 1,500 at K = 16384 31 / 35).
 bool gemm_unsplit_leads(uint32_t m, uint32_t n, uint32_t k) {
   int bn, ma;
   uint32_t splits;

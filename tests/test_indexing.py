@@ -637,7 +637,9 @@ def test_auto_ignores_a_workspace_that_only_slows_it(m, n, k):
 
 @pytest.mark.parametrize("m,n,k,split", [(64, 4096, 4096, True), (49, 4096, 4096, True), (48, 4096, 4096, False),
                                          (53, 3584, 4096, True), (52, 3584, 4096, False),
-                                         (57, 1024, 4096, True), (56, 1024, 4096, False), (64, 4096, 3584, False),
+                                         (53, 1024, 4096, True), (52, 1024, 4096, False),
+                                         (57, 1536, 4096, True), (56, 1536, 4096, False), (64, 4096, 3584, False),
+                                         (64, 2560, 4096, False),
                                          (64, 4095, 4096, False), (40, 4096, 4096, False)])
 def test_split_k_past_the_narrow_kernel(m, n, k, split):
     """At the most rows and the longest K of gemm_narrow a workspace gives
